@@ -1,0 +1,76 @@
+"""The per-step kernels' launch shapes agree bit for bit.
+
+A small system on a handle of its own takes the wide first and force passes;
+the same system in a pool, whose launches cover at least 65,536 slots, takes
+the two- or four-wave ones at the same split.  Both add the same terms in the
+same order, so positions, velocities, forces and densities are equal.
+"""
+import numpy as np
+import pytest
+
+from conftest import uniform_box
+from test_gpu_arb import DECK, LX, LY, LZ, channel
+from test_gpu_parity import dpd_system, mdpd_system
+
+pytestmark = pytest.mark.gpu
+
+
+def _box(engine, n, L, **kw):
+    x, v = uniform_box(n, L, 100 + n)
+    return mdpd_system(engine, x, v, L, **kw)
+
+
+def _two_types(engine):
+    n, L = 1500, 6.5
+    x, v = uniform_box(n, L, 17)
+    types = np.where(np.arange(n) % 3 == 0, 2, 1).astype(np.int32)
+    return mdpd_system(engine, x, v, L, types=types, ntypes=2, coeff="1 1 -40 25 4.5 1.0 0.75",
+                       extra="pair_coeff 1 2 -30 25 4.5 1.0 0.75\npair_coeff 2 2 -20 20 2.0 0.9 0.7")
+
+
+def _walls(engine):
+    x, v, types, _ = channel()
+    s = engine.System()
+    s.command("atom_style mdpd/atomic/meso 8.0")
+    s.create_box(2, (0, 0, 0), (LX, LY, LZ))
+    s.create_atoms(types, x, v)
+    s.commands(DECK)
+    return s
+
+
+def _dpd(engine):
+    x, v = uniform_box(648, 6.0, 5)
+    return dpd_system(engine, x, v, 6.0)
+
+
+CASES = {
+    "one": lambda e: _box(e, 1, 4.0),
+    "tile - 1": lambda e: _box(e, 63, 4.0),
+    "tile": lambda e: _box(e, 64, 4.0),
+    "tile + 1": lambda e: _box(e, 65, 4.0),
+    "liquid": lambda e: _box(e, 1296, 6.0),
+    "lucy": lambda e: _box(e, 1296, 6.0, lucy=True),
+    # ~170 entries and ~80 pairs a row: several rounds of chunks and of pairs
+    "dense": lambda e: _box(e, 1200, 4.0, rho_est=18.75, extra="timestep 0.001"),
+    "two types": _two_types,
+    "walls": _walls,
+    "dpd": _dpd,
+}
+
+
+@pytest.mark.parametrize("split", [2, 4])
+@pytest.mark.parametrize("case", list(CASES))
+def test_small_system_equals_its_pool_job(engine, case, split):
+    s = CASES[case](engine)
+    p = engine.Pool(float(1 << 29), 16)
+    p.tune("split", split)
+    j = p.submit(s, 12)
+    p.run()
+    s.tune("split", split)
+    s.run(12)
+    for k in ("x", "v", "f", "rho"):
+        a = s.gather(k)
+        assert np.isfinite(a).all()
+        np.testing.assert_array_equal(p.gather(j, k), a, err_msg=f"{case}, split {split}: {k}")
+    p.close()
+    s.close()

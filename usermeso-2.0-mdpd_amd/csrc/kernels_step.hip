@@ -95,6 +95,37 @@ __device__ inline float pair_rsq(const float4 &pi, const float4 &q, uint32_t cod
 // the same wave.
 // Partial densities are summed in LDS in wave order (deterministic).
 // --------------------------------------------------------------------------
+// the density weight of a neighbor at r = sqrt(rsq) < h, (h - r)^2 or Lucy's
+// (h + 3 r) (h - r)^3, as the two factors of the fused multiply-add that adds
+// it to a sum (both passes below round alike); rsq < 0: zero
+__device__ inline float2 weight_factors(float h, float rsq, bool lucy)
+{
+    const float r = __builtin_amdgcn_sqrtf(rsq);
+    const float hm = h - r;
+    const float g = lucy ? fmaf(r, 3.f, h) * hm * hm : hm;
+    return rsq < 0.f ? make_float2(0.f, 0.f) : make_float2(hm, g);
+}
+
+// system of a tile; one system (the plain path) holds them all
+__device__ inline int tile_system(const PoolDev &P, int tile) { return P.nsys == 1 ? 0 : P.wave_sys[tile]; }
+
+// density of particle i from its weight sum, and the record the force pass of
+// a one-type system gathers (position and density in one 16-byte load)
+template <bool WITH_RHO>
+__device__ inline void finish_density(const PoolDev &P, const SysDev *d, int i, const float4 &pi, float sum)
+{
+    if (WITH_RHO) {
+        const int mk = P.mask[d->sela][i];
+        const int ti = __float_as_int(pi.w);
+        const float r = (mk & d->rho_bit) ? P.mass[d->mass_base + ti] * d->rho_factor * sum : 0.f;
+        P.rho[i] = r;
+        P.pr[i] = make_float4(pi.x, pi.y, pi.z, r);
+    } else if (d->style == STYLE_MDPD) {
+        // mDPD without the density fix: zero density (P.rho keeps its zeros)
+        P.pr[i] = make_float4(pi.x, pi.y, pi.z, 0.f);
+    }
+}
+
 template <bool WITH_RHO, int SPLIT>
 __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
 {
@@ -105,7 +136,7 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = tile * WAVE + lane;
-    const int s = P.wave_sys[tile];
+    const int s = tile_system(P, tile);
     if (s < 0) return;
     const SysDev *d = P.sys + s;
     if (!d->active || d->overflow) return;    // an overflowed system waits for wider rows
@@ -130,9 +161,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
     auto visit = [&](uint32_t e, const float4 &q, auto room) {
         const float rsq = pair_rsq(pi, q, e >> IMG_SHIFT, d);
         if (WITH_RHO && rsq < h2 && rsq >= 1e-20f) {
-            const float r = __builtin_amdgcn_sqrtf(rsq);
-            const float hm = h - r;
-            sum += lucy ? (h + 3.f * r) * hm * hm * hm : hm * hm;
+            const float2 f = weight_factors(h, rsq, lucy);
+            sum = fmaf(f.x, f.y, sum);
         }
         if (rsq < rc2 && rsq >= 1e-20f) {
             if constexpr (decltype(room)::value) {
@@ -211,20 +241,113 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
     if (WITH_RHO) {
         s_sum[w][lane] = sum;
         __syncthreads();
-        if (w == 0 && valid) {
-            float tot = s_sum[0][lane];
-            for (int k = 1; k < SPLIT; ++k) tot += s_sum[k][lane];
-            const int mk = P.mask[d->sela][i];
-            const int ti = __float_as_int(pi.w);
-            const float r = (mk & d->rho_bit) ? P.mass[d->mass_base + ti] * d->rho_factor * tot : 0.f;
-            P.rho[i] = r;
-            // the force pass of a one-type system gathers a neighbor's
-            // position and density with one 16-byte load
-            P.pr[i] = make_float4(pi.x, pi.y, pi.z, r);
+        if (w == 0)
+            for (int k = 1; k < SPLIT; ++k) sum += s_sum[k][lane];
+    }
+    if (w == 0 && valid) finish_density<WITH_RHO>(P, d, i, pi, sum);
+}
+
+// --------------------------------------------------------------------------
+// The first pass with one wave per row chunk of a tile (split 2 and 4): lane
+// l of wave k holds chunk k of particle l, its eight gathers in flight at
+// once.  Each wave leaves its in-cutoff counts and its weight factors in LDS,
+// places its compact entries after those of the sub-row's earlier chunks, and
+// wave w adds up sub-row w's weights in row order.  Rounds of FS_WAVES chunks.
+// --------------------------------------------------------------------------
+template <int SPLIT>
+constexpr int FS_WAVES = SPLIT == 2 ? 10 : 12;
+
+template <bool WITH_RHO, int SPLIT>
+__global__ void __launch_bounds__(WAVE * FS_WAVES<SPLIT>) k_first_wide(PoolDev P, int ntiles)
+{
+    constexpr int NW = FS_WAVES<SPLIT>;
+    static_assert(NW % SPLIT == 0, "a wave keeps its sub-row from round to round");
+    __shared__ float2 s_w[WITH_RHO ? NW * NBR_CHUNK : 1][WAVE];    // weight factors of each entry
+    __shared__ int s_n[NW][WAVE];                                  // in-cutoff entries of each chunk
+    __shared__ float s_sum[SPLIT][WAVE];
+    const int tile = xcd_logical(blockIdx.x, ntiles);
+    if (tile >= ntiles) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int i = tile * WAVE + lane;
+    const int s = tile_system(P, tile);
+    if (s < 0) return;
+    const SysDev *d = P.sys + s;
+    if (!d->active || d->overflow) return;    // an overflowed system waits for wider rows
+    const bool valid = i < d->part_base + d->n;
+    const float4 *pos = P.pos[d->sel];
+    const int maxnbr = P.maxnbr;
+    int *crow = P.clist + (size_t)tile * maxnbr * WAVE + lane;
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
+    int cnt = 0;
+    if (valid) {
+        pi = pos[i];
+        cnt = min(P.ncount[i], maxnbr);
+    }
+    const float h = d->rd, h2 = h * h;
+    const float rc2 = d->rc2_max;
+    const bool lucy = d->lucy;
+    const int4 *row4 = (const int4 *)(P.nlist + nbr_at(i, 0, maxnbr));
+    float sum = 0.f;
+    int base = 0;                             // compact entries of this wave's sub-row in earlier rounds
+    for (int c0 = 0;; c0 += NW) {
+        const int c = c0 + wv, left = cnt - c * NBR_CHUNK;      // this chunk's entries, if fewer than eight
+        uint32_t e[NBR_CHUNK];
+        int flags = 0;
+        if (left > 0) {
+            const int4 ea = row4[(size_t)c * (NBR_CHUNK * WAVE / 4)], eb = row4[(size_t)c * (NBR_CHUNK * WAVE / 4) + 1];
+            e[0] = (uint32_t)ea.x; e[1] = (uint32_t)ea.y; e[2] = (uint32_t)ea.z; e[3] = (uint32_t)ea.w;
+            e[4] = (uint32_t)eb.x; e[5] = (uint32_t)eb.y; e[6] = (uint32_t)eb.z; e[7] = (uint32_t)eb.w;
+            float4 q[NBR_CHUNK];
+#pragma unroll
+            for (int k = 0; k < NBR_CHUNK; ++k) q[k] = pos[(k < left ? e[k] : (uint32_t)i) & IDX_MASK];
+#pragma unroll
+            for (int k = 0; k < NBR_CHUNK; ++k) {
+                const float rsq = pair_rsq(pi, q[k], k < left ? e[k] >> IMG_SHIFT : IMG_ZERO, d);
+                const bool in = k < left && rsq >= 1e-20f;
+                if (WITH_RHO) s_w[wv * NBR_CHUNK + k][lane] = weight_factors(h, in && rsq < h2 ? rsq : -1.f, lucy);
+                flags |= (in && rsq < rc2 ? 1 : 0) << k;
+            }
         }
-    } else if (w == 0 && valid && d->style == STYLE_MDPD) {
-        // mDPD without the density fix: zero density (P.rho keeps its zeros)
-        P.pr[i] = make_float4(pi.x, pi.y, pi.z, 0.f);
+        s_n[wv][lane] = __popc((unsigned)flags);
+        __syncthreads();
+        int at = base;                        // compact entries of the sub-row before this chunk
+#pragma unroll
+        for (int k = 0; k < NW / SPLIT; ++k) {
+            const int x = s_n[k * SPLIT + wv % SPLIT][lane];
+            at += k * SPLIT + wv % SPLIT < wv ? x : 0;
+            base += x;
+        }
+        int r = at * SPLIT + wv % SPLIT;
+#pragma unroll
+        for (int k = 0; k < NBR_CHUNK; ++k)
+            if (flags >> k & 1) {
+                crow[(size_t)r * WAVE] = (int)e[k];
+                r += SPLIT;
+            }
+        if (WITH_RHO && wv < SPLIT) {
+            for (int k = wv; k < NW; k += SPLIT) {
+                const int m = cnt - (c0 + k) * NBR_CHUNK;
+                if (m > 0)
+#pragma unroll
+                    for (int x = 0; x < NBR_CHUNK; ++x) {
+                        const float2 f = s_w[k * NBR_CHUNK + x][lane];
+                        sum = fmaf(f.x, f.y, sum);
+                    }
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(cnt > (c0 + NW) * NBR_CHUNK) == 0) break;
+        __syncthreads();                      // the next round reuses the slots
+    }
+    if (wv < SPLIT) {
+        P.ccount[ccount_at(tile, wv, lane)] = base;
+        s_sum[wv][lane] = sum;
+    }
+    __syncthreads();
+    if (wv == 0 && valid) {
+        float tot = s_sum[0][lane];
+#pragma unroll
+        for (int k = 1; k < SPLIT; ++k) tot += s_sum[k][lane];
+        finish_density<WITH_RHO>(P, d, i, pi, tot);
     }
 }
 
@@ -301,15 +424,23 @@ struct Acc {
     __device__ Acc() { for (int k = 0; k < N; ++k) v[k] = 0.f; }
 };
 
+// One pair: displacement, F / r and (EV) its energy.
 // TEST = false: the entry is known to pass the cutoff test (a one-type
 // system's compact row holds exactly the entries with
 // 1e-20 <= r^2 < rc^2, r^2 computed from the same positions by dist2, and
-// the system's largest cutoff is its only one)
+// the system's largest cutoff is its only one).
+// yx: dx.dv starts from the y product, as it does for the odd last entry of
+// the rows (or row parts) that the loops below walk in pairs; its rounding is
+// part of a trajectory, which grows any difference, so every kernel keeps it.
+struct PairF {
+    float dx, dy, dz, fpair, en;
+};
+
 template <int STYLE, bool EV, bool TEST = true>
-__device__ inline void pair_term(Acc<EV> &a, const float4 &pi, const float4 &vi, float rho_i, const float4 &q,
-                                 const float4 &vj, float rho_j, uint32_t code, const PairC &c, float dtis,
-                                 const SysDev *d)
+__device__ inline PairF pair_eval(const float4 &pi, const float4 &vi, float rho_i, const float4 &q, const float4 &vj,
+                                  float rho_j, uint32_t code, const PairC &c, float dtis, const SysDev *d, bool yx)
 {
+    PairF o;
     float dx, dy, dz;
     pair_delta(pi, q, code, d, dx, dy, dz);
     const float rsq = dist2(dx, dy, dz);
@@ -317,7 +448,7 @@ __device__ inline void pair_term(Acc<EV> &a, const float4 &pi, const float4 &vi,
     const float rinv = __builtin_amdgcn_rsqf(rsq);
     const float r = rsq * rinv;
     const float dvx = vi.x - vj.x, dvy = vi.y - vj.y, dvz = vi.z - vj.z;
-    const float dot = dx * dvx + dy * dvy + dz * dvz;
+    const float dot = fmaf(dz, dvz, yx ? fmaf(dx, dvx, dy * dvy) : fmaf(dy, dvy, dx * dvx));
     const float wc = 1.f - r * c.rcinv;
     const float xi = pair_gaussian(__float_as_uint(vi.w), __float_as_uint(vj.w));
     // sigma / sqrt(dt): uniform for a one-type system away from walls
@@ -342,13 +473,86 @@ __device__ inline void pair_term(Acc<EV> &a, const float4 &pi, const float4 &vi,
         fpair = fmaf(c.a, wc, wr * t) * rinv;
         if (EV) en = 0.5f * c.a * c.rc * wc * wc;
     }
-    fpair = in ? fpair : 0.f;
-    a.v[0] += dx * fpair; a.v[1] += dy * fpair; a.v[2] += dz * fpair;
+    o.dx = dx; o.dy = dy; o.dz = dz;
+    o.fpair = in ? fpair : 0.f;
+    o.en = in ? en : 0.f;
+    return o;
+}
+
+// a += the pair's terms.  The fused multiply-adds are spelled out: the two
+// force kernels below sum the same pairs in the same order and must agree
+// bit for bit.
+template <bool EV>
+__device__ inline void pair_add(Acc<EV> &a, const PairF &o)
+{
+    a.v[0] = fmaf(o.dx, o.fpair, a.v[0]);
+    a.v[1] = fmaf(o.dy, o.fpair, a.v[1]);
+    a.v[2] = fmaf(o.dz, o.fpair, a.v[2]);
     if (EV) {
-        a.v[3] += in ? en : 0.f;
-        a.v[4] += dx * dx * fpair; a.v[5] += dy * dy * fpair; a.v[6] += dz * dz * fpair;
-        a.v[7] += dx * dy * fpair; a.v[8] += dx * dz * fpair; a.v[9] += dy * dz * fpair;
+        a.v[3] += o.en;
+        a.v[4] = fmaf(o.dx * o.dx, o.fpair, a.v[4]);
+        a.v[5] = fmaf(o.dy * o.dy, o.fpair, a.v[5]);
+        a.v[6] = fmaf(o.dz * o.dz, o.fpair, a.v[6]);
+        a.v[7] = fmaf(o.dx * o.dy, o.fpair, a.v[7]);
+        a.v[8] = fmaf(o.dx * o.dz, o.fpair, a.v[8]);
+        a.v[9] = fmaf(o.dy * o.dz, o.fpair, a.v[9]);
     }
+}
+
+template <int STYLE, bool EV, bool TEST = true>
+__device__ inline void pair_term(Acc<EV> &a, const float4 &pi, const float4 &vi, float rho_i, const float4 &q,
+                                 const float4 &vj, float rho_j, uint32_t code, const PairC &c, float dtis,
+                                 const SysDev *d, bool yx)
+{
+    pair_add<EV>(a, pair_eval<STYLE, EV, TEST>(pi, vi, rho_i, q, vj, rho_j, code, c, dtis, d, yx));
+}
+
+// Force of particle i known: its outputs (EV) and, in a stepping mode, the
+// half-kicks, drift, next signature (SIG: already known, it reads no
+// velocity) and displacement test.  Returns whether it moved past skin / 2.
+template <int MODE, bool EV, bool STEP, bool SIG>
+__device__ inline int finish_particle(const PoolDev &P, SysDev *d, int i, int cur, const float4 &pi, const float4 &vi,
+                                      int ti, int mk, const Acc<EV> &a, uint32_t sig)
+{
+    float fx = a.v[0], fy = a.v[1], fz = a.v[2];
+    if (mk & d->add_bit) { fx += d->add[0]; fy += d->add[1]; fz += d->add[2]; }
+    if (EV) {
+        P.frc[i] = make_float4(fx, fy, fz, 0.5f * a.v[3]);
+        const size_t cap = (size_t)P.cap;
+        P.vir[i] = 0.5f * a.v[4]; P.vir[cap + i] = 0.5f * a.v[5]; P.vir[2 * cap + i] = 0.5f * a.v[6];
+        P.vir[3 * cap + i] = 0.5f * a.v[7]; P.vir[4 * cap + i] = 0.5f * a.v[8]; P.vir[5 * cap + i] = 0.5f * a.v[9];
+    }
+    if (STEP) {
+        // which half-kicks this pass applies: the pooled engine decides per
+        // system, the plain engine per launch
+        const int ph = MODE == MODE_PHASED ? d->phase : (MODE == MODE_FINAL ? (int)PH_LAST : (int)PH_RUN);
+        float vx = vi.x, vy = vi.y, vz = vi.z;
+        float4 pn = pi;
+        if ((mk & d->nve_bit) && ph != PH_FRESH) {
+            const float dtfm = d->dtf * P.minv[d->mass_base + ti];
+            vx += dtfm * fx; vy += dtfm * fy; vz += dtfm * fz;             // final_integrate
+        }
+        if (ph == PH_LAST) {
+            P.pos[cur ^ 1][i] = pi;
+            P.vel[cur ^ 1][i] = make_float4(vx, vy, vz, vi.w);
+            P.vend[i] = make_float4(vx, vy, vz, 0.f);
+            if (MODE == MODE_PHASED) P.frc[i] = make_float4(fx, fy, fz, 0.f);
+        } else {
+            if (MODE == MODE_FUSED_OUT) P.vend[i] = make_float4(vx, vy, vz, 0.f);
+            if (mk & d->nve_bit) {
+                const float dtfm = d->dtf * P.minv[d->mass_base + ti];
+                vx += dtfm * fx; vy += dtfm * fy; vz += dtfm * fz;         // next initial_integrate
+                pn.x += d->dt * vx; pn.y += d->dt * vy; pn.z += d->dt * vz;
+            }
+            const uint32_t sg = SIG ? sig : next_signature(d, P.tag[d->sela][i], vx, vy, vz);
+            P.pos[cur ^ 1][i] = pn;
+            P.vel[cur ^ 1][i] = make_float4(vx, vy, vz, __uint_as_float(sg));
+            const float4 h = P.xhold[i];
+            const float ex = pn.x - h.x, ey = pn.y - h.y, ez = pn.z - h.z;
+            return fmaf(ez, ez, fmaf(ex, ex, ey * ey)) > d->trig2;
+        }
+    }
+    return 0;
 }
 
 template <int STYLE, int MODE, bool UNI, int SPLIT>
@@ -372,7 +576,7 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
     const int tile = tile0 + lt;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = tile * WAVE + lane;
-    const int s = P.wave_sys[tile];
+    const int s = tile_system(P, tile);
     if (s < 0) return;
     SysDev *d = P.sys + s;
     if (!d->active && MODE != MODE_HARVEST) return;
@@ -453,7 +657,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
                 for (int u = 0; u < 4; ++u) {
                     PairC c = cu;
                     wall_scale(c, j[u]);
-                    pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q[u], vv[u], rj[u], e[u] >> IMG_SHIFT, c, dtis, d);
+                    pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q[u], vv[u], rj[u], e[u] >> IMG_SHIFT, c, dtis, d,
+                                               false);
                 }
             }
         }
@@ -470,8 +675,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
             PairC c1 = UNI ? cu : load_coef(coef, ti * nt + __float_as_int(q1.w));
             wall_scale(c0, j0);
             wall_scale(c1, j1);
-            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q0, w0, r0, e0 >> IMG_SHIFT, c0, dtis, d);
-            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q1, w1, r1, e1 >> IMG_SHIFT, c1, dtis, d);
+            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q0, w0, r0, e0 >> IMG_SHIFT, c0, dtis, d, false);
+            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q1, w1, r1, e1 >> IMG_SHIFT, c1, dtis, d, false);
         }
         if (t < end) {
             const uint32_t e0 = (uint32_t)crow[(size_t)(t * SPLIT + w) * WAVE];
@@ -481,7 +686,7 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
             nbr(j0, q0, r0);
             PairC c0 = UNI ? cu : load_coef(coef, ti * nt + __float_as_int(q0.w));
             wall_scale(c0, j0);
-            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q0, vel[j0], r0, e0 >> IMG_SHIFT, c0, dtis, d);
+            pair_term<STYLE, EV, !UNI>(a, pi, vi, rho_i, q0, vel[j0], r0, e0 >> IMG_SHIFT, c0, dtis, d, true);
         }
     };
     // Lane balance (one wave per tile, one type, no wall scaling): a wave
@@ -534,7 +739,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
                 float rj;
                 nbr(j, q, rj);
                 Acc<EV> b;
-                pair_term<STYLE, EV, !UNI>(b, s_pi[p], s_vi[p], s_ri[p], q, vel[j], rj, e >> IMG_SHIFT, cu, dtis, d);
+                pair_term<STYLE, EV, !UNI>(b, s_pi[p], s_vi[p], s_ri[p], q, vel[j], rj, e >> IMG_SHIFT, cu, dtis, d,
+                                           true);
                 if (act)
                     for (int k = 0; k < NA; ++k) s_tail[k * TAIL_CAP + f] = b.v[k];
             }
@@ -554,47 +760,194 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
                 for (int k = 0; k < NA; ++k) a.v[k] += s_acc[q][k][lane];
     }
     int moved = 0;
-    if (w == 0 && valid) {
-        float fx = a.v[0], fy = a.v[1], fz = a.v[2];
-        if (mk & d->add_bit) { fx += d->add[0]; fy += d->add[1]; fz += d->add[2]; }
-        if (EV) {
-            P.frc[i] = make_float4(fx, fy, fz, 0.5f * a.v[3]);
-            const size_t cap = (size_t)P.cap;
-            P.vir[i] = 0.5f * a.v[4]; P.vir[cap + i] = 0.5f * a.v[5]; P.vir[2 * cap + i] = 0.5f * a.v[6];
-            P.vir[3 * cap + i] = 0.5f * a.v[7]; P.vir[4 * cap + i] = 0.5f * a.v[8]; P.vir[5 * cap + i] = 0.5f * a.v[9];
-        }
-        if (STEP) {
-            // which half-kicks this pass applies: the pooled engine decides per
-            // system, the plain engine per launch
-            const int ph = MODE == MODE_PHASED ? d->phase : (MODE == MODE_FINAL ? (int)PH_LAST : (int)PH_RUN);
-            float vx = vi.x, vy = vi.y, vz = vi.z;
-            float4 pn = pi;
-            if ((mk & d->nve_bit) && ph != PH_FRESH) {
-                const float dtfm = d->dtf * P.minv[d->mass_base + ti];
-                vx += dtfm * fx; vy += dtfm * fy; vz += dtfm * fz;             // final_integrate
-            }
-            if (ph == PH_LAST) {
-                P.pos[cur ^ 1][i] = pi;
-                P.vel[cur ^ 1][i] = make_float4(vx, vy, vz, vi.w);
-                P.vend[i] = make_float4(vx, vy, vz, 0.f);
-                if (MODE == MODE_PHASED) P.frc[i] = make_float4(fx, fy, fz, 0.f);
-            } else {
-                if (MODE == MODE_FUSED_OUT) P.vend[i] = make_float4(vx, vy, vz, 0.f);
-                if (mk & d->nve_bit) {
-                    const float dtfm = d->dtf * P.minv[d->mass_base + ti];
-                    vx += dtfm * fx; vy += dtfm * fy; vz += dtfm * fz;         // next initial_integrate
-                    pn.x += d->dt * vx; pn.y += d->dt * vy; pn.z += d->dt * vz;
-                }
-                const uint32_t sg = next_signature(d, P.tag[d->sela][i], vx, vy, vz);
-                P.pos[cur ^ 1][i] = pn;
-                P.vel[cur ^ 1][i] = make_float4(vx, vy, vz, __uint_as_float(sg));
-                const float4 h = P.xhold[i];
-                const float ex = pn.x - h.x, ey = pn.y - h.y, ez = pn.z - h.z;
-                moved = ex * ex + ey * ey + ez * ez > d->trig2;
-            }
-        }
-    }
+    if (w == 0 && valid) moved = finish_particle<MODE, EV, STEP, false>(P, d, i, cur, pi, vi, ti, mk, a, 0u);
     if (MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) tile_flags(P.moved, tile, 1, moved);
+}
+
+// --------------------------------------------------------------------------
+// The same pass with FW_WAVES waves sharing a tile's compact rows (split 2
+// and 4): lane l of wave k evaluates particle l's pairs of rows k,
+// k + FW_WAVES, ... (row t * SPLIT + w holds entry t of sub-row w), FW_ROWS
+// of them with their gathers in flight at once, and leaves each pair's terms
+// in LDS; then a wave per sub-row and force component adds them in row order,
+// and the sub-rows' sums are added in order, so a particle's sum is that of a
+// loop over its row.  One more wave computes the mDPD signatures of the next
+// step meanwhile (they read only the tags).
+// --------------------------------------------------------------------------
+constexpr int FW_WAVES = 8, FW_ROWS = 5;
+
+template <int STYLE, int MODE, bool UNI, int SPLIT>
+__global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P, int tile0, int ntiles)
+{
+    constexpr bool EV = MODE != MODE_FUSED && MODE != MODE_PHASED;
+    constexpr bool STEP = MODE != MODE_SETUP && MODE != MODE_HARVEST;
+    constexpr int NA = Acc<EV>::N;
+    constexpr int R = FW_WAVES * FW_ROWS;              // rows per round
+    constexpr int NU = EV ? SPLIT : 3 * SPLIT;         // sums: sub-row x component (EV: all components)
+    constexpr int UPW = (NU + FW_WAVES - 1) / FW_WAVES;
+    static_assert(FW_WAVES % SPLIT == 0, "a wave's rows belong to one sub-row");
+    __shared__ float s_d[3][R][WAVE], s_f[R][WAVE];    // dx, dy, dz and F / r of each pair
+    __shared__ float s_en[EV ? R : 1][WAVE];
+    __shared__ float s_acc[SPLIT][NA][WAVE];
+    __shared__ uint32_t s_sig[WAVE];
+    const int lt = xcd_logical(blockIdx.x, ntiles);
+    if (lt >= ntiles) return;
+    const int tile = tile0 + lt;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int i = tile * WAVE + lane;
+    const int s = tile_system(P, tile);
+    if (s < 0) return;
+    SysDev *d = P.sys + s;
+    if (!d->active && MODE != MODE_HARVEST) return;
+    if (UNI != (d->ntypes == 1)) return;     // host launches the matching variant
+    if (STEP && d->overflow) return;
+    if (MODE == MODE_PHASED && d->style != STYLE) return;
+    if (MODE == MODE_HARVEST && d->split_last != SPLIT) return;
+    const bool valid = i < d->part_base + d->n;
+    const int cur = MODE == MODE_HARVEST ? d->sel ^ 1 : d->sel;
+    const float4 *pos = P.pos[cur];
+    const float4 *vel = P.vel[cur];
+    const int *maskv = P.mask[d->sela];
+    int n[SPLIT];
+#pragma unroll
+    for (int w = 0; w < SPLIT; ++w) n[w] = valid ? P.ccount[ccount_at(tile, w, lane)] : 0;
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), vi = pi;
+    float rho_i = 0.f, phi_i = 0.f;
+    int mk = 0;
+    if (valid) {
+        pi = pos[i];
+        vi = vel[i];
+        mk = maskv[i];
+        if (STYLE == STYLE_MDPD) rho_i = P.rho[i];
+    }
+    if (wv == FW_WAVES && STEP && STYLE == STYLE_MDPD)
+        s_sig[lane] = valid ? sig_mdpd(P.tag[d->sela][i], d->seed_next) : 0u;
+    // a mobile particle's wall fraction scales its pairs with wall particles
+    // (pair_mdpd_meso.cu:169-185)
+    const bool arb_i = STYLE == STYLE_MDPD && d->pair_arb && (mk & d->pair_mobile_bit);
+    if (arb_i) phi_i = P.phi[d->sela][i];
+    const int ti = __float_as_int(pi.w);
+    const float dtis = d->dtinvsqrt;
+    const float *coef = P.coef + d->coef_base;
+    const int nt = d->ntypes, wall_bit = d->pair_wall_bit;
+    PairC cu;
+    if (UNI) cu = load_coef(coef, 0);
+    const int maxnbr = P.maxnbr;
+    const int *crow = P.clist + (size_t)tile * maxnbr * WAVE + lane;
+    int nmax = n[0], nw = n[0];
+#pragma unroll
+    for (int w = 1; w < SPLIT; ++w) {
+        nmax = max(nmax, n[w]);
+        nw = wv % SPLIT == w ? n[w] : nw;
+    }
+    Acc<EV> a;                                // EV: all components of one sub-row
+    float sum[UPW];
+#pragma unroll
+    for (int k = 0; k < UPW; ++k) sum[k] = 0.f;
+    for (int r0 = 0;; r0 += R) {
+        if (wv < FW_WAVES) {
+            uint32_t e[FW_ROWS];
+            float4 q[FW_ROWS], vv[FW_ROWS];
+            float rj[FW_ROWS];
+#pragma unroll
+            for (int u = 0; u < FW_ROWS; ++u) {
+                const int r = r0 + u * FW_WAVES + wv;
+                // a lane without this row takes itself (stored nowhere)
+                e[u] = (uint32_t)i | ((uint32_t)IMG_ZERO << IMG_SHIFT);
+                if (r / SPLIT < nw) e[u] = (uint32_t)crow[(size_t)r * WAVE];
+            }
+#pragma unroll
+            for (int u = 0; u < FW_ROWS; ++u) {
+                const uint32_t j = e[u] & IDX_MASK;
+                if (UNI && STYLE == STYLE_MDPD) {
+                    q[u] = P.pr[j];
+                    rj[u] = q[u].w;
+                } else {
+                    q[u] = pos[j];
+                    rj[u] = STYLE == STYLE_MDPD ? P.rho[j] : 0.f;
+                }
+                vv[u] = vel[j];
+            }
+#pragma unroll
+            for (int u = 0; u < FW_ROWS; ++u) {
+                const int r = r0 + u * FW_WAVES + wv;
+                const bool on = r / SPLIT < nw;
+                if (__builtin_amdgcn_ballot_w64(on) == 0) break;
+                PairC c;
+                if (UNI) c = cu;
+                else c = load_coef(coef, ti * nt + (on ? __float_as_int(q[u].w) : 0));
+                if (arb_i && (maskv[e[u] & IDX_MASK] & wall_bit)) {
+                    const float ratio = wall_ratio(phi_i, c.rc);
+                    c.gamma *= ratio;
+                    c.sigma *= __builtin_amdgcn_sqrtf(ratio);
+                }
+                const PairF o = pair_eval<STYLE, EV, !UNI>(pi, vi, rho_i, q[u], vv[u], rj[u], e[u] >> IMG_SHIFT, c,
+                                                           dtis, d, (nw & 1) && r / SPLIT == nw - 1);
+                const int k = u * FW_WAVES + wv;
+                s_d[0][k][lane] = o.dx;
+                s_d[1][k][lane] = o.dy;
+                s_d[2][k][lane] = o.dz;
+                s_f[k][lane] = o.fpair;
+                if (EV) s_en[k][lane] = o.en;
+            }
+        }
+        __syncthreads();
+        if (EV) {
+            if (wv < SPLIT)
+                for (int k = wv; k < R && (r0 + k) / SPLIT < nw; k += SPLIT) {
+                    PairF o;
+                    o.dx = s_d[0][k][lane]; o.dy = s_d[1][k][lane]; o.dz = s_d[2][k][lane];
+                    o.fpair = s_f[k][lane]; o.en = s_en[k][lane];
+                    pair_add<EV>(a, o);
+                }
+        } else if (wv < FW_WAVES) {
+#pragma unroll
+            for (int y = 0; y < UPW; ++y) {
+                // component comp of sub-row wv % SPLIT
+                const int comp = (y * FW_WAVES + wv) / SPLIT;
+                if (comp < 3)
+                    for (int k0 = wv % SPLIT; k0 < R; k0 += 4 * SPLIT) {
+                        if (__builtin_amdgcn_ballot_w64((r0 + k0) / SPLIT < nw) == 0) break;
+                        float x[4], f[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const int k = min(k0 + u * SPLIT, R - 1);
+                            x[u] = s_d[comp][k][lane];
+                            f[u] = s_f[k][lane];
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const int k = k0 + u * SPLIT;
+                            sum[y] = k < R && (r0 + k) / SPLIT < nw ? fmaf(x[u], f[u], sum[y]) : sum[y];
+                        }
+                    }
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(nmax * SPLIT > r0 + R) == 0) break;
+        __syncthreads();                      // the next round reuses the slots
+    }
+    if (EV) {
+        if (wv < SPLIT)
+            for (int k = 0; k < NA; ++k) s_acc[wv][k][lane] = a.v[k];
+    } else if (wv < FW_WAVES) {
+#pragma unroll
+        for (int y = 0; y < UPW; ++y)
+            if ((y * FW_WAVES + wv) / SPLIT < 3) s_acc[wv % SPLIT][(y * FW_WAVES + wv) / SPLIT][lane] = sum[y];
+    }
+    __syncthreads();
+    if (wv > 0) return;
+    for (int k = 0; k < NA; ++k) {
+        a.v[k] = s_acc[0][k][lane];
+#pragma unroll
+        for (int w = 1; w < SPLIT; ++w) a.v[k] += s_acc[w][k][lane];
+    }
+    int moved = 0;
+    if (valid)
+        moved = finish_particle<MODE, EV, STEP, STYLE == STYLE_MDPD>(P, d, i, cur, pi, vi, ti, mk, a, s_sig[lane]);
+    if (MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) {
+        const uint64_t any = __builtin_amdgcn_ballot_w64(moved != 0);
+        if (lane == 0) P.moved[tile] = any != 0 ? 1 : 0;
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -841,13 +1194,33 @@ __global__ void k_premix(const uint32_t *a, const uint32_t *b, uint32_t *out, in
 // ----------------------------------------------------------------------------
 // launchers
 // ----------------------------------------------------------------------------
-template <int SPLIT>
-static void launch_first_t(const PoolDev &P, bool with_rho, int nt, hipStream_t st)
+// Tiles up to which a split of 2 or 4 takes the wide kernels: two of their
+// workgroups per CU, all of them resident at once.  A short launch is one
+// tile's chain of loads and of ~6.5 cycles per dependent instruction, which
+// the wide kernels cut (16 tiles: first pass 10.9 -> 6.8 us, force pass 12.5
+// -> 7.3 us; 500 tiles of the DPD fluid: step 1.04x faster); past that their
+// tiles queue and the two-wave kernels' occupancy wins (626 tiles: 13.4 and
+// 15.3 us against 13.2 and 16.3; 1,513 tiles: step 0.89x).
+constexpr int WIDE_TILES = 512;
+
+template <bool WITH_RHO>
+static hipError_t launch_first_t(const PoolDev &P, int split, int nt, hipStream_t st)
 {
-    if (with_rho)
-        hipLaunchKernelGGL((k_first<true, SPLIT>), dim3(xcd_grid(nt)), dim3(WAVE * SPLIT), 0, st, P, nt);
+    const dim3 g(xcd_grid(nt));
+    const bool wide = nt <= WIDE_TILES;
+    if (split == 1)
+        hipLaunchKernelGGL((k_first<WITH_RHO, 1>), g, dim3(WAVE), 0, st, P, nt);
+    else if (split == 2 && wide)
+        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 2>), g, dim3(WAVE * FS_WAVES<2>), 0, st, P, nt);
+    else if (split == 2)
+        hipLaunchKernelGGL((k_first<WITH_RHO, 2>), g, dim3(WAVE * 2), 0, st, P, nt);
+    else if (split == 4 && wide)
+        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 4>), g, dim3(WAVE * FS_WAVES<4>), 0, st, P, nt);
+    else if (split == 4)
+        hipLaunchKernelGGL((k_first<WITH_RHO, 4>), g, dim3(WAVE * 4), 0, st, P, nt);
     else
-        hipLaunchKernelGGL((k_first<false, SPLIT>), dim3(xcd_grid(nt)), dim3(WAVE * SPLIT), 0, st, P, nt);
+        return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 hipError_t launch_first(const PoolDev &P, bool with_rho, int split, hipStream_t st)
@@ -855,13 +1228,7 @@ hipError_t launch_first(const PoolDev &P, bool with_rho, int split, hipStream_t 
     const int nt = P.nact / WAVE;
     if (nt == 0) return hipSuccess;
     if (P.maxnbr % NBR_ALIGN) return hipErrorInvalidValue;   // a split wave's compact rows must fit
-    switch (split) {
-    case 1: launch_first_t<1>(P, with_rho, nt, st); break;
-    case 2: launch_first_t<2>(P, with_rho, nt, st); break;
-    case 4: launch_first_t<4>(P, with_rho, nt, st); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return with_rho ? launch_first_t<true>(P, split, nt, st) : launch_first_t<false>(P, split, nt, st);
 }
 
 hipError_t launch_commit_step(const PoolDev &P, int kind, int split, hipStream_t st)
@@ -896,25 +1263,31 @@ hipError_t launch_initial(const PoolDev &P, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int STYLE, int MODE, int SPLIT>
-static void launch_force_t(const PoolDev &P, bool uni, int t0, int nt, hipStream_t st)
+template <int STYLE, int MODE, bool UNI>
+static hipError_t launch_force_t(const PoolDev &P, int split, int t0, int nt, hipStream_t st)
 {
-    if (uni)
-        hipLaunchKernelGGL((k_force<STYLE, MODE, true, SPLIT>), dim3(xcd_grid(nt)), dim3(WAVE * SPLIT), 0, st, P, t0, nt);
+    const dim3 g(xcd_grid(nt)), bw(WAVE * (FW_WAVES + 1));
+    const bool wide = nt <= WIDE_TILES;
+    if (split == 1)
+        hipLaunchKernelGGL((k_force<STYLE, MODE, UNI, 1>), g, dim3(WAVE), 0, st, P, t0, nt);
+    else if (split == 2 && wide)
+        hipLaunchKernelGGL((k_force_wide<STYLE, MODE, UNI, 2>), g, bw, 0, st, P, t0, nt);
+    else if (split == 2)
+        hipLaunchKernelGGL((k_force<STYLE, MODE, UNI, 2>), g, dim3(WAVE * 2), 0, st, P, t0, nt);
+    else if (split == 4 && wide)
+        hipLaunchKernelGGL((k_force_wide<STYLE, MODE, UNI, 4>), g, bw, 0, st, P, t0, nt);
+    else if (split == 4)
+        hipLaunchKernelGGL((k_force<STYLE, MODE, UNI, 4>), g, dim3(WAVE * 4), 0, st, P, t0, nt);
     else
-        hipLaunchKernelGGL((k_force<STYLE, MODE, false, SPLIT>), dim3(xcd_grid(nt)), dim3(WAVE * SPLIT), 0, st, P, t0, nt);
+        return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 template <int STYLE, int MODE>
 static hipError_t launch_force_s(const PoolDev &P, bool uni, int split, int t0, int nt, hipStream_t st)
 {
-    switch (split) {
-    case 1: launch_force_t<STYLE, MODE, 1>(P, uni, t0, nt, st); break;
-    case 2: launch_force_t<STYLE, MODE, 2>(P, uni, t0, nt, st); break;
-    case 4: launch_force_t<STYLE, MODE, 4>(P, uni, t0, nt, st); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return uni ? launch_force_t<STYLE, MODE, true>(P, split, t0, nt, st)
+               : launch_force_t<STYLE, MODE, false>(P, split, t0, nt, st);
 }
 
 hipError_t launch_force(const PoolDev &P, int style, int mode, bool uni, int split, hipStream_t st)
