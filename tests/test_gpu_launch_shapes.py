@@ -74,3 +74,25 @@ def test_small_system_equals_its_pool_job(engine, case, split):
         np.testing.assert_array_equal(p.gather(j, k), a, err_msg=f"{case}, split {split}: {k}")
     p.close()
     s.close()
+
+
+# (particles, box edge): sub-cells of one scan chunk, just past it, several
+# chunks, and past the largest count the one-launch scan takes
+@pytest.mark.parametrize("n, L", [(300, 5.3), (2000, 13.1), (2000, 14.4), (3000, 27.5), (4000, 46.0)])
+def test_sorted_order_over_scan_sizes(engine, orc, n, L):
+    x, v = uniform_box(n, L, int(10 * L))
+    s = mdpd_system(engine, x, v, L)
+    s.setup()
+    xc = orc.wrap(x.astype(np.float32), (0, 0, 0), (L, L, L))
+    keys = orc.sort_keys(xc, (0, 0, 0), (L, L, L), 1.3)
+    origin, got, _ = s.debug_sorted()
+    assert np.array_equal(origin, orc.stable_sort(keys))
+    assert np.array_equal(got, keys[origin])
+    # after re-sorts on the step path every table still belongs to its positions
+    s.run(30)
+    assert s.nbuild >= 2
+    origin, got, xw = s.debug_sorted()
+    assert np.array_equal(np.sort(origin), np.arange(n))
+    assert np.array_equal(got, orc.sort_keys(xw, (0, 0, 0), (L, L, L), 1.3))
+    assert np.all(np.diff(got.astype(np.int64)) >= 0)
+    s.close()

@@ -64,7 +64,7 @@ __device__ inline int xcd_logical(int b, int nlogical)
     const int per = (nlogical + NXCD - 1) / NXCD;
     return (b % NXCD) * per + b / NXCD;
 }
-static inline int xcd_grid(int nlogical) { return ((nlogical + NXCD - 1) / NXCD) * NXCD; }
+__host__ __device__ inline int xcd_grid(int nlogical) { return ((nlogical + NXCD - 1) / NXCD) * NXCD; }
 
 // inclusive prefix sum over the 64 lanes of a wave (every lane active)
 __device__ inline int wave_incl_scan(int x, int lane)
@@ -134,6 +134,7 @@ struct SysDev {
     int steps_left;              // pooled engine: steps still to run
     long long step;              // ntimestep of the next / current force evaluation
     uint32_t seed_next;          // premix_TEA<64>(seed, step + 1)
+    uint32_t seed_after;         // premix_TEA<64>(seed, step + 2) (next_seeds)
     uint32_t seed_cur;           // premix_TEA<64>(seed, step): signatures of a fresh system
     int phase;                   // pooled engine: PH_FRESH / PH_RUN / PH_LAST / PH_DONE
     int job;                     // pooled engine: caller's job id of this slot
@@ -188,7 +189,7 @@ struct PoolDev {
     int *cell_sys;       // system of each cell slot
     int4 *cell_work;     // pools: the cells holding particles of the systems re-sorted this pass, as
                          // (system, packed coordinates, first particle, end) (k_scan_apply appends)
-    int *work_count;     // [0]: entries of cell_work (k_keys clears it)
+    int *work_count;     // [0]: entries of cell_work (k_keys clears it); [1]: one system: list its rows (k_keys)
     int2 *cell_lse;      // pools: particle range [start, end) of each cell by linear cell id (cell_base + lin)
     int *nlist;         // (cap/64) tiles * maxnbr * 64
     int *ncount;         // per particle
@@ -211,6 +212,7 @@ struct PoolDev {
     int nsys;            // descriptor slots [0, nsys) hold systems: extent of per-system launches
     int maxsub;          // sub-cell slots of the largest system (0: all cell slots, one system)
     int maxnbr;
+    int one;             // one system (slot 0) holds every tile and cell slot: the plain engine
 };
 
 // ----------------------------------------------------------------------------
@@ -244,6 +246,21 @@ __host__ inline uint32_t premix_host(uint32_t v0, uint32_t v1, int rounds)
 {
     tea_rounds(v0, v1, rounds);
     return v0 ^ v1;
+}
+
+// Lane s of workgroup k computes the seed two steps on of system 64 k + s, for
+// the step's commit.  64 TEA rounds are a chain of ~700 dependent instructions,
+// 2.5 us of a commit that every step waits for, so a spare workgroup of a
+// kernel that takes longer computes them: of the first pass (split 1 and the
+// wide kernels), else of the one system's row build.  (In the two- and
+// four-wave first passes it costs registers: 72 VGPRs, a wave per SIMD less,
+// 480,000 particles 83 -> 98 us.)
+__device__ inline void next_seeds(const PoolDev &P, int k)
+{
+    const int s = k * WAVE + threadIdx.x;
+    if (threadIdx.x >= WAVE || s >= P.nsys) return;
+    SysDev *d = P.sys + s;
+    if (d->active) d->seed_after = premix<64>(d->seed, (uint32_t)(d->step + 2));
 }
 
 __device__ inline uint32_t brev32(uint32_t x) { return __builtin_bitreverse32(x); }

@@ -22,12 +22,11 @@ enum CommitKind : int {
     COMMIT_DECIDE = 3,   // plain engine: COMMIT_ADVANCE with the reneighbor decision
 };
 
-// rebuild phase: wrap, keys, sort, gather, neighbor rows (stale systems only)
-hipError_t launch_rebuild(const PoolDev &P, hipStream_t st);
+// rebuild phase: wrap, keys, sort, gather, neighbor rows, commit (stale systems only)
+hipError_t launch_rebuild(const PoolDev &P, int split, hipStream_t st);
 hipError_t launch_nlist_only(const PoolDev &P, hipStream_t st);
 // neighbor rows of every sorted active system rebuilt in place (row width grew)
 hipError_t launch_relist(const PoolDev &P, hipStream_t st);
-hipError_t launch_commit_rebuild(const PoolDev &P, hipStream_t st);
 hipError_t launch_signatures(const PoolDev &P, hipStream_t st);
 
 // per step
@@ -35,8 +34,12 @@ hipError_t launch_signatures(const PoolDev &P, hipStream_t st);
 hipError_t launch_first(const PoolDev &P, bool with_rho, int split, hipStream_t st);
 hipError_t launch_initial(const PoolDev &P, hipStream_t st);
 // after launch_initial / a fused force pass (advance) or a final pass (!advance)
-// kind: CommitKind; split = waves per tile of the pass
-hipError_t launch_commit_step(const PoolDev &P, int kind, int split, hipStream_t st);
+// kind: CommitKind; split = waves per tile of the pass; after_pass: a rebuild
+// phase and a first pass of that split have run since the last commit
+hipError_t launch_commit_step(const PoolDev &P, int kind, int split, bool after_pass, hipStream_t st);
+// whether a first pass of this split over nt tiles computes the seeds the
+// step's commit moves on to; otherwise, for one system, the row build does
+bool first_seeds(int split, int nt);
 hipError_t launch_force(const PoolDev &P, int style, int mode, bool uni, int split, hipStream_t st);
 // the same over the 64-particle tiles [tile0, tile0 + ntiles) only
 hipError_t launch_force_range(const PoolDev &P, int style, int mode, bool uni, int split, int tile0, int ntiles,

@@ -19,7 +19,7 @@ namespace mdpd {
 // The neighbor-row build of a pool walks a worklist of the cells to list
 // (k_scan_apply appends them); one system (the plain path) keeps one wave
 // per cell slot: its slots are few and the list would only add its own cost.
-__host__ __device__ inline bool nlist_listed(const PoolDev &P) { return P.nsys > 1; }
+__host__ __device__ inline bool nlist_listed(const PoolDev &P) { return !P.one; }
 
 // --------------------------------------------------------------------------
 // K1: wrap into the box (Domain::pbc in FP32), reference sort key, sub-cell
@@ -29,9 +29,14 @@ __host__ __device__ inline bool nlist_listed(const PoolDev &P) { return P.nsys >
 __global__ void __launch_bounds__(256) k_keys(PoolDev P)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0 && P.work_count) *P.work_count = 0;        // this rebuild's worklist starts empty
+    if (i == 0) {
+        P.work_count[0] = 0;                              // this rebuild's worklist starts empty
+        // one system: the row build's waves read this word, not the flag that
+        // their commit clears
+        if (P.one) P.work_count[1] = P.sys->active && P.sys->stale ? 1 : 0;
+    }
     if (i >= P.nact) return;
-    const int s = P.wave_sys[i >> 6];
+    const int s = P.one ? 0 : P.wave_sys[i >> 6];
     if (s < 0) return;
     SysDev *d = P.sys + s;
     if (!d->active || !d->stale) return;
@@ -270,17 +275,66 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
 }
 
 // --------------------------------------------------------------------------
-// K3: scatter particle indices into their sub-cell segments (arrival order),
-// the sub-bin key beside each (cl is free once k_scan has used it).
+// The same scan for one system in one launch: workgroup g adds up all the
+// counts before its chunk itself, which costs it reads (two rounds of loads
+// for the 54,000 sub-cells of a 97,000-particle slab) where k_scan_sums and
+// k_scan_chunks cost a launch each, 1.6 us idle and 4.7 us working.  Other
+// workgroups may still read a chunk's counts, so k_scatter clears them.
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_scatter(PoolDev P)
+constexpr int SCAN1_BLK = 1024, SCAN1_CH = SCAN1_BLK * 4;
+constexpr int SCAN1_MAX = 40;          // chunks: past that the last workgroup's reads (10 rounds) cost the launches saved
+
+__global__ void __launch_bounds__(SCAN1_BLK) k_scan_one(PoolDev P)
+{
+    const SysDev *d = P.sys;
+    if (!d->active || !d->stale) return;
+    __shared__ int s_before[SCAN1_BLK / WAVE], s_own[SCAN1_BLK / WAVE];
+    const int nc = d->ncell * SUBCELLS;                    // a multiple of four
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int c0 = blockIdx.x * SCAN1_CH, c = c0 + 4 * t;
+    const int4 *cnt4 = (const int4 *)P.cell_count;
+    int before = 0;
+    for (int k = 0; k < c0; k += 4 * SCAN1_CH) {
+        int4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            v[u] = k + u * SCAN1_CH < c0 ? cnt4[(k + u * SCAN1_CH) / 4 + t] : make_int4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) before += v[u].x + v[u].y + v[u].z + v[u].w;
+    }
+    const int4 own = c < nc ? cnt4[c / 4] : make_int4(0, 0, 0, 0);
+    const int sum = own.x + own.y + own.z + own.w;
+    const int incl = wave_incl_scan(sum, lane);
+    before = wave_sum(before);
+    if (lane == 63) {
+        s_own[wv] = incl;
+        s_before[wv] = before;
+    }
+    __syncthreads();
+    int run = d->part_base + incl - sum;
+    for (int k = 0; k < SCAN1_BLK / WAVE; ++k) run += s_before[k] + (k < wv ? s_own[k] : 0);
+    if (c < nc) {
+        const int4 st = make_int4(run, run + own.x, run + own.x + own.y, run + own.x + own.y + own.z);
+        ((int4 *)P.cell_start)[c / 4] = st;
+        if (c + 4 == nc) P.cell_start[nc] = d->part_base + d->n;
+    }
+}
+
+// --------------------------------------------------------------------------
+// K3: scatter particle indices into their sub-cell segments (arrival order),
+// the sub-bin key beside each (cl is free once k_scan has used it); with
+// `clear` the sub-cell counts of the one system are cleared here.
+// --------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_scatter(PoolDev P, int clear)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P.nact) return;
-    const int s = P.wave_sys[i >> 6];
+    const int s = P.one ? 0 : P.wave_sys[i >> 6];
     if (s < 0) return;
     SysDev *d = P.sys + s;
     if (!d->active || !d->stale) return;
+    if (clear)
+        for (int c = i; c < d->ncell * SUBCELLS; c += P.nact) P.cell_count[c] = 0;
     if (i >= d->part_base + d->n) return;
     const int f = P.cell_start[P.pcell[i]] + P.pslot[i];
     P.tmp[f] = i;
@@ -300,7 +354,7 @@ __global__ void __launch_bounds__(256) k_sortgather(PoolDev P)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P.nact) return;
-    const int s = P.wave_sys[i >> 6];
+    const int s = P.one ? 0 : P.wave_sys[i >> 6];
     if (s < 0) return;
     const SysDev *d = P.sys + s;
     if (!d->active || !d->stale) return;
@@ -407,7 +461,9 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
     SysDev *d = P.sys + s;
     const int cb = d->cell_base;
     if (!LISTED) {
-        if (!d->active || (relist ? d->stale != 0 : d->stale == 0)) return;
+        // relist: the systems not flagged stale; otherwise the one system when
+        // k_keys found it stale
+        if (!d->active || (relist ? d->stale != 0 : P.work_count[1] == 0)) return;
         if (cs < cb || cs >= cb + d->ncell) return;       // the end slot holds no cell
         c0 = P.cell_start[cs * SUBCELLS];
         c1 = P.cell_start[(cs + 1) * SUBCELLS];
@@ -531,15 +587,6 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
     }
 }
 
-// one wave per cell slot (a relist, or one system): eight waves per SIMD
-// (seven candidate tiles in registers, no spills), measured faster than seven
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) k_nlist(PoolDev P, int relist, int ncells)
-{
-    __shared__ int s_row[NL_ITER * WAVE];                   // one centre's entries of one batch
-    const int cs = xcd_logical(blockIdx.x, ncells);        // cell slot (Morton rank order)
-    if (cs < ncells) nlist_cell<false>(P, make_int4(cs, 0, 0, 0), relist, s_row);
-}
-
 // Commit after a rebuild: the sorted data in the other buffers becomes current.
 __device__ inline void commit_rebuild_sys(const PoolDev &P, int s)
 {
@@ -550,6 +597,19 @@ __device__ inline void commit_rebuild_sys(const PoolDev &P, int s)
     d->stale = 0;
     d->ago = 0;
     d->builds += 1;
+}
+
+// one wave per cell slot (a relist, or one system): eight waves per SIMD
+// (seven candidate tiles in registers, no spills), measured faster than seven
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) k_nlist(PoolDev P, int relist, int ncells)
+{
+    __shared__ int s_row[NL_ITER * WAVE];                   // one centre's entries of one batch
+    // the one system's rebuild is committed here: the row build reads only its
+    // geometry and the flag word
+    if (!relist && blockIdx.x == 0 && threadIdx.x == 0 && P.work_count[1]) commit_rebuild_sys(P, 0);
+    if ((int)blockIdx.x >= xcd_grid(ncells)) { next_seeds(P, 0); return; }
+    const int cs = xcd_logical(blockIdx.x, ncells);        // cell slot (Morton rank order)
+    if (cs < ncells) nlist_cell<false>(P, make_int4(cs, 0, 0, 0), relist, s_row);
 }
 
 // the worklist walk; it also commits the rebuild of every re-sorted system
@@ -578,15 +638,6 @@ __global__ void k_clear_overflow(PoolDev P)
 }
 
 // --------------------------------------------------------------------------
-// Commit after a rebuild with one wave per cell slot (the plain path)
-// --------------------------------------------------------------------------
-__global__ void k_commit_rebuild(PoolDev P)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < P.nsys) commit_rebuild_sys(P, s);
-}
-
-// --------------------------------------------------------------------------
 // Signatures of the current step (setup only; in the step loop the fused
 // force epilogue writes them for the following step).
 // --------------------------------------------------------------------------
@@ -610,38 +661,44 @@ __global__ void __launch_bounds__(256) k_signatures(PoolDev P)
 // host launchers
 // ----------------------------------------------------------------------------
 static inline int nblk(int n, int b) { return (n + b - 1) / b; }
-static void launch_nlist(const PoolDev &P, int relist, hipStream_t st)
+static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t st)
 {
     if (P.ncact <= 0) return;
     if (relist || !nlist_listed(P))
-        hipLaunchKernelGGL(k_nlist, dim3(xcd_grid(P.ncact)), dim3(WAVE), 0, st, P, relist, P.ncact);
+        hipLaunchKernelGGL(k_nlist, dim3(xcd_grid(P.ncact) + (seeds ? 1 : 0)), dim3(WAVE), 0, st, P, relist,
+                           P.ncact);
     else
         hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(P.ncact))), dim3(WAVE), 0, st, P);
 }
 
-hipError_t launch_rebuild(const PoolDev &P, hipStream_t st)
+hipError_t launch_rebuild(const PoolDev &P, int split, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
     const dim3 g(nblk(P.nact, 256)), b(256);
     hipLaunchKernelGGL(k_keys, g, b, 0, st, P);
-    // workgroups per system for the chunked scan: as many as the largest
-    // system has chunks, up to 64 (smaller systems' extra workgroups exit)
     const long long nsub = P.maxsub > 0 ? (long long)P.maxsub : (long long)P.ncellslots * SUBCELLS;
-    const int nch = (int)((nsub + SCAN_CH - 1) / SCAN_CH);
-    const int gs = std::max(1, std::min(64, nch));
-    hipLaunchKernelGGL(k_scan_sums, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
-    hipLaunchKernelGGL(k_scan_chunks, dim3(P.nsys), dim3(SCAN_BLK), 0, st, P);
-    hipLaunchKernelGGL(k_scan_apply, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
-    hipLaunchKernelGGL(k_scatter, g, b, 0, st, P);
+    const bool scan_one = P.one && nblk((int)nsub, SCAN1_CH) <= SCAN1_MAX;
+    if (scan_one) {
+        hipLaunchKernelGGL(k_scan_one, dim3(nblk((int)nsub, SCAN1_CH)), dim3(SCAN1_BLK), 0, st, P);
+    } else {
+        // workgroups per system for the chunked scan: as many as the largest
+        // system has chunks, up to 64 (smaller systems' extra workgroups exit)
+        const int nch = (int)((nsub + SCAN_CH - 1) / SCAN_CH);
+        const int gs = std::max(1, std::min(64, nch));
+        hipLaunchKernelGGL(k_scan_sums, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
+        hipLaunchKernelGGL(k_scan_chunks, dim3(P.nsys), dim3(SCAN_BLK), 0, st, P);
+        hipLaunchKernelGGL(k_scan_apply, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
+    }
+    hipLaunchKernelGGL(k_scatter, g, b, 0, st, P, scan_one ? 1 : 0);
     hipLaunchKernelGGL(k_sortgather, g, b, 0, st, P);
-    launch_nlist(P, 0, st);
+    launch_nlist(P, 0, P.one && !first_seeds(split, P.nact / WAVE), st);
     return hipGetLastError();
 }
 
 hipError_t launch_nlist_only(const PoolDev &P, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
-    launch_nlist(P, 0, st);
+    launch_nlist(P, 0, false, st);
     return hipGetLastError();
 }
 
@@ -649,15 +706,7 @@ hipError_t launch_relist(const PoolDev &P, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
     hipLaunchKernelGGL(k_clear_overflow, dim3(nblk(P.nsys, 64)), dim3(64), 0, st, P);
-    launch_nlist(P, 1, st);
-    return hipGetLastError();
-}
-
-hipError_t launch_commit_rebuild(const PoolDev &P, hipStream_t st)
-{
-    // after a worklist walk the commit has been made by the walk itself
-    if (nlist_listed(P) && P.ncact > 0 && P.nact > 0) return hipSuccess;
-    hipLaunchKernelGGL(k_commit_rebuild, dim3(nblk(P.nsys, 64)), dim3(64), 0, st, P);
+    launch_nlist(P, 1, false, st);
     return hipGetLastError();
 }
 

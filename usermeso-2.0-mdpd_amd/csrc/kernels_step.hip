@@ -107,7 +107,7 @@ __device__ inline float2 weight_factors(float h, float rsq, bool lucy)
 }
 
 // system of a tile; one system (the plain path) holds them all
-__device__ inline int tile_system(const PoolDev &P, int tile) { return P.nsys == 1 ? 0 : P.wave_sys[tile]; }
+__device__ inline int tile_system(const PoolDev &P, int tile) { return P.one ? 0 : P.wave_sys[tile]; }
 
 // density of particle i from its weight sum, and the record the force pass of
 // a one-type system gathers (position and density in one 16-byte load)
@@ -132,6 +132,10 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
     constexpr int STAGE = 32 / SPLIT;   // LDS-staged compact entries per lane (measured best)
     __shared__ int s_c[SPLIT][STAGE * WAVE];
     __shared__ float s_sum[SPLIT][WAVE];
+    if (SPLIT == 1 && (int)blockIdx.x >= xcd_grid(ntiles)) {
+        next_seeds(P, blockIdx.x - xcd_grid(ntiles));
+        return;
+    }
     const int tile = xcd_logical(blockIdx.x, ntiles);
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -265,6 +269,7 @@ __global__ void __launch_bounds__(WAVE * FS_WAVES<SPLIT>) k_first_wide(PoolDev P
     __shared__ float2 s_w[WITH_RHO ? NW * NBR_CHUNK : 1][WAVE];    // weight factors of each entry
     __shared__ int s_n[NW][WAVE];                                  // in-cutoff entries of each chunk
     __shared__ float s_sum[SPLIT][WAVE];
+    if ((int)blockIdx.x >= xcd_grid(ntiles)) { next_seeds(P, blockIdx.x - xcd_grid(ntiles)); return; }
     const int tile = xcd_logical(blockIdx.x, ntiles);
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -359,11 +364,12 @@ __device__ inline uint32_t next_signature(const SysDev *d, int tag, float vx, fl
     return d->style == STYLE_MDPD ? sig_mdpd(tag, d->seed_next) : sig_dpd(tag, d->seed_next, vx, vy, vz);
 }
 
-__device__ inline void commit_advance(SysDev *d, bool moved)
+// seeded: a kernel of the step left the seed two steps on in seed_after
+__device__ inline void commit_advance(SysDev *d, bool moved, bool seeded)
 {
     d->sel ^= 1;
     d->step += 1;
-    d->seed_next = premix<64>(d->seed, (uint32_t)(d->step + 1));
+    d->seed_next = seeded ? d->seed_after : premix<64>(d->seed, (uint32_t)(d->step + 1));
     d->stale = moved ? 1 : 0;
 }
 
@@ -1075,7 +1081,7 @@ __global__ void __launch_bounds__(WAVE) k_aboundary(PoolDev P, int ntiles, int p
 // PHASED also follows each system's lifecycle.  A system whose rows
 // overflowed was skipped by the pass and is not advanced.
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, int split)
+__global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, int split, int seeded)
 {
     __shared__ int s_any;
     SysDev *d = P.sys + blockIdx.x;
@@ -1114,7 +1120,7 @@ __global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, in
                 d->phase = PH_DONE;
                 d->active = 0;
             } else {
-                commit_advance(d, false);
+                commit_advance(d, false, seeded);
                 const int ago = ++d->ago;
                 const bool due = ago >= d->n_delay && ago % d->n_every == 0;
                 d->stale = due && (!d->n_check || s_any != 0) ? 1 : 0;
@@ -1123,12 +1129,12 @@ __global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, in
             }
             P.status[blockIdx.x] = (d->job << 3) | (d->stale ? 1 : 0) | (d->phase == PH_DONE ? 2 : 0);
         } else if (advance == COMMIT_DECIDE) {
-            commit_advance(d, false);
+            commit_advance(d, false, seeded);
             const int ago = ++d->ago;
             const bool due = ago >= d->n_delay && ago % d->n_every == 0;
             d->stale = due && (!d->n_check || s_any != 0) ? 1 : 0;
         } else if (advance == COMMIT_ADVANCE) {
-            commit_advance(d, s_any != 0);
+            commit_advance(d, s_any != 0, seeded);
         } else {
             d->sel ^= 1;
         }
@@ -1203,10 +1209,13 @@ __global__ void k_premix(const uint32_t *a, const uint32_t *b, uint32_t *out, in
 // 15.3 us against 13.2 and 16.3; 1,513 tiles: step 0.89x).
 constexpr int WIDE_TILES = 512;
 
+bool first_seeds(int split, int nt) { return split == 1 || nt <= WIDE_TILES; }
+
 template <bool WITH_RHO>
 static hipError_t launch_first_t(const PoolDev &P, int split, int nt, hipStream_t st)
 {
-    const dim3 g(xcd_grid(nt));
+    // the tiles, then the seed workgroups
+    const dim3 g(xcd_grid(nt) + (first_seeds(split, nt) ? (P.nsys + WAVE - 1) / WAVE : 0));
     const bool wide = nt <= WIDE_TILES;
     if (split == 1)
         hipLaunchKernelGGL((k_first<WITH_RHO, 1>), g, dim3(WAVE), 0, st, P, nt);
@@ -1231,10 +1240,11 @@ hipError_t launch_first(const PoolDev &P, bool with_rho, int split, hipStream_t 
     return with_rho ? launch_first_t<true>(P, split, nt, st) : launch_first_t<false>(P, split, nt, st);
 }
 
-hipError_t launch_commit_step(const PoolDev &P, int kind, int split, hipStream_t st)
+hipError_t launch_commit_step(const PoolDev &P, int kind, int split, bool after_pass, hipStream_t st)
 {
     if (P.nsys == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_commit_step, dim3(P.nsys), dim3(1024), 0, st, P, kind, split);
+    const int seeded = after_pass && (P.one || first_seeds(split, P.nact / WAVE)) ? 1 : 0;
+    hipLaunchKernelGGL(k_commit_step, dim3(P.nsys), dim3(1024), 0, st, P, kind, split, seeded);
     return hipGetLastError();
 }
 

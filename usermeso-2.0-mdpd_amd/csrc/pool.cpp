@@ -481,7 +481,7 @@ struct mdpd_pool {
         dsys.alloc(max_sys);
         hip_check(hipMemsetAsync(cell_count.p, 0, sizeof(int) * (size_t)nslots * SUBCELLS, stream), "memset");
         hip_check(hipMemsetAsync(cell_sys.p, 0xFF, sizeof(int) * nslots, stream), "memset");
-        hip_check(hipMemsetAsync(work_count.p, 0, sizeof(int), stream), "memset");
+        hip_check(hipMemsetAsync(work_count.p, 0, 2 * sizeof(int), stream), "memset");
         hip_check(hipMemsetAsync(wave_sys.p, 0xFF, sizeof(int) * (cap / WAVE), stream), "memset");
         hip_check(hipMemsetAsync(status.p, 0, sizeof(int) * max_sys, stream), "memset");
         hip_check(hipMemsetAsync(dsys.p, 0, sizeof(SysDev) * max_sys, stream), "memset");
@@ -788,8 +788,7 @@ struct mdpd_pool {
             if (ev) hip_check(hipEventRecord(ev->e[k], stream), "hipEventRecord");
         };
         mark(PP_REBUILD);
-        hip_check(launch_rebuild(P, stream), "rebuild");
-        hip_check(launch_commit_rebuild(P, stream), "commit rebuild");
+        hip_check(launch_rebuild(P, sp, stream), "rebuild");
         mark(PP_FIRST);
         hip_check(launch_first(P, with_rho, sp, stream), "first pass");
         mark(PP_FORCE);
@@ -797,7 +796,7 @@ struct mdpd_pool {
         if (with_arb) hip_check(launch_aboundary(P, 1, stream), "aboundary");
         if (with_obs) hip_check(launch_obs_pool(P, stream), "observables");
         mark(PP_COMMIT);
-        hip_check(launch_commit_step(P, COMMIT_PHASED, sp, stream), "commit step");
+        hip_check(launch_commit_step(P, COMMIT_PHASED, sp, true, stream), "commit step");
         mark(PP_COUNT);
     }
 

@@ -1451,7 +1451,7 @@ struct mdpd_system {
         P.clist = clist.p; P.ccount = ccount.p; P.moved = moved.p; P.status = status.p;
         P.cl = cl.p; P.wall_near = wall_near.p;
         P.sys = dsys.p; P.coef = coef.p; P.minv = minv.p; P.mass = mmass.p;
-        P.cap = cap; P.nact = cap; P.ncellslots = nslots; P.ncact = nslots; P.nsys = 1; P.maxsub = 0;
+        P.cap = cap; P.nact = cap; P.ncellslots = nslots; P.ncact = nslots; P.nsys = 1; P.maxsub = 0; P.one = 1;
         P.maxnbr = maxnbr;
         return P;
     }
@@ -1670,7 +1670,7 @@ struct mdpd_system {
         up(minv.p, ds.minv.data(), ntypes * sizeof(float));
         up(mmass.p, ds.mass.data(), ntypes * sizeof(float));
         hip_check(hipMemsetAsync(cell_count.p, 0, (size_t)nslots * SUBCELLS * sizeof(int), stream), "memset");
-        hip_check(hipMemsetAsync(work_count.p, 0, sizeof(int), stream), "memset");
+        hip_check(hipMemsetAsync(work_count.p, 0, 2 * sizeof(int), stream), "memset");
         hip_check(hipMemsetAsync(ncount.p, 0, cap * sizeof(int), stream), "memset");
         hip_check(hipMemsetAsync(rho.p, 0, cap * sizeof(float), stream), "memset");
         std::vector<float> hph(cap, 0.f);   // per-atom state of fix aboundary/rho/meso
@@ -1700,7 +1700,7 @@ struct mdpd_system {
     void rebuild()
     {
         PoolDev P = view();
-        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, stream), "rebuild"); });
+        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, stream), "rebuild"); });
         for (int attempt = 0;; ++attempt) {
             int ovf = read_field(offsetof(SysDev, overflow));
             if (!ovf) break;
@@ -1717,7 +1717,6 @@ struct mdpd_system {
             P = view();
             hip_check(launch_nlist_only(P, stream), "nlist");
         }
-        hip_check(launch_commit_rebuild(P, stream), "commit");
         graph_valid = false;
     }
 
@@ -1796,7 +1795,7 @@ struct mdpd_system {
         if ((mode == MODE_FUSED || mode == MODE_FUSED_OUT) && hsys.fix_arb)
             timed(PH_WALL, [&]() { hip_check(launch_aboundary(P, 0, stream), "aboundary"); });   // post_integrate
         if (mode != MODE_SETUP)
-            hip_check(launch_commit_step(P, mode == MODE_FINAL ? COMMIT_FINAL : COMMIT_DECIDE, split, stream), "commit");
+            hip_check(launch_commit_step(P, mode == MODE_FINAL ? COMMIT_FINAL : COMMIT_DECIDE, split, true, stream), "commit");
     }
 
     // The rebuild phase of a step, launched every step: its kernels re-sort
@@ -1805,8 +1804,7 @@ struct mdpd_system {
     void rebuild_phase()
     {
         PoolDev P = view();
-        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, stream), "rebuild"); });
-        hip_check(launch_commit_rebuild(P, stream), "commit rebuild");
+        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, stream), "rebuild"); });
     }
 
     // the graph of one fused step whose observables take the samples of
@@ -1899,7 +1897,7 @@ struct mdpd_system {
         PoolDev P = view();
         timed(PH_INITIAL, [&]() { hip_check(launch_initial(P, stream), "initial"); });
         if (hsys.fix_arb) timed(PH_WALL, [&]() { hip_check(launch_aboundary(P, 0, stream), "aboundary"); });
-        hip_check(launch_commit_step(P, COMMIT_DECIDE, split, stream), "commit");
+        hip_check(launch_commit_step(P, COMMIT_DECIDE, split, false, stream), "commit");
         const long long t0 = ntimestep;
         long long k = 1;                  // the step whose force pass runs next
         while (k < nsteps) {
