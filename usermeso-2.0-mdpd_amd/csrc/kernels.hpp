@@ -47,14 +47,23 @@ hipError_t launch_force_range(const PoolDev &P, int style, int mode, bool uni, i
 // wall branch of aboundary/rho/meso (wall fraction, bounce-back, displacement
 // flags) on the buffer a pass just wrote; pooled: only systems that integrated
 hipError_t launch_aboundary(const PoolDev &P, int pooled, hipStream_t st);
-// pooled engine, finished system s (npad slots from part_base): its results
-// packed into dst (room bytes, at least harvest_bytes(npad)) in this layout:
+// pooled engine, finished system s (npad slots from part_base): its results in
+// creation order, packed into dst (room bytes, at least harvest_bytes(npad)):
 //   float4 x[npad] | float4 v[npad] | float4 f[npad] (w: pair energy) |
-//   int tag[npad], mask[npad], origin[npad], image[npad] | float rho[npad] |
+//   int tag[npad], mask[npad], image[npad] | float rho[npad] |
 //   float virial[6][npad] | SysDev
-constexpr size_t HARVEST_SLOT_BYTES = 3 * 16 + 4 * 4 + 4 + 6 * 4;
+constexpr size_t HARVEST_SLOT_BYTES = 3 * 16 + 3 * 4 + 4 + 6 * 4;
 inline size_t harvest_bytes(size_t npad) { return npad * HARVEST_SLOT_BYTES + sizeof(SysDev); }
 hipError_t launch_harvest(const PoolDev &P, int s, int part_base, int npad, void *dst, size_t room, hipStream_t st);
+
+// one system: a per-atom quantity in creation order, gather_words(field) 4-byte
+// words per particle (floats, or ints from G_TAG on; image unpacked, type 1-based)
+enum GatherField : int { G_X = 0, G_V, G_F, G_EPAIR, G_RHO, G_PHI, G_VIRIAL, G_TAG, G_TYPE, G_MASK, G_IMAGE };
+constexpr int gather_words(int field)
+{
+    return field == G_X || field == G_V || field == G_F || field == G_IMAGE ? 3 : field == G_VIRIAL ? 6 : 1;
+}
+hipError_t launch_gather(const PoolDev &P, int field, int *out, hipStream_t st);
 
 // observables (accumulate into device histograms of nbin + 1 slots, slot nbin
 // counting the samples; a system whose rows overflowed is not sampled)

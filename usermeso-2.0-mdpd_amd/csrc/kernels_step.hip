@@ -1143,9 +1143,9 @@ __global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, in
 
 // --------------------------------------------------------------------------
 // Finished pooled system: its current state, the last force evaluation and
-// its descriptor packed into one block at dst (x, v, f | tag, mask, origin,
-// image | rho, virial | SysDev, each array npad long), so the host copies one
-// range.  Runs after the HARVEST force pass, which reads the other buffer.
+// its descriptor packed into one block at dst (x, v, f | tag, mask, image |
+// rho, virial | SysDev, each array npad long, in creation order), so the host
+// copies one range.  Runs after the HARVEST force pass, which reads the other buffer.
 // The system's tiles and cell slots are unmapped here (no kernel after it
 // finds the system through them); the host frees the ranges once the copy
 // has landed.
@@ -1161,22 +1161,60 @@ __global__ void __launch_bounds__(256) k_harvest(PoolDev P, int s, int pb, int n
     }
     for (int c = k, nc = d->ncell + 1; c < nc; c += gridDim.x * blockDim.x) P.cell_sys[d->cell_base + c] = -1;
     if (k < npad / WAVE) P.wave_sys[pb / WAVE + k] = -1;
-    if (k >= npad) return;
+    if (k >= d->n) return;
     const int i = pb + k, cur = d->sel, cura = d->sela;
+    const int c = P.origin[cura][i];                          // creation index
+    if (c < 0 || c >= d->n) return;
     const size_t n = npad;
     float4 *o4 = (float4 *)dst;
-    o4[k] = P.pos[cur][i];
-    o4[n + k] = P.vel[cur][i];
-    o4[2 * n + k] = P.frc[i];
+    o4[c] = P.pos[cur][i];
+    o4[n + c] = P.vel[cur][i];
+    o4[2 * n + c] = P.frc[i];
     int *oi = (int *)(o4 + 3 * n);
-    oi[k] = P.tag[cura][i];
-    oi[n + k] = P.mask[cura][i];
-    oi[2 * n + k] = P.origin[cura][i];
-    oi[3 * n + k] = P.image[cura][i];
-    float *of = (float *)(oi + 4 * n);
-    of[k] = P.rho[i];
+    oi[c] = P.tag[cura][i];
+    oi[n + c] = P.mask[cura][i];
+    oi[2 * n + c] = P.image[cura][i];
+    float *of = (float *)(oi + 3 * n);
+    of[c] = P.rho[i];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) of[(c + 1) * n + k] = P.vir[(size_t)c * P.cap + i];
+    for (int m = 0; m < 6; ++m) of[(m + 1) * n + c] = P.vir[(size_t)m * P.cap + i];
+}
+
+// --------------------------------------------------------------------------
+// One system's per-atom quantity in creation order (the host copies one block
+// and only widens it).
+// --------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_gather(PoolDev P, int field, int *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const SysDev *d = P.sys;
+    if (i >= d->n) return;
+    const int sel = d->sel, sela = d->sela;
+    const int c = P.origin[sela][i];
+    if (c < 0 || c >= d->n) return;
+    float *of = (float *)out;
+    auto put3 = [&](const float4 &q) { of[3 * c] = q.x; of[3 * c + 1] = q.y; of[3 * c + 2] = q.z; };
+    switch (field) {
+    case G_X: put3(P.pos[sel][i]); break;
+    case G_V: put3(P.vel[sel][i]); break;
+    case G_F: put3(P.frc[i]); break;
+    case G_EPAIR: of[c] = P.frc[i].w; break;
+    case G_RHO: of[c] = P.rho[i]; break;
+    case G_PHI: of[c] = P.phi[sela][i]; break;
+    case G_VIRIAL:
+        for (int m = 0; m < 6; ++m) of[6 * c + m] = P.vir[(size_t)m * P.cap + i];
+        break;
+    case G_TAG: out[c] = P.tag[sela][i]; break;
+    case G_TYPE: out[c] = __float_as_int(P.pos[sel][i].w) + 1; break;
+    case G_MASK: out[c] = P.mask[sela][i]; break;
+    case G_IMAGE: {
+        const int im = P.image[sela][i];
+        out[3 * c] = (im & 1023) - 512;
+        out[3 * c + 1] = ((im >> 10) & 1023) - 512;
+        out[3 * c + 2] = ((im >> 20) & 1023) - 512;
+        break;
+    }
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -1262,6 +1300,14 @@ hipError_t launch_harvest(const PoolDev &P, int s, int part_base, int npad, void
     if (s < 0 || s >= P.nsys || part_base < 0 || part_base + npad > P.cap || !dst || harvest_bytes(npad) > room)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_harvest, dim3((npad + 255) / 256), dim3(256), 0, st, P, s, part_base, npad, (char *)dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_gather(const PoolDev &P, int field, int *out, hipStream_t st)
+{
+    if (!P.one || field < G_X || field > G_IMAGE || !out) return hipErrorInvalidValue;
+    if (P.nact == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_gather, dim3((P.nact + 255) / 256), dim3(256), 0, st, P, field, out);
     return hipGetLastError();
 }
 

@@ -156,11 +156,10 @@ struct Job {
     double t_submit = 0, t_admit = 0, t_done = 0;
 };
 
-// typed views of a finished job's stage (slot k holds the particle with
-// creation index origin[k], k < n)
+// typed views of a finished job's stage (creation order, k < n)
 struct HarvestView {
     const float4 *x, *v, *f;
-    const int *tag, *mask, *origin, *image;
+    const int *tag, *mask, *image;
     const float *rho, *vir;   // vir: six planes of npad
     const char *desc;
     explicit HarvestView(const Job &j)
@@ -171,14 +170,13 @@ struct HarvestView {
         f = x + 2 * np;
         tag = (const int *)(x + 3 * np);
         mask = tag + np;
-        origin = tag + 2 * np;
-        image = tag + 3 * np;
-        rho = (const float *)(tag + 4 * np);
+        image = tag + 2 * np;
+        rho = (const float *)(tag + 3 * np);
         vir = rho + np;
         desc = (const char *)j.results() + np * HARVEST_SLOT_BYTES;
     }
 };
-static_assert(HARVEST_SLOT_BYTES == 92, "stage layout");
+static_assert(HARVEST_SLOT_BYTES == 88, "stage layout");
 // the packed results fit the finished system's neighbor-row range, whose
 // width is at least NBR_ALIGN entries for at least 256 slots
 static_assert(sizeof(SysDev) <= 256 * (4 * NBR_ALIGN - HARVEST_SLOT_BYTES), "harvest block fits the rows");
@@ -1042,9 +1040,6 @@ struct mdpd_pool {
             if (q == hipErrorNotReady) continue;
             hip_check(q, "harvest event");
             const HarvestView h(j);
-            for (int k = 0; k < j.n; ++k)
-                if (h.origin[k] < 0 || h.origin[k] >= j.n)
-                    fail(MDPD_E_HIP, "harvest of job %d: bad particle origin %d", j.id, h.origin[k]);
             SysDev d;
             memcpy(&d, h.desc, sizeof(SysDev));
             j.step_end = d.step;
@@ -1265,31 +1260,29 @@ int mdpd_pool_gather(mdpd_pool *pool, int job, const char *name, int type, int c
         const std::string nm(name);
         const HarvestView h(j);
         const int n = j.n;
-        // checks the caller's type and width, then clears the output
         auto want = [&](int t, int c) {
             if (type != t || count != c) fail(MDPD_E_ARG, "gather of %s needs type %d count %d", name, t, c);
-            memset(data, 0, (size_t)n * c * (t == 1 ? sizeof(double) : sizeof(int)));
         };
         if (nm == "x" || nm == "v" || nm == "f") {
             want(1, 3);
             const float4 *src = nm == "x" ? h.x : (nm == "v" ? h.v : h.f);
             double *o = (double *)data;
             for (int k = 0; k < n; ++k) {
-                double *r = o + 3 * (size_t)h.origin[k];
+                double *r = o + 3 * (size_t)k;
                 r[0] = src[k].x; r[1] = src[k].y; r[2] = src[k].z;
             }
         } else if (nm == "e_pair" || nm == "rho") {
             want(1, 1);
             double *o = (double *)data;
             if (nm == "rho")
-                for (int k = 0; k < n; ++k) o[h.origin[k]] = h.rho[k];
+                for (int k = 0; k < n; ++k) o[k] = h.rho[k];
             else
-                for (int k = 0; k < n; ++k) o[h.origin[k]] = h.f[k].w;
+                for (int k = 0; k < n; ++k) o[k] = h.f[k].w;
         } else if (nm == "virial") {
             want(1, 6);
             double *o = (double *)data;
             for (int k = 0; k < n; ++k)
-                for (int c = 0; c < 6; ++c) o[6 * (size_t)h.origin[k] + c] = h.vir[(size_t)c * j.npad + k];
+                for (int c = 0; c < 6; ++c) o[6 * (size_t)k + c] = h.vir[(size_t)c * j.npad + k];
         } else if (nm == "tag" || nm == "type" || nm == "mask") {
             want(0, 1);
             int *o = (int *)data;
@@ -1298,14 +1291,14 @@ int mdpd_pool_gather(mdpd_pool *pool, int job, const char *name, int type, int c
                 if (nm == "tag") val = h.tag[k];
                 else if (nm == "mask") val = h.mask[k];
                 else { memcpy(&val, &h.x[k].w, 4); val += 1; }
-                o[h.origin[k]] = val;
+                o[k] = val;
             }
         } else if (nm == "image") {
             want(0, 3);
             int *o = (int *)data;
             for (int k = 0; k < n; ++k) {
                 const int im = h.image[k];
-                int *r = o + 3 * (size_t)h.origin[k];
+                int *r = o + 3 * (size_t)k;
                 r[0] = (im & 1023) - 512; r[1] = ((im >> 10) & 1023) - 512; r[2] = ((im >> 20) & 1023) - 512;
             }
         } else {
@@ -1326,7 +1319,7 @@ int mdpd_pool_thermo(mdpd_pool *pool, int job, double out[4])
         std::vector<int> ty(n);
         std::vector<double> v(3 * (size_t)n), vir(6 * (size_t)n), e(n);
         for (int k = 0; k < n; ++k) {
-            const size_t i = h.origin[k];
+            const size_t i = k;
             int t;
             memcpy(&t, &h.x[k].w, 4);
             ty[i] = t + 1;

@@ -228,6 +228,9 @@ struct mdpd_system {
     DevBuf<unsigned long long> key;
     DevBuf<SysDev> dsys;
     int *pinned = nullptr;            // host-visible readback of flags
+    static constexpr size_t STAGE_WORDS = 1 << 17;
+    int *stage = nullptr;             // two pinned halves of STAGE_WORDS words (gather)
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
 
     // ---- kernel timing with HIP events (phase -> total ms, launches) ----
     bool prof = false;
@@ -256,6 +259,9 @@ struct mdpd_system {
         for (auto &e : ev_open) { (void)hipEventDestroy(e.second.first); (void)hipEventDestroy(e.second.second); }
         for (auto e : ev_free) (void)hipEventDestroy(e);
         if (pinned) (void)hipHostFree(pinned);
+        if (stage) (void)hipHostFree(stage);
+        for (auto e : stage_ev)
+            if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -1970,62 +1976,49 @@ struct mdpd_system {
             }
             fail(MDPD_E_STATE, "%s is only available after setup", name.c_str());
         }
-        sync_sys();
-        const int sel = hsys.sel, sela = hsys.sela;
-        std::vector<int> org = download(origin[sela].p, cap);
-        hip_check(hipStreamSynchronize(stream), "sync");
-        auto put_d = [&](int k, int c, double v) { ((double *)data)[(size_t)org[k] * count + c] = v; };
-        auto put_i = [&](int k, int c, int v) { ((int *)data)[(size_t)org[k] * count + c] = v; };
-        auto want = [&](int t, int c) {
-            if (type != t || count != c) fail(MDPD_E_ARG, "gather of %s needs type %d count %d", name.c_str(), t, c);
-        };
-        if (name == "x" || name == "v" || name == "f") {
-            want(1, 3);
-            std::vector<float4> h = download(name == "x" ? pos[sel].p : (name == "v" ? vel[sel].p : frc.p), cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) { put_d(k, 0, h[k].x); put_d(k, 1, h[k].y); put_d(k, 2, h[k].z); }
-        } else if (name == "e_pair") {
-            want(1, 1);
-            std::vector<float4> h = download(frc.p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) put_d(k, 0, h[k].w);
-        } else if (name == "rho") {
-            want(1, 1);
-            std::vector<float> h = download(rho.p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) put_d(k, 0, h[k]);
-        } else if (name == "phi") {
-            want(1, 1);
-            std::vector<float> h = download(phi[sela].p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) put_d(k, 0, h[k]);
-        } else if (name == "virial") {
-            want(1, 6);
-            std::vector<float> h = download(vir.p, (size_t)6 * cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k)
-                for (int c = 0; c < 6; ++c) put_d(k, c, h[(size_t)c * cap + k]);
-        } else if (name == "tag" || name == "mask") {
-            want(0, 1);
-            std::vector<int> h = download(name == "tag" ? tag[sela].p : mask[sela].p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) put_i(k, 0, h[k]);
-        } else if (name == "type") {
-            want(0, 1);
-            std::vector<float4> h = download(pos[sel].p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) { int t; memcpy(&t, &h[k].w, 4); put_i(k, 0, t + 1); }
-        } else if (name == "image") {
-            want(0, 3);
-            std::vector<int> h = download(image[sela].p, cap);
-            hip_check(hipStreamSynchronize(stream), "sync");
-            for (int k = 0; k < n; ++k) {
-                put_i(k, 0, (h[k] & 1023) - 512);
-                put_i(k, 1, ((h[k] >> 10) & 1023) - 512);
-                put_i(k, 2, ((h[k] >> 20) & 1023) - 512);
+        static const struct { const char *name; int field, type; } known[] = {
+            {"x", G_X, 1}, {"v", G_V, 1}, {"f", G_F, 1}, {"e_pair", G_EPAIR, 1}, {"rho", G_RHO, 1}, {"phi", G_PHI, 1},
+            {"virial", G_VIRIAL, 1}, {"tag", G_TAG, 0}, {"mask", G_MASK, 0}, {"type", G_TYPE, 0}, {"image", G_IMAGE, 0}};
+        for (auto &q : known) {
+            if (name != q.name) continue;
+            const int c = gather_words(q.field);
+            if (type != q.type || count != c)
+                fail(MDPD_E_ARG, "gather of %s needs type %d count %d", name.c_str(), q.type, c);
+            gather_field(q.field, (size_t)n * c, q.type == 1 ? (double *)data : nullptr, (int *)data);
+            return;
+        }
+        fail(MDPD_E_ARG, "unknown per-atom quantity '%s'", name.c_str());
+    }
+
+    // `words` 4-byte words of a quantity, put in creation order on the device
+    // (in the compact rows, which no pass reads after its own force pass),
+    // copied through two halves of a pinned stage and widened to `d` (floats)
+    // or copied to `k` (ints) half by half while the next one is on its way
+    void gather_field(int field, size_t words, double *d, int *k)
+    {
+        static_assert(NBR_ALIGN >= 6, "six words per particle fit the narrowest compact rows");
+        if (!stage) {
+            hip_check(hipHostMalloc((void **)&stage, 2 * STAGE_WORDS * sizeof(int), hipHostMallocDefault),
+                      "hipHostMalloc");
+            for (auto &e : stage_ev) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        }
+        hip_check(launch_gather(view(), field, clist.p, stream), "gather");
+        const size_t nc = (words + STAGE_WORDS - 1) / STAGE_WORDS;
+        auto len = [&](size_t c) { return std::min(STAGE_WORDS, words - c * STAGE_WORDS); };
+        for (size_t c = 0; c <= nc; ++c) {
+            if (c < nc) {
+                hip_check(hipMemcpyAsync(stage + (c & 1) * STAGE_WORDS, clist.p + c * STAGE_WORDS, len(c) * sizeof(int),
+                                         hipMemcpyDeviceToHost, stream), "gather");
+                hip_check(hipEventRecord(stage_ev[c & 1], stream), "gather");
             }
-        } else {
-            fail(MDPD_E_ARG, "unknown per-atom quantity '%s'", name.c_str());
+            if (c == 0) continue;
+            hip_check(hipEventSynchronize(stage_ev[(c - 1) & 1]), "gather");
+            const int *src = stage + ((c - 1) & 1) * STAGE_WORDS;
+            const size_t at = (c - 1) * STAGE_WORDS, m = len(c - 1);
+            if (d)
+                for (size_t i = 0; i < m; ++i) d[at + i] = ((const float *)src)[i];
+            else
+                memcpy(k + at, src, m * sizeof(int));
         }
     }
 
