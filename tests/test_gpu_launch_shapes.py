@@ -96,3 +96,31 @@ def test_sorted_order_over_scan_sizes(engine, orc, n, L):
     assert np.array_equal(got, orc.sort_keys(xw, (0, 0, 0), (L, L, L), 1.3))
     assert np.all(np.diff(got.astype(np.int64)) >= 0)
     s.close()
+
+
+def test_jobs_harvested_together_equal_their_own_runs(engine):
+    # two mDPD jobs and a DPD job end in the same pass, with a longer two-type
+    # job between them (evaluated by the same launches only once it has ended)
+    # and a box of far more cells than particles; the second batch is packed
+    # into pinned memory at submission
+    def systems():
+        x, v = uniform_box(700, 5.0, 8)
+        sparse = uniform_box(10, 20.0, 9)
+        return [(mdpd_system(engine, x, v, 5.0), 15), (_two_types(engine), 22), (_dpd(engine), 15),
+                (mdpd_system(engine, *sparse, 20.0), 15)]
+    ref = []
+    for s, k in systems():
+        s.tune("split", 1)
+        s.run(k)
+        ref.append({q: s.gather(q) for q in ("x", "v", "f", "image", "e_pair", "virial", "tag", "type", "mask")})
+        s.close()
+    p = engine.Pool(float(1 << 29), 16)
+    p.tune("split", 1)
+    for batch in range(2):
+        ids = [p.submit(s, k) for s, k in systems()]
+        p.run()
+        for j, want in zip(ids, ref):
+            for q, w in want.items():
+                np.testing.assert_array_equal(p.gather(j, q), w, err_msg=f"batch {batch}, job {j}: {q}")
+            p.release(j)
+    p.close()

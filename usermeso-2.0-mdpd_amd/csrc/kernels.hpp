@@ -47,14 +47,44 @@ hipError_t launch_force_range(const PoolDev &P, int style, int mode, bool uni, i
 // wall branch of aboundary/rho/meso (wall fraction, bounce-back, displacement
 // flags) on the buffer a pass just wrote; pooled: only systems that integrated
 hipError_t launch_aboundary(const PoolDev &P, int pooled, hipStream_t st);
-// pooled engine, finished system s (npad slots from part_base): its results in
-// creation order, packed into dst (room bytes, at least harvest_bytes(npad)):
+// pooled engine: a submitted system's input block (InLayout, readable from the
+// device) unpacked into slots [part_base, + npad) and cell slots [cell_base,
+// + nc1) of buffer 0, descriptor slot s
+struct InLayout {
+    size_t pos, vel, tag, mask, image, phi, rank, xyz, coef, mass, sys, bytes;
+    int n, npad, nc1, ncoef, nt, has_phi;
+    InLayout(int n_, int npad_, int nc1_, int ncoef_, int nt_, bool phi_)
+        : n(n_), npad(npad_), nc1(nc1_), ncoef(ncoef_), nt(nt_), has_phi(phi_ ? 1 : 0)
+    {
+        size_t at = 0;
+        auto take = [&](size_t b) { const size_t o = at; at += (b + 15) / 16 * 16; return o; };
+        pos = take(sizeof(float4) * n);
+        vel = take(sizeof(float) * 3 * n);
+        tag = take(sizeof(int) * n);
+        mask = take(sizeof(int) * n);
+        image = take(sizeof(int) * n);
+        phi = take(has_phi ? sizeof(float) * n : 0);
+        rank = take(sizeof(int) * nc1);
+        xyz = take(sizeof(int) * nc1);
+        coef = take(sizeof(float) * ncoef);
+        mass = take(sizeof(float) * 2 * nt);            // m, 1 / m
+        sys = take(sizeof(SysDev));
+        bytes = at;
+    }
+};
+hipError_t launch_admit(const PoolDev &P, const InLayout &in, const void *block, int s, int part_base, int cell_base,
+                        hipStream_t st);
+
+// pooled engine, finished systems in descriptor slots[0 .. count): each one's
+// results in creation order, packed at the start of its own neighbor-row range
+// (harvest_dst), harvest_bytes(npad) bytes:
 //   float4 x[npad] | float4 v[npad] | float4 f[npad] (w: pair energy) |
 //   int tag[npad], mask[npad], image[npad] | float rho[npad] |
 //   float virial[6][npad] | SysDev
 constexpr size_t HARVEST_SLOT_BYTES = 3 * 16 + 3 * 4 + 4 + 6 * 4;
 inline size_t harvest_bytes(size_t npad) { return npad * HARVEST_SLOT_BYTES + sizeof(SysDev); }
-hipError_t launch_harvest(const PoolDev &P, int s, int part_base, int npad, void *dst, size_t room, hipStream_t st);
+inline size_t harvest_dst(const PoolDev &P, int part_base) { return (size_t)part_base * P.maxnbr; }
+hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, hipStream_t st);
 
 // one system: a per-atom quantity in creation order, gather_words(field) 4-byte
 // words per particle (floats, or ints from G_TAG on; image unpacked, type 1-based)

@@ -591,8 +591,9 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
     // passes (no state change until the host has regrown the rows), and a
     // pool may mix styles: each launch takes the systems of its style
     if (STEP && d->overflow) return;
-    if (MODE == MODE_PHASED && d->style != STYLE) return;
-    if (MODE == MODE_HARVEST && d->split_last != SPLIT) return;   // the split of its last pass
+    if ((MODE == MODE_PHASED || MODE == MODE_HARVEST) && d->style != STYLE) return;
+    // a finished system, at the split of its last pass
+    if (MODE == MODE_HARVEST && (d->phase != PH_DONE || d->split_last != SPLIT)) return;
     const bool valid = i < d->part_base + d->n;
     const int cur = MODE == MODE_HARVEST ? d->sel ^ 1 : d->sel;
     const float4 *pos = P.pos[cur];
@@ -807,8 +808,8 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
     if (!d->active && MODE != MODE_HARVEST) return;
     if (UNI != (d->ntypes == 1)) return;     // host launches the matching variant
     if (STEP && d->overflow) return;
-    if (MODE == MODE_PHASED && d->style != STYLE) return;
-    if (MODE == MODE_HARVEST && d->split_last != SPLIT) return;
+    if ((MODE == MODE_PHASED || MODE == MODE_HARVEST) && d->style != STYLE) return;
+    if (MODE == MODE_HARVEST && (d->phase != PH_DONE || d->split_last != SPLIT)) return;
     const bool valid = i < d->part_base + d->n;
     const int cur = MODE == MODE_HARVEST ? d->sel ^ 1 : d->sel;
     const float4 *pos = P.pos[cur];
@@ -1142,18 +1143,75 @@ __global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, in
 }
 
 // --------------------------------------------------------------------------
-// Finished pooled system: its current state, the last force evaluation and
-// its descriptor packed into one block at dst (x, v, f | tag, mask, image |
-// rho, virial | SysDev, each array npad long, in creation order), so the host
-// copies one range.  Runs after the HARVEST force pass, which reads the other buffer.
-// The system's tiles and cell slots are unmapped here (no kernel after it
-// finds the system through them); the host frees the ranges once the copy
-// has landed.
+// Admission: one launch unpacks a submitted system's input block, read in
+// place from the pinned host memory it was packed in, and derives the rest
+// (creation indices, owners of tiles and cell slots, cleared counts).  As
+// sixteen copies and fills per job, admitting 256 droplets (2.3 million particles)
+// took 30 ms, most of
+// it the host copying and ~5 us per command; 5.5 ms so.
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_harvest(PoolDev P, int s, int pb, int npad, char *dst)
+__global__ void __launch_bounds__(256) k_admit(PoolDev P, InLayout in, const char *src, int s, int pb, int cb)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const SysDev *d = P.sys + s;
+    if (blockIdx.x == 0) {
+        const SysDev *d = (const SysDev *)(src + in.sys);
+        const int *w = (const int *)d;
+        int *o = (int *)(P.sys + s);
+        for (int q = threadIdx.x; q < (int)(sizeof(SysDev) / 4); q += blockDim.x) o[q] = w[q];
+        const float *cf = (const float *)(src + in.coef), *ms = (const float *)(src + in.mass);
+        const int c0 = s * MAXTYPES * MAXTYPES * NCOEF, m0 = s * MAXTYPES;
+        for (int q = threadIdx.x; q < in.ncoef; q += blockDim.x) P.coef[c0 + q] = cf[q];
+        for (int q = threadIdx.x; q < in.nt; q += blockDim.x) {
+            P.mass[m0 + q] = ms[q];
+            P.minv[m0 + q] = ms[in.nt + q];
+        }
+    }
+    if (k < in.nc1) {
+        P.cell_rank[cb + k] = ((const int *)(src + in.rank))[k];
+        P.cell_xyz[cb + k] = ((const int *)(src + in.xyz))[k];
+        P.cell_sys[cb + k] = s;
+        for (int q = 0; q < SUBCELLS; ++q) P.cell_count[(cb + k) * SUBCELLS + q] = 0;
+    }
+    if (k < in.npad / WAVE) P.wave_sys[pb / WAVE + k] = s;
+    if (k >= in.npad) return;
+    const int i = pb + k;
+    const bool live = k < in.n;                            // padding slots are inert
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f), v = x;
+    if (live) {
+        x = ((const float4 *)(src + in.pos))[k];
+        const float *u = (const float *)(src + in.vel) + 3 * (size_t)k;
+        v = make_float4(u[0], u[1], u[2], 0.f);
+    }
+    P.pos[0][i] = x;
+    P.vel[0][i] = v;
+    P.tag[0][i] = live ? ((const int *)(src + in.tag))[k] : 0;
+    P.mask[0][i] = live ? ((const int *)(src + in.mask))[k] : 0;
+    P.origin[0][i] = live ? k : -1;
+    P.image[0][i] = live ? ((const int *)(src + in.image))[k] : 512 | (512 << 10) | (512 << 20);
+    P.phi[0][i] = live && in.has_phi ? ((const float *)(src + in.phi))[k] : 0.f;
+}
+
+// --------------------------------------------------------------------------
+// Finished pooled systems (blockIdx.y: one of the list): current state, last
+// force evaluation and descriptor packed into one block in the system's own
+// neighbor-row range, which no pass reads once it has stopped (x, v, f | tag,
+// mask, image | rho, virial | SysDev, each array npad long, in creation
+// order), so the host copies one range.  Runs after the HARVEST force pass,
+// which reads the other buffer.  The system's tiles and cell slots are
+// unmapped here (no kernel after it finds the system through them); the host
+// frees the ranges once the copy has landed.
+// --------------------------------------------------------------------------
+constexpr int HARVEST_LIST = 64;
+struct HarvestList {
+    int slot[HARVEST_LIST];
+};
+
+__global__ void __launch_bounds__(256) k_harvest(PoolDev P, HarvestList list)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const SysDev *d = P.sys + list.slot[blockIdx.y];
+    const int pb = d->part_base, npad = d->npad;
+    char *dst = (char *)(P.nlist + (size_t)pb * P.maxnbr);
     if (blockIdx.x == 0) {
         const int *src = (const int *)d;
         int *o = (int *)(dst + (size_t)npad * HARVEST_SLOT_BYTES);
@@ -1294,12 +1352,33 @@ hipError_t launch_aboundary(const PoolDev &P, int pooled, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_harvest(const PoolDev &P, int s, int part_base, int npad, void *dst, size_t room, hipStream_t st)
+hipError_t launch_admit(const PoolDev &P, const InLayout &in, const void *block, int s, int part_base, int cell_base,
+                        hipStream_t st)
 {
-    if (npad <= 0) return hipSuccess;
-    if (s < 0 || s >= P.nsys || part_base < 0 || part_base + npad > P.cap || !dst || harvest_bytes(npad) > room)
+    if (!block || s < 0 || part_base < 0 || part_base % 256 || in.npad % 256 || in.n > in.npad ||
+        part_base + in.npad > P.cap || cell_base < 0 || cell_base + in.nc1 > P.ncellslots ||
+        in.ncoef > MAXTYPES * MAXTYPES * NCOEF || in.nt > MAXTYPES)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_harvest, dim3((npad + 255) / 256), dim3(256), 0, st, P, s, part_base, npad, (char *)dst);
+    const int threads = in.npad > in.nc1 ? in.npad : in.nc1;
+    hipLaunchKernelGGL(k_admit, dim3((threads + 255) / 256), dim3(256), 0, st, P, in, (const char *)block, s, part_base,
+                       cell_base);
+    return hipGetLastError();
+}
+
+hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, hipStream_t st)
+{
+    // the packed block fits the rows: maxnbr entries per slot, at least NBR_ALIGN
+    static_assert(sizeof(SysDev) <= 256 * (4 * NBR_ALIGN - HARVEST_SLOT_BYTES), "harvest block fits the rows");
+    if (P.maxnbr < NBR_ALIGN || npad_max <= 0 || npad_max > P.cap) return hipErrorInvalidValue;
+    for (int q0 = 0; q0 < count; q0 += HARVEST_LIST) {
+        HarvestList list{};
+        const int m = count - q0 < HARVEST_LIST ? count - q0 : HARVEST_LIST;
+        for (int q = 0; q < m; ++q) {
+            list.slot[q] = slots[q0 + q];
+            if (list.slot[q] < 0 || list.slot[q] >= P.nsys) return hipErrorInvalidValue;
+        }
+        hipLaunchKernelGGL(k_harvest, dim3((npad_max + 255) / 256, m), dim3(256), 0, st, P, list);
+    }
     return hipGetLastError();
 }
 

@@ -102,7 +102,7 @@ struct PinnedCache {
             free_.erase(it);
             return p;
         }
-        size_t sz = (size_t)1 << 20;
+        size_t sz = (size_t)1 << 16;
         while (sz < bytes) sz <<= 1;
         void *p = nullptr;
         hip_check(hipHostMalloc(&p, sz, hipHostMallocDefault), "hipHostMalloc");
@@ -122,9 +122,16 @@ struct Job {
     double volume = 0;
     double box[3] = {0, 0, 0};            // edge lengths
     double mass[MAXTYPES + 1] = {0};
-    std::vector<float4> hp, hv;           // packed input, npad slots
-    std::vector<int> ht, hm, ho, himg;
-    std::vector<float> hph;               // wall fraction carried in (fix aboundary/rho/meso)
+    // packed input (InLayout) until it has been unpacked on the device: in a
+    // pinned block of in_bytes, or in pageable memory (in_heap)
+    char *in = nullptr;
+    size_t in_bytes = 0;
+    std::unique_ptr<char[]> in_heap;
+    bool has_phi = false;                 // wall fractions carried in (fix aboundary/rho/meso)
+    InLayout in_layout() const
+    {
+        return InLayout(n, npad, ncell + 1, (int)ds.coef.size(), ntypes, has_phi);
+    }
     std::vector<FixDesc> rdf;             // its rdf/fast/meso fixes (their counts follow the
     double rdf_cut = 0;                   // harvested block), over pairs r < rdf_cut
     std::vector<FixDesc> dens;            // its density/meso fix (at most one): windows
@@ -177,10 +184,6 @@ struct HarvestView {
     }
 };
 static_assert(HARVEST_SLOT_BYTES == 88, "stage layout");
-// the packed results fit the finished system's neighbor-row range, whose
-// width is at least NBR_ALIGN entries for at least 256 slots
-static_assert(sizeof(SysDev) <= 256 * (4 * NBR_ALIGN - HARVEST_SLOT_BYTES), "harvest block fits the rows");
-
 // bytes of device memory per particle slot (state and scratch), per cell
 // slot (rank, coordinates, system; worklist entry, linear range; count and
 // start per sub-cell), and per neighbor-row entry (nlist + clist);
@@ -195,6 +198,7 @@ constexpr size_t ADMIT_LOOKAHEAD = 64;    // queued jobs considered per admissio
 // density windows
 constexpr size_t SLOT_OBS_WORDS = (size_t)POOL_RDF * (OBS_MAXBIN + 1) + POOL_DENS_WORDS;
 constexpr int MAX_BATCH = 16;             // passes captured in one batch graph
+constexpr size_t MAX_STAGED = (size_t)1 << 28;   // pinned bytes of inputs packed ahead of their admission
 constexpr int MAX_BYPASS = 64;            // admissions past one waiting head job
 
 }  // namespace
@@ -233,6 +237,7 @@ struct mdpd_pool {
 
     // ---- launch shape ----
     int split = 2;
+    int splits_used = 0;                  // splits that passes have run at (bit mask)
     bool autotune = true, tuned = false, retuned = false;
     long long retune_at = 0;              // passes after which the split may be tuned again
     double tuned_load = 0;                // resident particle slots when the split was last tuned
@@ -256,6 +261,7 @@ struct mdpd_pool {
     int poll_cur = 0;
     bool need_regrow = false;
     PinnedCache pinned;
+    size_t staged = 0;                    // pinned bytes of packed inputs waiting for admission
     size_t held_pinned = 0;               // stage bytes kept by finished jobs
     size_t max_held = (size_t)1 << 30;    // beyond this their results move to pageable memory
     std::vector<std::pair<hipEvent_t, std::pair<void *, size_t>>> uploads;
@@ -290,6 +296,7 @@ struct mdpd_pool {
         for (auto &j : jobs) {
             if (j.second->ev) (void)hipEventDestroy(j.second->ev);
             if (j.second->stage) (void)hipHostFree(j.second->stage);
+            if (j.second->in && !j.second->in_heap) (void)hipHostFree(j.second->in);
         }
         for (auto e : ev_free) (void)hipEventDestroy(e);
         for (auto &pe : prof_open)
@@ -425,11 +432,8 @@ struct mdpd_pool {
         if (j->npad > c || j->ncell + 1 > cs)
             fail(MDPD_E_NOMEM, "job of %d atoms / %d cells does not fit a pool of %lld slots / %lld cells", j->n,
                  j->ncell, c, cs);
-        j->hp.resize(j->npad); j->hv.resize(j->npad);
-        j->ht.resize(j->npad); j->hm.resize(j->npad); j->ho.resize(j->npad); j->himg.resize(j->npad);
-        sys->pack(j->npad, j->hp.data(), j->hv.data(), j->ht.data(), j->hm.data(), j->ho.data(), j->himg.data());
-        j->hph.assign(j->npad, 0.f);
-        for (size_t i = 0; i < sys->h_phi.size() && i < (size_t)j->n; ++i) j->hph[i] = (float)sys->h_phi[i];
+        j->has_phi = !sys->h_phi.empty();
+        pack_input(*j, sys);
         j->id = next_id++;
         if (next_id >= (1 << 27)) next_id = 1;
         j->t_submit = now_s();
@@ -437,6 +441,54 @@ struct mdpd_pool {
         jobs[id] = std::move(j);
         queue.push_back(id);
         return id;
+    }
+
+    // the input block, packed once where the admission kernel reads it: in
+    // pinned memory while the waiting blocks stay below MAX_STAGED (and once
+    // the pool is on its device), else in pageable memory
+    void pack_input(Job &j, const mdpd_system *sys)
+    {
+        const InLayout L = j.in_layout();
+        if (allocated && staged + L.bytes <= MAX_STAGED) {
+            hip_check(hipSetDevice(device), "hipSetDevice");
+            j.in = (char *)pinned.get(L.bytes, j.in_bytes);
+            staged += j.in_bytes;
+        } else {
+            j.in_heap.reset(new char[L.bytes]);
+            j.in = j.in_heap.get();
+        }
+        float4 *p = (float4 *)(j.in + L.pos);
+        float *v = (float *)(j.in + L.vel);
+        int *img = (int *)(j.in + L.image);
+        const double *x = sys->h_x.data(), *u = sys->h_v.data();
+        const int *ty = sys->h_type.data(), *im = sys->h_image.data();
+        for (int i = 0; i < j.n; ++i) {
+            const int t = ty[i] - 1;
+            float tf;
+            memcpy(&tf, &t, 4);
+            p[i] = make_float4((float)x[3 * i], (float)x[3 * i + 1], (float)x[3 * i + 2], tf);
+        }
+        for (int i = 0; i < 3 * j.n; ++i) v[i] = (float)u[i];
+        for (int i = 0; i < j.n; ++i)
+            img[i] = ((im[3 * i] + 512) & 1023) | (((im[3 * i + 1] + 512) & 1023) << 10) |
+                     (((im[3 * i + 2] + 512) & 1023) << 20);
+        memcpy(j.in + L.tag, sys->h_tag.data(), sizeof(int) * j.n);
+        memcpy(j.in + L.mask, sys->h_mask.data(), sizeof(int) * j.n);
+        if (j.has_phi) {
+            float *f = (float *)(j.in + L.phi);
+            for (int i = 0; i < j.n; ++i) f[i] = (size_t)i < sys->h_phi.size() ? (float)sys->h_phi[i] : 0.f;
+        }
+        memcpy(j.in + L.rank, j.ds.rank.data(), sizeof(int) * L.nc1);
+        memcpy(j.in + L.xyz, j.ds.xyz.data(), sizeof(int) * L.nc1);
+        memcpy(j.in + L.coef, j.ds.coef.data(), sizeof(float) * L.ncoef);
+        float *ms = (float *)(j.in + L.mass);
+        for (int k = 0; k < L.nt; ++k) {
+            ms[k] = j.ds.mass[k];
+            ms[L.nt + k] = j.ds.minv[k];
+        }
+        // only the descriptor is kept beside it
+        std::vector<int>().swap(j.ds.rank);
+        std::vector<int>().swap(j.ds.xyz);
     }
 
     // ------------------------------------------------------------------
@@ -506,16 +558,16 @@ struct mdpd_pool {
         hip_check(hipMemcpyAsync(h.data(), dsys.p, sizeof(SysDev) * max_sys, hipMemcpyDeviceToHost, stream),
                   "readback");
         hip_check(hipStreamSynchronize(stream), "readback");
-        bool any = false;
+        std::vector<Job *> fin;
         for (int s = 0; s < max_sys; ++s) {
             const int jid = slot_job[s];
             if (!jid || h[s].job != jid || h[s].phase != PH_DONE) continue;
             Job &j = *jobs[jid];
-            if (j.harvesting) continue;
-            start_harvest(j);
-            any = true;
+            if (!j.harvesting) fin.push_back(&j);
         }
-        if (any) hip_check(hipStreamSynchronize(stream), "harvest before regrow");
+        if (fin.empty()) return;
+        start_harvests(fin);
+        hip_check(hipStreamSynchronize(stream), "harvest before regrow");
     }
 
     // wider neighbor rows for every system, rows rebuilt in place (no re-sort,
@@ -635,56 +687,19 @@ struct mdpd_pool {
                 d.rdf_hist[k] = base + (size_t)k * per;
             }
         }
-        const int npad = j.npad, nc1 = j.ncell + 1, ntw = npad / WAVE;
-        const size_t ncoef = j.ds.coef.size(), nt = j.ntypes;
-        // staging layout (every piece 16-byte aligned)
-        auto al = [](size_t b) { return (b + 15) / 16 * 16; };
-        size_t off[14], at = 0;
-        const size_t sz[14] = {sizeof(float4) * npad, sizeof(float4) * npad, sizeof(int) * npad, sizeof(int) * npad,
-                               sizeof(int) * npad, sizeof(int) * npad, sizeof(int) * nc1, sizeof(int) * nc1,
-                               sizeof(int) * nc1, sizeof(int) * ntw, sizeof(float) * ncoef, sizeof(float) * 2 * nt,
-                               sizeof(SysDev), sizeof(float) * npad};
-        for (int k = 0; k < 14; ++k) { off[k] = at; at += al(sz[k]); }
-        size_t got = 0;
-        char *st = (char *)pinned.get(at, got);
-        memcpy(st + off[0], j.hp.data(), sz[0]);
-        memcpy(st + off[1], j.hv.data(), sz[1]);
-        memcpy(st + off[2], j.ht.data(), sz[2]);
-        memcpy(st + off[3], j.hm.data(), sz[3]);
-        memcpy(st + off[4], j.ho.data(), sz[4]);
-        memcpy(st + off[5], j.himg.data(), sz[5]);
-        memcpy(st + off[13], j.hph.data(), sz[13]);
-        memcpy(st + off[6], j.ds.rank.data(), sz[6]);
-        memcpy(st + off[7], j.ds.xyz.data(), sz[7]);
-        int *cs = (int *)(st + off[8]);
-        for (int k = 0; k < nc1; ++k) cs[k] = s;
-        int *ws = (int *)(st + off[9]);
-        for (int k = 0; k < ntw; ++k) ws[k] = s;
-        memcpy(st + off[10], j.ds.coef.data(), sz[10]);
-        float *ms = (float *)(st + off[11]);
-        for (size_t t = 0; t < nt; ++t) { ms[t] = j.ds.mass[t]; ms[nt + t] = j.ds.minv[t]; }
-        memcpy(st + off[12], &d, sizeof(SysDev));
-        auto up = [&](void *dst, int k) {
-            hip_check(hipMemcpyAsync(dst, st + off[k], sz[k], hipMemcpyHostToDevice, stream), "upload");
-        };
-        up(pos[0].p + pbase, 0);
-        up(vel[0].p + pbase, 1);
-        up(tag[0].p + pbase, 2);
-        up(mask[0].p + pbase, 3);
-        up(origin[0].p + pbase, 4);
-        up(image[0].p + pbase, 5);
-        up(cell_rank.p + cbase, 6);
-        up(cell_xyz.p + cbase, 7);
-        up(cell_sys.p + cbase, 8);
-        up(wave_sys.p + pbase / WAVE, 9);
-        up(coef.p + d.coef_base, 10);
-        hip_check(hipMemcpyAsync(mmass.p + d.mass_base, ms, sizeof(float) * nt, hipMemcpyHostToDevice, stream), "upload");
-        hip_check(hipMemcpyAsync(minv.p + d.mass_base, ms + nt, sizeof(float) * nt, hipMemcpyHostToDevice, stream),
-                  "upload");
-        hip_check(hipMemsetAsync(cell_count.p + (size_t)cbase * SUBCELLS, 0, sizeof(int) * (size_t)nc1 * SUBCELLS, stream),
-                  "memset");
-        up(phi[0].p + pbase, 13);
-        up(dsys.p + s, 12);
+        const InLayout L = j.in_layout();
+        char *st = j.in;
+        size_t got = j.in_bytes;
+        if (j.in_heap) {
+            st = (char *)pinned.get(L.bytes, got);
+            memcpy(st, j.in, L.bytes);
+            j.in_heap.reset();
+        } else {
+            staged -= got;
+        }
+        j.in = nullptr;
+        memcpy(st + L.sys, &d, sizeof(SysDev));
+        hip_check(launch_admit(view(), L, st, s, (int)pbase, (int)cbase, stream), "admit");
         hipEvent_t e = take_event();
         hip_check(hipEventRecord(e, stream), "hipEventRecord");
         uploads.push_back({e, {st, got}});
@@ -702,11 +717,6 @@ struct mdpd_pool {
         if (d.style == STYLE_MDPD && d.rho_bit && !with_rho) { with_rho = true; graph_valid = false; }
         if (d.fix_arb && !with_arb) { with_arb = true; graph_valid = false; }
         if ((d.nrdf || d.ndens) && !with_obs) { with_obs = true; graph_valid = false; }
-        // the host copy of the input is no longer needed
-        std::vector<float4>().swap(j.hp); std::vector<float4>().swap(j.hv);
-        std::vector<int>().swap(j.ht); std::vector<int>().swap(j.hm);
-        std::vector<int>().swap(j.ho); std::vector<int>().swap(j.himg);
-        std::vector<float>().swap(j.hph);
     }
 
     // launches cover particle slots [0, nact) and cell slots [0, ncact): the
@@ -782,6 +792,7 @@ struct mdpd_pool {
     void launch_pass(int sp, PassEvents *ev = nullptr)
     {
         PoolDev P = view();
+        splits_used |= sp;
         auto mark = [&](int k) {
             if (ev) hip_check(hipEventRecord(ev->e[k], stream), "hipEventRecord");
         };
@@ -976,6 +987,7 @@ struct mdpd_pool {
     void handle(const int *st)
     {
         collect_profile(false);
+        std::vector<Job *> fin;
         for (int s = 0; s < max_sys; ++s) {
             const int jid = slot_job[s];
             if (!jid) continue;
@@ -983,30 +995,50 @@ struct mdpd_pool {
             if ((w >> 3) != jid) continue;          // no commit yet for this occupant
             Job &j = *jobs[jid];
             if (j.harvesting) continue;
-            if (w & 2) start_harvest(j);
+            if (w & 2) fin.push_back(&j);
             if (w & 4) need_regrow = true;
         }
+        if (!fin.empty()) start_harvests(fin);
         if (need_regrow) {
             need_regrow = false;
             regrow(0);
         }
     }
 
-    void start_harvest(Job &j)
+    // Jobs that have finished on the device: energy / virial of their last
+    // pass in one launch over the tiles between the first and the last of them
+    // (it skips systems that are not done), their results packed in one
+    // launch, and a copy per job.  A batch whose jobs end together had a
+    // launch of a few tiles per job here, 32 us each.
+    void start_harvests(const std::vector<Job *> &fin)
     {
         PoolDev P = view();
-        const int t0 = (int)(j.part_base / WAVE), nt = j.npad / WAVE;
-        const int style = j.ds.d.style;
-        const bool uni = j.ntypes == 1;
-        // energy / virial of the last pass; the launch whose split matches it runs
-        for (int sp : {1, 2, 4}) hip_check(launch_force_range(P, style, MODE_HARVEST, uni, sp, t0, nt, stream), "harvest");
-        // the results are packed into the system's own neighbor-row range
-        // (no pass reads it once the system has stopped) and copied as one
-        // block; they stay in the pinned stage until the job is released
+        long long lo = cap, hi = 0;
+        int npad_max = 0;
+        std::vector<int> slots;
+        std::set<std::pair<int, bool>> kinds;
+        for (const Job *j : fin) {
+            lo = std::min(lo, j->part_base);
+            hi = std::max(hi, j->part_base + j->npad);
+            npad_max = std::max(npad_max, j->npad);
+            slots.push_back(j->slot);
+            kinds.insert({j->ds.d.style, j->ntypes == 1});
+        }
+        // each system is evaluated by the launch of its last pass's split
+        for (auto &k : kinds)
+            for (int sp : {1, 2, 4})
+                if (splits_used & sp)
+                    hip_check(launch_force_range(P, k.first, MODE_HARVEST, k.second, sp, (int)(lo / WAVE),
+                                                 (int)((hi - lo) / WAVE), stream), "harvest");
+        hip_check(launch_harvest(P, slots.data(), (int)slots.size(), npad_max, stream), "harvest");
+        for (Job *j : fin) copy_harvest(P, *j);
+    }
+
+    // the packed results stay in the pinned stage until the job is released
+    void copy_harvest(const PoolDev &P, Job &j)
+    {
         const size_t bytes = harvest_bytes(j.npad);
-        int *dst = nlist.p + (size_t)t0 * maxnbr * WAVE;
-        const size_t room = (size_t)j.npad * maxnbr * sizeof(int);
-        hip_check(launch_harvest(P, j.slot, (int)j.part_base, j.npad, dst, room, stream), "harvest");
+        const int *dst = nlist.p + harvest_dst(P, (int)j.part_base);
         j.stage = pinned.get(j.result_bytes(), j.stage_bytes);
         hip_check(hipMemcpyAsync(j.stage, dst, bytes, hipMemcpyDeviceToHost, stream), "harvest copy");
         size_t at = bytes;

@@ -1570,24 +1570,26 @@ struct mdpd_system {
         int want = std::max(32, (int)std::ceil(2.0 * expect));
         out.want_maxnbr = (want + NBR_ALIGN - 1) / NBR_ALIGN * NBR_ALIGN;
 
-        // ---- Morton rank of interior cells (order of the sort key's bin part) ----
+        // ---- Morton rank of interior cells (order of the sort key's bin part,
+        // whose bins start at 1): the octants of the enclosing power-of-two
+        // cube in Morton order, those outside the box skipped ----
         const int nc = d.ncell;
-        std::vector<std::pair<uint64_t, int>> order(nc);
-        for (int z = 0; z < d.nb[2]; ++z)
-            for (int y = 0; y < d.nb[1]; ++y)
-                for (int x = 0; x < d.nb[0]; ++x) {
-                    int lin = x + d.nb[0] * (y + d.nb[1] * z);
-                    order[lin] = {morton3(x + 1, y + 1, z + 1), lin};
-                }
-        std::sort(order.begin(), order.end());
         out.rank.assign(nc + 1, 0);
         out.xyz.assign(nc + 1, 0);
-        for (int r = 0; r < nc; ++r) {
-            int lin = order[r].second;
-            out.rank[lin] = r;
-            int x = lin % d.nb[0], y = (lin / d.nb[0]) % d.nb[1], z = lin / (d.nb[0] * d.nb[1]);
-            out.xyz[r] = x | (y << 10) | (z << 20);
-        }
+        int size = 1, r = 0;
+        while (size <= std::max(d.nb[0], std::max(d.nb[1], d.nb[2]))) size *= 2;
+        std::function<void(int, int, int, int)> visit = [&](int x, int y, int z, int s) {
+            if (x > d.nb[0] || y > d.nb[1] || z > d.nb[2]) return;
+            if (s > 1) {
+                for (int o = 0; o < 8; ++o)
+                    visit(x + (o & 1) * s / 2, y + (o >> 1 & 1) * s / 2, z + (o >> 2) * s / 2, s / 2);
+                return;
+            }
+            if (x < 1 || y < 1 || z < 1) return;
+            out.rank[(x - 1) + d.nb[0] * ((y - 1) + d.nb[1] * (z - 1))] = r;
+            out.xyz[r++] = (x - 1) | ((y - 1) << 10) | ((z - 1) << 20);
+        };
+        visit(0, 0, 0, size);
         out.mass.resize(ntypes);
         out.minv.resize(ntypes);
         for (int t = 0; t < ntypes; ++t) { out.mass[t] = (float)mass[t + 1]; out.minv[t] = (float)(1.0 / mass[t + 1]); }
