@@ -10,7 +10,7 @@ import pytest
 
 from conftest import uniform_box
 from test_gpu_arb import DECK, LX, LY, LZ, channel
-from test_gpu_parity import dpd_system, mdpd_system
+from test_gpu_parity import IDX, _neighbor_sets, dpd_system, mdpd_system
 
 pytestmark = pytest.mark.gpu
 
@@ -95,6 +95,14 @@ def test_sorted_order_over_scan_sizes(engine, orc, n, L):
     assert np.array_equal(np.sort(origin), np.arange(n))
     assert np.array_equal(got, orc.sort_keys(xw, (0, 0, 0), (L, L, L), 1.3))
     assert np.all(np.diff(got.astype(np.int64)) >= 0)
+    # and so do the rows (a cell's centres shared by four waves up to 2,560 cells)
+    counts, rows = s.debug_neighbors()
+    mine = _neighbor_sets(origin, counts, rows)
+    xc = np.empty_like(xw)
+    xc[origin] = xw
+    _, want = orc.neighbors(xc, (0, 0, 0), (L, L, L), 1.3)
+    for i in range(n):
+        assert mine[i] == {(int(e) & IDX, int(e) >> 27) for e in want[i]}, i
     s.close()
 
 

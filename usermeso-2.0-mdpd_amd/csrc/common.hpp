@@ -250,9 +250,11 @@ __host__ inline uint32_t premix_host(uint32_t v0, uint32_t v1, int rounds)
 
 // Lane s of workgroup k computes the seed two steps on of system 64 k + s, for
 // the step's commit.  64 TEA rounds are a chain of ~700 dependent instructions,
-// 2.5 us of a commit that every step waits for, so a spare workgroup of a
-// kernel that takes longer computes them: of the first pass (split 1 and the
-// wide kernels), else of the one system's row build.  (In the two- and
+// 2.5 us of a commit that every step waits for, so spare workgroups of a
+// kernel that takes longer compute them: of the first pass (split 1 and the
+// wide kernels), else of the one system's row build.  They are the launch's
+// first (seed_grid of them, a multiple of NXCD): as its last ones they started
+// when thousands of others had been dispatched and ended after them.  (In the two- and
 // four-wave first passes it costs registers: 72 VGPRs, a wave per SIMD less,
 // 480,000 particles 83 -> 98 us.)
 __device__ inline void next_seeds(const PoolDev &P, int k)
@@ -262,6 +264,8 @@ __device__ inline void next_seeds(const PoolDev &P, int k)
     SysDev *d = P.sys + s;
     if (d->active) d->seed_after = premix<64>(d->seed, (uint32_t)(d->step + 2));
 }
+
+static inline int seed_grid(const PoolDev &P) { return xcd_grid((P.nsys + WAVE - 1) / WAVE); }
 
 __device__ inline uint32_t brev32(uint32_t x) { return __builtin_bitreverse32(x); }
 

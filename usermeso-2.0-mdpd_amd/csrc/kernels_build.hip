@@ -449,21 +449,20 @@ constexpr int NL_GRID = 65536;         // its waves (measured against 7,168 and 
 // cell, whose neighbor cells' ranges come from the linear table; otherwise
 // e.x = a cell slot, looked up through its system and the Morton rank table
 template <bool LISTED>
-__device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4 e, int relist, int *s_row)
+__device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4 e, int relist, int part, int parts,
+                                                          int *s_row)
 {
     int s, xyz, c0, c1, cs = e.x;
     if (LISTED) {
         s = e.x; xyz = e.y; c0 = e.z; c1 = e.w;
     } else {
-        s = P.cell_sys[cs];
+        s = P.one ? 0 : P.cell_sys[cs];
         if (s < 0) return;
     }
     SysDev *d = P.sys + s;
     const int cb = d->cell_base;
     if (!LISTED) {
-        // relist: the systems not flagged stale; otherwise the one system when
-        // k_keys found it stale
-        if (!d->active || (relist ? d->stale != 0 : P.work_count[1] == 0)) return;
+        if (relist && (!d->active || d->stale != 0)) return;       // a relist: the systems not flagged stale
         if (cs < cb || cs >= cb + d->ncell) return;       // the end slot holds no cell
         c0 = P.cell_start[cs * SUBCELLS];
         c1 = P.cell_start[(cs + 1) * SUBCELLS];
@@ -505,6 +504,9 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
     const int ntot = __builtin_amdgcn_readlane(kend, 26);
     const float rc2 = d->rc2_list;
     const int maxnbr = P.maxnbr;
+    // a cell away from the box's edges has no shifted candidate: four of eleven
+    // cross-lane reads per tile less
+    const bool images = __builtin_amdgcn_ballot_w64(lane < 27 && kcode != (uint32_t)IMG_ZERO) != 0;
     for (int cg = c0; cg < c1; cg += WAVE) {
         const int ng = min(WAVE, c1 - cg);
         int cntv = 0;                                       // lane l: row length of centre cg + l
@@ -527,18 +529,23 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
                 }
                 // every shuffle with the whole wave active (a lane reads a
                 // source lane's register only while that lane is active)
-                const int st_k = __shfl(kst, k), pre_k = __shfl(kpre, k);
-                const uint32_t code = (uint32_t)__shfl((int)kcode, k);
-                const float sx_k = __shfl(ksx, k), sy_k = __shfl(ksy, k), sz_k = __shfl(ksz, k);
+                const int j0 = __shfl(kst - kpre, k);
                 const bool valid = t < ntot;
-                const int j = valid ? st_k + (t - pre_k) : c0;
+                const int j = valid ? j0 + t : c0;
                 const float4 q = pos[j];
-                qx[m] = valid ? q.x + sx_k : __builtin_inff();
-                qy[m] = valid ? q.y + sy_k : __builtin_inff();
-                qz[m] = valid ? q.z + sz_k : __builtin_inff();
+                qx[m] = valid ? q.x : __builtin_inff();
+                qy[m] = valid ? q.y : __builtin_inff();
+                qz[m] = valid ? q.z : __builtin_inff();
+                uint32_t code = IMG_ZERO;
+                if (images) {
+                    qx[m] += __shfl(ksx, k);
+                    qy[m] += __shfl(ksy, k);
+                    qz[m] += __shfl(ksz, k);
+                    code = (uint32_t)__shfl((int)kcode, k);
+                }
                 qe[m] = (int)((uint32_t)j | (code << IMG_SHIFT));
             }
-            for (int c = cg; c < cg + ng; ++c) {
+            for (int c = cg + part; c < cg + ng; c += parts) {
                 const int cl = c - cg;
                 const float pcx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pg.x), cl));
                 const float pcy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pg.y), cl));
@@ -582,8 +589,9 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
                 if (lane == cl) cntv = q0 + n - shift;
             }
         }
-        if (lane < ng) P.ncount[cg + lane] = cntv;
-        if (__ballot(lane < ng && cntv > maxnbr) && lane == 0) atomicOr(&d->overflow, 1);
+        const bool mine = lane < ng && (parts == 1 || lane % parts == part);
+        if (mine) P.ncount[cg + lane] = cntv;
+        if (__ballot(mine && cntv > maxnbr) && lane == 0) atomicOr(&d->overflow, 1);
     }
 }
 
@@ -601,15 +609,21 @@ __device__ inline void commit_rebuild_sys(const PoolDev &P, int s)
 
 // one wave per cell slot (a relist, or one system): eight waves per SIMD
 // (seven candidate tiles in registers, no spills), measured faster than seven
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) k_nlist(PoolDev P, int relist, int ncells)
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) k_nlist(PoolDev P, int relist, int ncells, int lparts, int nseed)
 {
     __shared__ int s_row[NL_ITER * WAVE];                   // one centre's entries of one batch
-    // the one system's rebuild is committed here: the row build reads only its
-    // geometry and the flag word
-    if (!relist && blockIdx.x == 0 && threadIdx.x == 0 && P.work_count[1]) commit_rebuild_sys(P, 0);
-    if ((int)blockIdx.x >= xcd_grid(ncells)) { next_seeds(P, 0); return; }
-    const int cs = xcd_logical(blockIdx.x, ncells);        // cell slot (Morton rank order)
-    if (cs < ncells) nlist_cell<false>(P, make_int4(cs, 0, 0, 0), relist, s_row);
+    const int nu = ncells << lparts;                        // 2^lparts waves share a cell's centres
+    const int b = (int)blockIdx.x - nseed;
+    if (b < 0) { next_seeds(P, blockIdx.x); return; }
+    if (!relist) {
+        // the one system, when k_keys found it stale; its rebuild is committed
+        // here: the row build reads only its geometry and the flag word
+        if (P.work_count[1] == 0) return;
+        if (b == 0 && threadIdx.x == 0) commit_rebuild_sys(P, 0);
+    }
+    const int u = xcd_logical(b, nu), cs = u >> lparts;     // cell slot (Morton rank order)
+    if (cs < ncells)
+        nlist_cell<false>(P, make_int4(cs, 0, 0, 0), relist, u & ((1 << lparts) - 1), 1 << lparts, s_row);
 }
 
 // the worklist walk; it also commits the rebuild of every re-sorted system
@@ -624,7 +638,7 @@ __global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(NL_WA
     const int x = blockIdx.x % NXCD, per = gridDim.x / NXCD;
     const int hi = (int)((long long)n * (x + 1) / NXCD);
     for (int w = (int)((long long)n * x / NXCD) + blockIdx.x / NXCD; w < hi; w += per)
-        nlist_cell<true>(P, P.cell_work[w], 0, s_row);
+        nlist_cell<true>(P, P.cell_work[w], 0, 0, 1, s_row);
 }
 
 // overflow flags of the sorted systems cleared before their rows are rebuilt
@@ -661,13 +675,19 @@ __global__ void __launch_bounds__(256) k_signatures(PoolDev P)
 // host launchers
 // ----------------------------------------------------------------------------
 static inline int nblk(int n, int b) { return (n + b - 1) / b; }
+// One system of few cells: four waves share a cell's centres, each listing the
+// stencil for itself (1,000 particles: 21 -> 13 us; every cell of a larger
+// system has its wave at once anyway, and the launch grows by 0.2 ns a wave).
+constexpr int NL_FEW = 2560, NL_LPARTS = 2;
+
 static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t st)
 {
     if (P.ncact <= 0) return;
-    if (relist || !nlist_listed(P))
-        hipLaunchKernelGGL(k_nlist, dim3(xcd_grid(P.ncact) + (seeds ? 1 : 0)), dim3(WAVE), 0, st, P, relist,
-                           P.ncact);
-    else
+    if (relist || !nlist_listed(P)) {
+        const int lparts = P.one && P.ncact <= NL_FEW ? NL_LPARTS : 0;
+        hipLaunchKernelGGL(k_nlist, dim3(xcd_grid(P.ncact << lparts) + (seeds ? seed_grid(P) : 0)), dim3(WAVE), 0, st, P,
+                           relist, P.ncact, lparts, seeds ? seed_grid(P) : 0);
+    } else
         hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(P.ncact))), dim3(WAVE), 0, st, P);
 }
 

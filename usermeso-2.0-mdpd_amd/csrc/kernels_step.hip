@@ -127,16 +127,14 @@ __device__ inline void finish_density(const PoolDev &P, const SysDev *d, int i, 
 }
 
 template <bool WITH_RHO, int SPLIT>
-__global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles)
+__global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles, int nseed)
 {
     constexpr int STAGE = 32 / SPLIT;   // LDS-staged compact entries per lane (measured best)
     __shared__ int s_c[SPLIT][STAGE * WAVE];
     __shared__ float s_sum[SPLIT][WAVE];
-    if (SPLIT == 1 && (int)blockIdx.x >= xcd_grid(ntiles)) {
-        next_seeds(P, blockIdx.x - xcd_grid(ntiles));
-        return;
-    }
-    const int tile = xcd_logical(blockIdx.x, ntiles);
+    const int b = (int)blockIdx.x - (SPLIT == 1 ? nseed : 0);
+    if (SPLIT == 1 && b < 0) { next_seeds(P, blockIdx.x); return; }
+    const int tile = xcd_logical(b, ntiles);
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = tile * WAVE + lane;
@@ -262,15 +260,16 @@ template <int SPLIT>
 constexpr int FS_WAVES = SPLIT == 2 ? 10 : 12;
 
 template <bool WITH_RHO, int SPLIT>
-__global__ void __launch_bounds__(WAVE * FS_WAVES<SPLIT>) k_first_wide(PoolDev P, int ntiles)
+__global__ void __launch_bounds__(WAVE * FS_WAVES<SPLIT>) k_first_wide(PoolDev P, int ntiles, int nseed)
 {
     constexpr int NW = FS_WAVES<SPLIT>;
     static_assert(NW % SPLIT == 0, "a wave keeps its sub-row from round to round");
     __shared__ float2 s_w[WITH_RHO ? NW * NBR_CHUNK : 1][WAVE];    // weight factors of each entry
     __shared__ int s_n[NW][WAVE];                                  // in-cutoff entries of each chunk
     __shared__ float s_sum[SPLIT][WAVE];
-    if ((int)blockIdx.x >= xcd_grid(ntiles)) { next_seeds(P, blockIdx.x - xcd_grid(ntiles)); return; }
-    const int tile = xcd_logical(blockIdx.x, ntiles);
+    const int b = (int)blockIdx.x - nseed;
+    if (b < 0) { next_seeds(P, blockIdx.x); return; }
+    const int tile = xcd_logical(b, ntiles);
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int i = tile * WAVE + lane;
@@ -1310,19 +1309,19 @@ bool first_seeds(int split, int nt) { return split == 1 || nt <= WIDE_TILES; }
 template <bool WITH_RHO>
 static hipError_t launch_first_t(const PoolDev &P, int split, int nt, hipStream_t st)
 {
-    // the tiles, then the seed workgroups
-    const dim3 g(xcd_grid(nt) + (first_seeds(split, nt) ? (P.nsys + WAVE - 1) / WAVE : 0));
+    const int ns = first_seeds(split, nt) ? seed_grid(P) : 0;       // seed workgroups, then the tiles
+    const dim3 g(ns + xcd_grid(nt));
     const bool wide = nt <= WIDE_TILES;
     if (split == 1)
-        hipLaunchKernelGGL((k_first<WITH_RHO, 1>), g, dim3(WAVE), 0, st, P, nt);
+        hipLaunchKernelGGL((k_first<WITH_RHO, 1>), g, dim3(WAVE), 0, st, P, nt, ns);
     else if (split == 2 && wide)
-        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 2>), g, dim3(WAVE * FS_WAVES<2>), 0, st, P, nt);
+        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 2>), g, dim3(WAVE * FS_WAVES<2>), 0, st, P, nt, ns);
     else if (split == 2)
-        hipLaunchKernelGGL((k_first<WITH_RHO, 2>), g, dim3(WAVE * 2), 0, st, P, nt);
+        hipLaunchKernelGGL((k_first<WITH_RHO, 2>), g, dim3(WAVE * 2), 0, st, P, nt, ns);
     else if (split == 4 && wide)
-        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 4>), g, dim3(WAVE * FS_WAVES<4>), 0, st, P, nt);
+        hipLaunchKernelGGL((k_first_wide<WITH_RHO, 4>), g, dim3(WAVE * FS_WAVES<4>), 0, st, P, nt, ns);
     else if (split == 4)
-        hipLaunchKernelGGL((k_first<WITH_RHO, 4>), g, dim3(WAVE * 4), 0, st, P, nt);
+        hipLaunchKernelGGL((k_first<WITH_RHO, 4>), g, dim3(WAVE * 4), 0, st, P, nt, ns);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
