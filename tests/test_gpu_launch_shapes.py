@@ -76,9 +76,11 @@ def test_small_system_equals_its_pool_job(engine, case, split):
     s.close()
 
 
-# (particles, box edge): sub-cells of one scan chunk, just past it, several
-# chunks, and past the largest count the one-launch scan takes
-@pytest.mark.parametrize("n, L", [(300, 5.3), (2000, 13.1), (2000, 14.4), (3000, 27.5), (4000, 46.0)])
+# (particles, box edge): the one-launch sort at its smallest, at one particle
+# per thread and past it, at its largest and past it; a box of too many cells
+# for it (several chunks of the one-launch scan); one past that scan's largest
+@pytest.mark.parametrize("n, L", [(300, 5.3), (1024, 5.6), (1025, 5.6), (2000, 13.1), (2000, 14.4), (10240, 12.0),
+                                  (10241, 12.0), (3000, 27.5), (4000, 46.0)])
 def test_sorted_order_over_scan_sizes(engine, orc, n, L):
     x, v = uniform_box(n, L, int(10 * L))
     s = mdpd_system(engine, x, v, L)

@@ -181,7 +181,6 @@ struct PoolDev {
     int *pslot;          // arrival rank within the sub-cell; after the re-sort: sub-cell slot of each sorted slot
     int *psub;           // 12-bit sub-bin Morton code
     int *tmp;            // particle index per sorted slot (pre-order)
-    unsigned long long *key;  // optional: reference sort key per particle (debug)
     int *cell_count;     // per sub-cell slot
     int *cell_start;     // per sub-cell slot, global particle index; slot ncell * SUBCELLS = end
     int *cell_xyz;       // packed interior coords of the cell at this Morton rank
@@ -263,6 +262,25 @@ __device__ inline void next_seeds(const PoolDev &P, int k)
     if (threadIdx.x >= WAVE || s >= P.nsys) return;
     SysDev *d = P.sys + s;
     if (d->active) d->seed_after = premix<64>(d->seed, (uint32_t)(d->step + 2));
+}
+
+// A step done: the buffer it wrote becomes current, the next step's seed.
+// seeded: a kernel of the step left the seed two steps on in seed_after.
+__device__ inline void commit_advance(SysDev *d, bool moved, bool seeded)
+{
+    d->sel ^= 1;
+    d->step += 1;
+    d->seed_next = seeded ? d->seed_after : premix<64>(d->seed, (uint32_t)(d->step + 1));
+    d->stale = moved ? 1 : 0;
+}
+
+// the same with the reneighbor decision of Neighbor::decide
+__device__ inline void commit_decide(SysDev *d, bool moved, bool seeded)
+{
+    commit_advance(d, false, seeded);
+    const int ago = ++d->ago;
+    const bool due = ago >= d->n_delay && ago % d->n_every == 0;
+    d->stale = due && (!d->n_check || moved) ? 1 : 0;
 }
 
 static inline int seed_grid(const PoolDev &P) { return xcd_grid((P.nsys + WAVE - 1) / WAVE); }

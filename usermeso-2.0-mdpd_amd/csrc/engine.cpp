@@ -258,8 +258,11 @@ int mdpd_debug_sorted(mdpd_system *sys, int *origin_out, unsigned long long *key
             memcpy(origin_out, h.data(), sizeof(int) * n);
         }
         if (key_out) {
-            // k_sortgather copies each particle's key to key[cap + sorted slot]
-            auto k = sys->download(sys->key.p + sys->cap, n);
+            // two words per key in the compact rows (free between passes)
+            static_assert(NBR_ALIGN >= 2, "a key per particle fits the narrowest compact rows");
+            unsigned long long *keys = (unsigned long long *)sys->clist.p;
+            hip_check(launch_sort_keys(sys->view(), keys, sys->stream), "sort keys");
+            auto k = sys->download(keys, n);
             hip_check(hipStreamSynchronize(sys->stream), "sync");
             memcpy(key_out, k.data(), sizeof(unsigned long long) * n);
         }

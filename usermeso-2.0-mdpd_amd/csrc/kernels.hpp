@@ -23,11 +23,16 @@ enum CommitKind : int {
 };
 
 // rebuild phase: wrap, keys, sort, gather, neighbor rows, commit (stale systems only)
-hipError_t launch_rebuild(const PoolDev &P, int split, hipStream_t st);
+// split: of the pass that follows; commit: the commit of the pass before
+// (COMMIT_DECIDE, after_pass) is made first, for the systems whose rebuild can
+hipError_t launch_rebuild(const PoolDev &P, int split, bool commit, hipStream_t st);
+bool commit_in_rebuild(const PoolDev &P);
 hipError_t launch_nlist_only(const PoolDev &P, hipStream_t st);
 // neighbor rows of every sorted active system rebuilt in place (row width grew)
 hipError_t launch_relist(const PoolDev &P, hipStream_t st);
 hipError_t launch_signatures(const PoolDev &P, hipStream_t st);
+// one system: its sort keys at the last build, in sorted order
+hipError_t launch_sort_keys(const PoolDev &P, unsigned long long *out, hipStream_t st);
 
 // per step
 // first pass of a step: density (mDPD with the density fix) and compact rows

@@ -21,6 +21,55 @@ namespace mdpd {
 // per cell slot: its slots are few and the list would only add its own cost.
 __host__ __device__ inline bool nlist_listed(const PoolDev &P) { return !P.one; }
 
+// particle at p with packed image flags img wrapped into the box (Domain::pbc
+// in FP32)
+__device__ inline void wrap_particle(const SysDev *d, float4 &p, int &img)
+{
+    float c[3] = {p.x, p.y, p.z};
+    int im[3] = {(img & 1023) - 512, ((img >> 10) & 1023) - 512, ((img >> 20) & 1023) - 512};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float flo = d->lo[a], fhi = d->hi[a], prd = d->L[a];
+        float v = c[a];
+        if (v < flo) { v = v + prd; im[a] -= 1; }
+        if (v >= fhi) { v = v - prd; v = fmaxf(v, flo); im[a] += 1; }
+        c[a] = v;
+    }
+    p.x = c[0]; p.y = c[1]; p.z = c[2];
+    img = ((im[0] + 512) & 1023) | (((im[1] + 512) & 1023) << 10) | (((im[2] + 512) & 1023) << 20);
+}
+
+// bin coordinates b of a wrapped position and its 12-bit sub-bin Morton code
+__device__ inline uint32_t particle_bins(const SysDev *d, const float4 &p, int b[3])
+{
+    const float c[3] = {p.x, p.y, p.z};
+    uint32_t sub[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        // bin: (int)((x - lo) * bininv + 1.0), FP64, clamped to the interior
+        const double t = ((double)c[a] - d->lo_d[a]) * d->bininv_d[a];
+        const double u = t + 1.0;
+        int bb = (int)u;
+        bb = bb > d->mbin[a] - 2 ? d->mbin[a] - 2 : bb;
+        bb = bb < 1 ? 1 : bb;
+        b[a] = bb;
+        // sub-bin: (x - (bin-1) * binsize) * 16 * bininv (atom_meso.cu:298-300)
+        const double off = (double)(uint32_t)(bb - 1) * d->binsize_d[a];
+        const double rel = (double)c[a] - off;
+        const double sc = rel * (16.0 * d->bininv_d[a]);
+        int ss = (int)sc;
+        ss = ss > 15 ? 15 : ss;
+        ss = ss < 0 ? 0 : ss;
+        sub[a] = (uint32_t)ss;
+    }
+    // four bits per axis, bit i to bit 3 i (+ axis)
+    uint32_t z = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        z |= ((sub[a] & 1) | (sub[a] & 2) << 2 | (sub[a] & 4) << 4 | (sub[a] & 8) << 6) << a;
+    return z;
+}
+
 // --------------------------------------------------------------------------
 // K1: wrap into the box (Domain::pbc in FP32), reference sort key, sub-cell
 // slot (cell slot * SUBCELLS + top bits of the sub-bin key), arrival rank
@@ -48,42 +97,11 @@ __global__ void __launch_bounds__(256) k_keys(PoolDev P)
     const int cur = d->sel, cura = d->sela;
     float4 p = P.pos[cur][i];
     int img = P.image[cura][i];
-    float c[3] = {p.x, p.y, p.z};
-    int im[3] = {(img & 1023) - 512, ((img >> 10) & 1023) - 512, ((img >> 20) & 1023) - 512};
-    for (int a = 0; a < 3; ++a) {
-        const float flo = d->lo[a], fhi = d->hi[a], prd = d->L[a];
-        float v = c[a];
-        if (v < flo) { v = v + prd; im[a] -= 1; }
-        if (v >= fhi) { v = v - prd; v = fmaxf(v, flo); im[a] += 1; }
-        c[a] = v;
-    }
-    P.pos[cur][i] = make_float4(c[0], c[1], c[2], p.w);
-    P.image[cura][i] = ((im[0] + 512) & 1023) | (((im[1] + 512) & 1023) << 10) | (((im[2] + 512) & 1023) << 20);
-
+    wrap_particle(d, p, img);
+    P.pos[cur][i] = p;
+    P.image[cura][i] = img;
     int b[3];
-    uint32_t sub[3];
-    for (int a = 0; a < 3; ++a) {
-        // bin: (int)((x - lo) * bininv + 1.0), FP64, clamped to the interior
-        const double t = ((double)c[a] - d->lo_d[a]) * d->bininv_d[a];
-        const double u = t + 1.0;
-        int bb = (int)u;
-        bb = bb > d->mbin[a] - 2 ? d->mbin[a] - 2 : bb;
-        bb = bb < 1 ? 1 : bb;
-        b[a] = bb;
-        // sub-bin: (x - (bin-1) * binsize) * 16 * bininv (atom_meso.cu:298-300)
-        const double off = (double)(uint32_t)(bb - 1) * d->binsize_d[a];
-        const double rel = (double)c[a] - off;
-        const double sc = rel * (16.0 * d->bininv_d[a]);
-        int ss = (int)sc;
-        ss = ss > 15 ? 15 : ss;
-        ss = ss < 0 ? 0 : ss;
-        sub[a] = (uint32_t)ss;
-    }
-    const uint32_t z2 = (uint32_t)morton3(sub[0], sub[1], sub[2]);
-    if (P.key) {
-        const uint64_t z1 = morton3((uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2]);
-        P.key[i] = (z1 << d->l1_shift) | z2;
-    }
+    const uint32_t z2 = particle_bins(d, p, b);
     const int lin = (b[0] - 1) + d->nb[0] * ((b[1] - 1) + d->nb[1] * (b[2] - 1));
     gc = (d->cell_base + P.cell_rank[d->cell_base + lin]) * SUBCELLS + (int)(z2 >> SUBCELL_SHIFT);
     P.pcell[i] = gc;
@@ -399,7 +417,122 @@ __global__ void __launch_bounds__(256) k_sortgather(PoolDev P)
     P.image[cura ^ 1][dst] = im;
     P.phi[cura ^ 1][dst] = ph;
     P.pslot[dst] = cell;
-    if (P.key) P.key[(size_t)P.cap + dst] = P.key[i];
+}
+
+// --------------------------------------------------------------------------
+// K1 to K4 for one small system in one launch: a workgroup holds the sub-cell
+// counts and the sort keys in LDS, each thread up to SORT1_PER particles.  Four
+// launches of a few workgroups cost 6.8 us per step when no re-sort is due
+// and 10 to 17 us when one is; this one 1.7 us, and 6 us at 1,000 particles,
+// 29 us at 8,667 (~340 instructions per particle on one CU), where it still
+// wins: a re-sort is due every third step.  `commit`: the previous step's
+// commit (COMMIT_DECIDE) is made here first, one launch of 2.7 us less.
+// --------------------------------------------------------------------------
+constexpr int SORT1_BLK = 1024, SORT1_PER = 10, SORT1_N = SORT1_BLK * SORT1_PER, SORT1_SUB = 16384;
+
+template <int PER>
+__global__ void __launch_bounds__(SORT1_BLK) k_sort_one(PoolDev P, int commit, int seeded)
+{
+    __shared__ __align__(16) int s_cnt[SORT1_SUB + 4];     // counts, then first slots
+    __shared__ uint32_t s_key[SORT1_N];                    // sub-bin key << 14 | previous index, by sub-cell
+    __shared__ int s_wave[SORT1_BLK / WAVE], s_now[3];      // stale, sel, sela after the commit
+    SysDev *d = P.sys;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const bool skip = !d->active || (commit && d->overflow);
+    if (commit && !skip) {
+        const int nt = d->npad / WAVE;
+        const int any = __syncthreads_or(t < nt ? P.moved[t] : 0);
+        if (t == 0) commit_decide(d, any != 0, seeded);
+    }
+    if (t == 0) {
+        s_now[0] = skip ? 0 : d->stale;
+        s_now[1] = d->sel;
+        s_now[2] = d->sela;
+    }
+    __syncthreads();
+    const int stale = s_now[0], cur = s_now[1], cura = s_now[2];
+    if (t == 0) P.work_count[1] = stale;                   // the row build's flag
+    if (!stale) return;
+    const int n = d->n, nsub = d->ncell * SUBCELLS;        // part_base and cell_base are 0
+    for (int c = 4 * t; c < nsub; c += 4 * SORT1_BLK) *(int4 *)(s_cnt + c) = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    uint32_t pk[PER];                                      // sub-cell << 12 | sub-bin key
+    int slot[PER];                                         // arrival rank in the sub-cell
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = k * SORT1_BLK + t;
+        if (k * SORT1_BLK >= n) break;
+        if (i < n) {
+            float4 p = P.pos[cur][i];
+            int img = P.image[cura][i], b[3];
+            wrap_particle(d, p, img);
+            const uint32_t z2 = particle_bins(d, p, b);
+            const int lin = (b[0] - 1) + d->nb[0] * ((b[1] - 1) + d->nb[1] * (b[2] - 1));
+            const int gc = P.cell_rank[lin] * SUBCELLS + (int)(z2 >> SUBCELL_SHIFT);
+            pk[k] = (uint32_t)gc << 12 | z2;
+            slot[k] = atomicAdd(s_cnt + gc, 1);
+        }
+    }
+    __syncthreads();
+    // exclusive scan, sixteen counts per thread
+    int4 v[4];
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int c = 16 * t + 4 * u;
+        v[u] = c < nsub ? *(const int4 *)(s_cnt + c) : make_int4(0, 0, 0, 0);
+        sum += v[u].x + v[u].y + v[u].z + v[u].w;
+    }
+    const int incl = wave_incl_scan(sum, lane);
+    if (lane == 63) s_wave[wv] = incl;
+    __syncthreads();
+    int run = incl - sum;
+    for (int k = 0; k < wv; ++k) run += s_wave[k];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int c = 16 * t + 4 * u;
+        const int4 st = make_int4(run, run + v[u].x, run + v[u].x + v[u].y, run + v[u].x + v[u].y + v[u].z);
+        run = st.w + v[u].w;
+        if (c < nsub) {
+            *(int4 *)(s_cnt + c) = st;
+            ((int4 *)P.cell_start)[c / 4] = st;
+        }
+    }
+    if (t == 0) s_cnt[nsub] = P.cell_start[nsub] = n;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = k * SORT1_BLK + t;
+        if (k * SORT1_BLK >= n) break;
+        if (i < n) s_key[s_cnt[pk[k] >> 12] + slot[k]] = (pk[k] & 4095u) << 14 | (uint32_t)i;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = k * SORT1_BLK + t;
+        if (k * SORT1_BLK >= n) break;
+        if (i < n) {
+            float4 p = P.pos[cur][i];
+            const float4 vel = P.vel[cur][i];
+            int img = P.image[cura][i];
+            const int tg = P.tag[cura][i], mk = P.mask[cura][i], og = P.origin[cura][i];
+            const float ph = P.phi[cura][i];
+            wrap_particle(d, p, img);
+            const int gc = (int)(pk[k] >> 12);
+            const uint32_t key = (pk[k] & 4095u) << 14 | (uint32_t)i;
+            const int lo = s_cnt[gc], hi = s_cnt[gc + 1];
+            int dst = lo;
+            for (int g = lo; g < hi; ++g) dst += s_key[g] < key;
+            P.pos[cur ^ 1][dst] = p;
+            P.vel[cur ^ 1][dst] = vel;
+            P.xhold[dst] = p;
+            P.tag[cura ^ 1][dst] = tg;
+            P.mask[cura ^ 1][dst] = mk;
+            P.origin[cura ^ 1][dst] = og;
+            P.image[cura ^ 1][dst] = img;
+            P.phi[cura ^ 1][dst] = ph;
+        }
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -652,6 +785,20 @@ __global__ void k_clear_overflow(PoolDev P)
 }
 
 // --------------------------------------------------------------------------
+// The reference's 2-level Morton keys of one system's particles at the last
+// build, in sorted order (parity hook; the sort itself orders sub-cells).
+// --------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_sort_keys(PoolDev P, unsigned long long *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const SysDev *d = P.sys;
+    if (i >= d->n) return;
+    int b[3];
+    const uint32_t z2 = particle_bins(d, P.xhold[i], b);
+    out[i] = (morton3((uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2]) << d->l1_shift) | z2;
+}
+
+// --------------------------------------------------------------------------
 // Signatures of the current step (setup only; in the step loop the fused
 // force epilogue writes them for the following step).
 // --------------------------------------------------------------------------
@@ -691,9 +838,26 @@ static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t s
         hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(P.ncact))), dim3(WAVE), 0, st, P);
 }
 
-hipError_t launch_rebuild(const PoolDev &P, int split, hipStream_t st)
+bool commit_in_rebuild(const PoolDev &P)
+{
+    return P.one && P.nact <= SORT1_N && (P.ncellslots - 1) * SUBCELLS <= SORT1_SUB;
+}
+
+hipError_t launch_rebuild(const PoolDev &P, int split, bool commit, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
+    const bool small = commit_in_rebuild(P);
+    if (commit && !small) return hipErrorInvalidValue;
+    if (small) {
+        // such a system's first pass computes the seeds (at most 160 tiles)
+        const int c = commit ? 1 : 0;
+        if (P.nact <= SORT1_BLK)
+            hipLaunchKernelGGL((k_sort_one<1>), dim3(1), dim3(SORT1_BLK), 0, st, P, c, 1);
+        else
+            hipLaunchKernelGGL((k_sort_one<SORT1_PER>), dim3(1), dim3(SORT1_BLK), 0, st, P, c, 1);
+        launch_nlist(P, 0, P.one && !first_seeds(split, P.nact / WAVE), st);
+        return hipGetLastError();
+    }
     const dim3 g(nblk(P.nact, 256)), b(256);
     hipLaunchKernelGGL(k_keys, g, b, 0, st, P);
     const long long nsub = P.maxsub > 0 ? (long long)P.maxsub : (long long)P.ncellslots * SUBCELLS;
@@ -727,6 +891,13 @@ hipError_t launch_relist(const PoolDev &P, hipStream_t st)
     if (P.nact == 0) return hipSuccess;
     hipLaunchKernelGGL(k_clear_overflow, dim3(nblk(P.nsys, 64)), dim3(64), 0, st, P);
     launch_nlist(P, 1, false, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_sort_keys(const PoolDev &P, unsigned long long *out, hipStream_t st)
+{
+    if (!P.one || !out) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_sort_keys, dim3(nblk(P.nact, 256)), dim3(256), 0, st, P, out);
     return hipGetLastError();
 }
 

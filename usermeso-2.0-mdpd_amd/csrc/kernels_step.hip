@@ -363,15 +363,6 @@ __device__ inline uint32_t next_signature(const SysDev *d, int tag, float vx, fl
     return d->style == STYLE_MDPD ? sig_mdpd(tag, d->seed_next) : sig_dpd(tag, d->seed_next, vx, vy, vz);
 }
 
-// seeded: a kernel of the step left the seed two steps on in seed_after
-__device__ inline void commit_advance(SysDev *d, bool moved, bool seeded)
-{
-    d->sel ^= 1;
-    d->step += 1;
-    d->seed_next = seeded ? d->seed_after : premix<64>(d->seed, (uint32_t)(d->step + 1));
-    d->stale = moved ? 1 : 0;
-}
-
 __global__ void __launch_bounds__(BLK) k_initial(PoolDev P, int nlogical)
 {
     const int lb = xcd_logical(blockIdx.x, nlogical);
@@ -1129,10 +1120,7 @@ __global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, in
             }
             P.status[blockIdx.x] = (d->job << 3) | (d->stale ? 1 : 0) | (d->phase == PH_DONE ? 2 : 0);
         } else if (advance == COMMIT_DECIDE) {
-            commit_advance(d, false, seeded);
-            const int ago = ++d->ago;
-            const bool due = ago >= d->n_delay && ago % d->n_every == 0;
-            d->stale = due && (!d->n_check || s_any != 0) ? 1 : 0;
+            commit_decide(d, s_any != 0, seeded);
         } else if (advance == COMMIT_ADVANCE) {
             commit_advance(d, s_any != 0, seeded);
         } else {

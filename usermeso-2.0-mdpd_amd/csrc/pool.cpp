@@ -345,7 +345,7 @@ struct mdpd_pool {
         }
         P.xhold = xhold.p; P.rho = rho.p; P.pr = pr.p; P.frc = frc.p; P.vir = vir.p; P.vend = vend.p;
         P.phi[0] = phi[0].p; P.phi[1] = phi[1].p;
-        P.pcell = pcell.p; P.pslot = pslot.p; P.psub = psub.p; P.tmp = tmp.p; P.key = nullptr;
+        P.pcell = pcell.p; P.pslot = pslot.p; P.psub = psub.p; P.tmp = tmp.p;
         P.cell_count = cell_count.p; P.cell_start = cell_start.p; P.cell_xyz = cell_xyz.p;
         P.cell_rank = cell_rank.p; P.cell_sys = cell_sys.p;
         P.work_count = work_count.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
@@ -797,7 +797,7 @@ struct mdpd_pool {
             if (ev) hip_check(hipEventRecord(ev->e[k], stream), "hipEventRecord");
         };
         mark(PP_REBUILD);
-        hip_check(launch_rebuild(P, sp, stream), "rebuild");
+        hip_check(launch_rebuild(P, sp, false, stream), "rebuild");
         mark(PP_FIRST);
         hip_check(launch_first(P, with_rho, sp, stream), "first pass");
         mark(PP_FORCE);

@@ -225,7 +225,6 @@ struct mdpd_system {
     DevBuf<int4> cell_work;
     DevBuf<int2> cell_lse;
     DevBuf<int> nlist, ncount, clist, ccount, wave_sys, moved, status, cl, wall_near;
-    DevBuf<unsigned long long> key;
     DevBuf<SysDev> dsys;
     int *pinned = nullptr;            // host-visible readback of flags
     static constexpr size_t STAGE_WORDS = 1 << 17;
@@ -245,6 +244,8 @@ struct mdpd_system {
     // reads the device step counter once per batch of STEP_BATCH steps ----
     bool use_graph = true;
     hipGraphExec_t gexec = nullptr;
+    hipGraphExec_t gsteps = nullptr;           // GRAPH_STEPS steps: a graph launch costs the host ~16 us
+    static constexpr int GRAPH_STEPS = 8;
     std::map<uint32_t, hipGraphExec_t> gobs;   // steps with observable samples, by sample mask
     bool graph_valid = false;
     static constexpr int STEP_BATCH = 64;
@@ -252,6 +253,7 @@ struct mdpd_system {
     ~mdpd_system()
     {
         if (gexec) (void)hipGraphExecDestroy(gexec);
+        if (gsteps) (void)hipGraphExecDestroy(gsteps);
         for (auto &v : gobs) (void)hipGraphExecDestroy(v.second);
         for (auto &f : fixes) {
             try { finish_obs(f); } catch (...) {}
@@ -1449,7 +1451,7 @@ struct mdpd_system {
         }
         P.xhold = xhold.p; P.rho = rho.p; P.pr = pr.p; P.frc = frc.p; P.vir = vir.p; P.vend = vend.p;
         P.phi[0] = phi[0].p; P.phi[1] = phi[1].p;
-        P.pcell = pcell.p; P.pslot = pslot.p; P.psub = psub.p; P.tmp = tmp.p; P.key = key.p;
+        P.pcell = pcell.p; P.pslot = pslot.p; P.psub = psub.p; P.tmp = tmp.p;
         P.cell_count = cell_count.p; P.cell_start = cell_start.p; P.cell_xyz = cell_xyz.p;
         P.cell_rank = cell_rank.p; P.cell_sys = cell_sys.p;
         P.work_count = work_count.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
@@ -1644,7 +1646,7 @@ struct mdpd_system {
         }
         xhold.alloc(cap); frc.alloc(cap); vend.alloc(cap);
         rho.alloc(cap); pr.alloc(cap); vir.alloc((size_t)6 * cap); phi[0].alloc(cap); phi[1].alloc(cap);
-        pcell.alloc(cap); pslot.alloc(cap); psub.alloc(cap); tmp.alloc(cap); key.alloc(2 * (size_t)cap);
+        pcell.alloc(cap); pslot.alloc(cap); psub.alloc(cap); tmp.alloc(cap);
         ncount.alloc(cap); ccount.alloc((size_t)MAXSPLIT * cap);
         nlist.alloc((size_t)cap * maxnbr);
         clist.alloc((size_t)cap * maxnbr);
@@ -1708,7 +1710,7 @@ struct mdpd_system {
     void rebuild()
     {
         PoolDev P = view();
-        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, stream), "rebuild"); });
+        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, false, stream), "rebuild"); });
         for (int attempt = 0;; ++attempt) {
             int ovf = read_field(offsetof(SysDev, overflow));
             if (!ovf) break;
@@ -1789,8 +1791,9 @@ struct mdpd_system {
     }
 
     // t: timestep this pass evaluates (observables sample it), -1 at setup
-    // and in a captured step, which takes the samples of `mask` instead
-    void force_pass(int mode, long long t = -1, uint32_t mask = 0)
+    // and in a captured step, which takes the samples of `mask` instead;
+    // commit: false when the next rebuild phase makes it
+    void force_pass(int mode, long long t = -1, uint32_t mask = 0, bool commit = true)
     {
         PoolDev P = view();
         const bool with_rho = pair_style == STYLE_MDPD && hsys.rho_bit;
@@ -1802,47 +1805,54 @@ struct mdpd_system {
         else if (mask) obs_launch(-1, mask, false);
         if ((mode == MODE_FUSED || mode == MODE_FUSED_OUT) && hsys.fix_arb)
             timed(PH_WALL, [&]() { hip_check(launch_aboundary(P, 0, stream), "aboundary"); });   // post_integrate
-        if (mode != MODE_SETUP)
+        if (mode != MODE_SETUP && commit)
             hip_check(launch_commit_step(P, mode == MODE_FINAL ? COMMIT_FINAL : COMMIT_DECIDE, split, true, stream), "commit");
     }
 
     // The rebuild phase of a step, launched every step: its kernels re-sort
     // and re-list the system only when the previous commit flagged it stale
     // (Neighbor::decide made on the device), otherwise they exit at once.
-    void rebuild_phase()
+    void rebuild_phase(bool commit = false)
     {
         PoolDev P = view();
-        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, stream), "rebuild"); });
+        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, commit, stream), "rebuild"); });
     }
 
     // the graph of one fused step whose observables take the samples of
     // `mask` (0: none); all are captured again after a change
-    hipGraphExec_t step_graph(uint32_t mask)
+    hipGraphExec_t step_graph(uint32_t mask, int steps = 1)
     {
         if (!graph_valid) {
             if (gexec) hip_check(hipGraphExecDestroy(gexec), "hipGraphExecDestroy");
             gexec = nullptr;
+            if (gsteps) hip_check(hipGraphExecDestroy(gsteps), "hipGraphExecDestroy");
+            gsteps = nullptr;
             for (auto &v : gobs) hip_check(hipGraphExecDestroy(v.second), "hipGraphExecDestroy");
             gobs.clear();
-            gexec = capture_step(0);
             graph_valid = true;
         }
+        if (steps > 1) return gsteps ? gsteps : gsteps = capture_steps(steps, 0);
+        if (!mask && !gexec) gexec = capture_steps(1, 0);
         if (!mask) return gexec;
         auto it = gobs.find(mask);
         if (it != gobs.end()) return it->second;
         for (auto &f : fixes)
             if (is_obs(f)) obs_state(f);           // histograms allocated outside the capture
-        return gobs[mask] = capture_step(mask);
+        return gobs[mask] = capture_steps(1, mask);
     }
 
-    // one fused step (rebuild phase, passes, commit) as a hipGraph
-    hipGraphExec_t capture_step(uint32_t mask)
+    // fused steps (rebuild phase, passes, commit) as a hipGraph; between steps
+    // a small system's commit is made by the next rebuild phase
+    hipGraphExec_t capture_steps(int steps, uint32_t mask)
     {
         hipGraph_t g = nullptr;
         hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try {
-            rebuild_phase();
-            force_pass(MODE_FUSED, -1, mask);
+            const bool fold = commit_in_rebuild(view());
+            for (int q = 0; q < steps; ++q) {
+                rebuild_phase(fold && q > 0);
+                force_pass(MODE_FUSED, -1, mask, !fold || q + 1 == steps);
+            }
         } catch (...) {
             (void)hipStreamEndCapture(stream, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -1926,8 +1936,15 @@ struct mdpd_system {
                 ++m;
             // step t+q replays the graph whose observables sample t+q; a step
             // that overflows skips the rest of the batch, samples included
-            for (long long q = 0; q < m; ++q)
-                hip_check(hipGraphLaunch(step_graph(obs.empty() ? 0 : obs_sample_mask(t + q)), stream), "hipGraphLaunch");
+            for (long long q = 0; q < m;) {
+                const uint32_t mask = obs.empty() ? 0 : obs_sample_mask(t + q);
+                int b = 1;                // GRAPH_STEPS steps without samples replay one graph
+                if (!mask)
+                    while (b < GRAPH_STEPS && q + b < m && (obs.empty() || !obs_sample_mask(t + q + b))) ++b;
+                if (b < GRAPH_STEPS) b = 1;
+                hip_check(hipGraphLaunch(step_graph(mask, b), stream), "hipGraphLaunch");
+                q += b;
+            }
             k = settle() - t0;
             if (k < 1 || k > nsteps) fail(MDPD_E_HIP, "device step counter out of range (%lld)", k + t0);
         }
