@@ -108,6 +108,41 @@ def test_sorted_order_over_scan_sizes(engine, orc, n, L):
     s.close()
 
 
+# within a graph of several steps the rebuild phase makes the commit of the
+# step before, launched by itself the commit is its own launch: the one-launch
+# sort, the one-launch scan, the chunked scan, wall passes, a pool's jobs
+@pytest.mark.parametrize("case", ["one", "liquid", "dpd", "walls", (10241, 12.0), (4000, 46.0)], ids=str)
+@pytest.mark.parametrize("neigh", ["every 1 delay 0 check yes", "every 3 delay 5 check yes", "every 2 delay 4 check no"])
+def test_graph_steps_equal_single_launches(engine, case, neigh):
+    def make():
+        s = CASES[case](engine) if isinstance(case, str) else _box(engine, *case)
+        s.command("neigh_modify " + neigh)
+        return s
+    steps = 27
+    got = []
+    for graph in (0, 1):
+        s = make()
+        s.tune("split", 2)
+        s.tune("graph", graph)
+        s.run(steps)
+        got.append([s.gather(k) for k in ("x", "v", "f", "image")] + [s.nbuild])
+        s.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+    for graph in (0, 1):
+        p = engine.Pool(float(1 << 29), 16)
+        p.tune("split", 2)
+        p.tune("graph", graph)
+        made = [make(), make()]
+        jobs = [p.submit(made[0], steps), p.submit(made[1], 5)]
+        p.run()
+        for k, want in zip(("x", "v", "f", "image"), got[0]):
+            np.testing.assert_array_equal(p.gather(jobs[0], k), want, err_msg=f"pool, graph {graph}: {k}")
+        p.close()
+        for s in made:
+            s.close()
+
+
 def test_jobs_harvested_together_equal_their_own_runs(engine):
     # two mDPD jobs and a DPD job end in the same pass, with a longer two-type
     # job between them (evaluated by the same launches only once it has ended)

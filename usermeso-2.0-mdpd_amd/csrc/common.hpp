@@ -128,7 +128,8 @@ struct SysDev {
     int sel;                     // buffer holding x, v (flips every step and at re-sort)
     int sela;                    // buffer holding tag, mask, origin, image (flips at re-sort)
     int stale;                   // neighbor list must be rebuilt before the next force pass
-    int stale_pending;           // set during a step by the displacement check
+    int moved;                   // a particle moved past skin/2 since the last build (a pass sets it, the commit clears it)
+    int due;                     // k_keys: this rebuild phase re-sorts the system
     int overflow;                // a neighbor row or cell exceeded its capacity
     int active;                  // 0: slot idle (batched / served engine)
     int steps_left;              // pooled engine: steps still to run
@@ -195,7 +196,6 @@ struct PoolDev {
     int *clist;          // per step: entries of nlist within the pair cutoff, same layout
     int *ccount;         // per particle
     int *wave_sys;       // system of each 64-particle wave
-    int *moved;          // per 64-particle tile: a particle moved past skin/2 this step
     int *status;         // pooled engine, per system: job << 3 | 1 stale | 2 done | 4 overflow
     int *cl;             // per particle slot, in cell-segment order: sub-bin key (re-sort scratch)
     int *wall_near;      // per particle: its neighbor row holds a wall particle (wall branch; set by
@@ -247,6 +247,13 @@ __host__ inline uint32_t premix_host(uint32_t v0, uint32_t v1, int rounds)
     return v0 ^ v1;
 }
 
+// step commit after a pass
+enum CommitKind : int {
+    COMMIT_FINAL = 0,    // end-of-run half-kick: flip the buffer only
+    COMMIT_PHASED = 2,   // pooled engine: per-system lifecycle + reneighbor decision
+    COMMIT_DECIDE = 3,   // plain engine: flip, step + 1, next seed, reneighbor decision
+};
+
 // Lane s of workgroup k computes the seed two steps on of system 64 k + s, for
 // the step's commit.  64 TEA rounds are a chain of ~700 dependent instructions,
 // 2.5 us of a commit that every step waits for, so spare workgroups of a
@@ -264,23 +271,60 @@ __device__ inline void next_seeds(const PoolDev &P, int k)
     if (d->active) d->seed_after = premix<64>(d->seed, (uint32_t)(d->step + 2));
 }
 
-// A step done: the buffer it wrote becomes current, the next step's seed.
-// seeded: a kernel of the step left the seed two steps on in seed_after.
-__device__ inline void commit_advance(SysDev *d, bool moved, bool seeded)
+// Neighbor::decide after one more step
+__device__ inline bool relist_due(const SysDev *d, int ago)
+{
+    return ago >= d->n_delay && ago % d->n_every == 0 && (!d->n_check || d->moved);
+}
+
+// A step done: the buffer it wrote becomes current, the next step's seed, the
+// reneighbor decision.  seeded: a kernel of the step left the seed two steps
+// on in seed_after.
+__device__ inline void commit_advance(SysDev *d, bool seeded)
 {
     d->sel ^= 1;
     d->step += 1;
     d->seed_next = seeded ? d->seed_after : premix<64>(d->seed, (uint32_t)(d->step + 1));
-    d->stale = moved ? 1 : 0;
+    const int ago = ++d->ago;
+    d->stale = relist_due(d, ago) ? 1 : 0;
+    d->moved = 0;
 }
 
-// the same with the reneighbor decision of Neighbor::decide
-__device__ inline void commit_decide(SysDev *d, bool moved, bool seeded)
+// The step commit of system s by one thread (k_commit_step has the rules).
+__device__ inline void commit_system(const PoolDev &P, int s, int kind, int split, bool seeded)
 {
-    commit_advance(d, false, seeded);
-    const int ago = ++d->ago;
-    const bool due = ago >= d->n_delay && ago % d->n_every == 0;
-    d->stale = due && (!d->n_check || moved) ? 1 : 0;
+    SysDev *d = P.sys + s;
+    if (!d->active) return;
+    if (d->overflow) {
+        // skipped by the passes: no state change until the rows are regrown
+        if (kind == COMMIT_PHASED) P.status[s] = (d->job << 3) | (d->stale ? 1 : 0) | 4;
+        return;
+    }
+    if (kind == COMMIT_PHASED) {
+        d->split_last = split;
+        if (d->phase == PH_LAST) {
+            d->sel ^= 1;
+            d->phase = PH_DONE;
+            d->active = 0;
+        } else {
+            commit_advance(d, seeded);
+            d->steps_left -= 1;
+            d->phase = d->steps_left <= 0 ? PH_LAST : PH_RUN;
+        }
+        P.status[s] = (d->job << 3) | (d->stale ? 1 : 0) | (d->phase == PH_DONE ? 2 : 0);
+    } else if (kind == COMMIT_DECIDE) {
+        commit_advance(d, seeded);
+    } else {
+        d->sel ^= 1;
+    }
+}
+
+// whether that commit is going to flag the system stale (no commit: whether it is)
+__device__ inline bool due_after(const SysDev *d, int kind)
+{
+    if (!d->active) return false;
+    if (kind == COMMIT_FINAL || d->overflow) return d->stale != 0;
+    return !(kind == COMMIT_PHASED && d->phase == PH_LAST) && relist_due(d, d->ago + 1);
 }
 
 static inline int seed_grid(const PoolDev &P) { return xcd_grid((P.nsys + WAVE - 1) / WAVE); }

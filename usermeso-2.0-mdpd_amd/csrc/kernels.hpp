@@ -14,19 +14,10 @@ enum ForceMode : int {
     MODE_HARVEST = 5,    // pooled engine, finished system: f, e, virial of its last pass
 };
 
-// step commit after a pass (k_commit_step)
-enum CommitKind : int {
-    COMMIT_FINAL = 0,    // end-of-run half-kick: flip the buffer only
-    COMMIT_ADVANCE = 1,  // flip, step + 1, next seed; stale = a particle moved past skin/2
-    COMMIT_PHASED = 2,   // pooled engine: per-system lifecycle + reneighbor decision
-    COMMIT_DECIDE = 3,   // plain engine: COMMIT_ADVANCE with the reneighbor decision
-};
-
 // rebuild phase: wrap, keys, sort, gather, neighbor rows, commit (stale systems only)
-// split: of the pass that follows; commit: the commit of the pass before
-// (COMMIT_DECIDE, after_pass) is made first, for the systems whose rebuild can
-hipError_t launch_rebuild(const PoolDev &P, int split, bool commit, hipStream_t st);
-bool commit_in_rebuild(const PoolDev &P);
+// split: of the pass that follows; commit: the commit that the pass before,
+// at the same split, has left to this phase (its CommitKind after_pass), or 0
+hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t st);
 hipError_t launch_nlist_only(const PoolDev &P, hipStream_t st);
 // neighbor rows of every sorted active system rebuilt in place (row width grew)
 hipError_t launch_relist(const PoolDev &P, hipStream_t st);
@@ -38,7 +29,7 @@ hipError_t launch_sort_keys(const PoolDev &P, unsigned long long *out, hipStream
 // first pass of a step: density (mDPD with the density fix) and compact rows
 hipError_t launch_first(const PoolDev &P, bool with_rho, int split, hipStream_t st);
 hipError_t launch_initial(const PoolDev &P, hipStream_t st);
-// after launch_initial / a fused force pass (advance) or a final pass (!advance)
+// after launch_initial or a force pass
 // kind: CommitKind; split = waves per tile of the pass; after_pass: a rebuild
 // phase and a first pass of that split have run since the last commit
 hipError_t launch_commit_step(const PoolDev &P, int kind, int split, bool after_pass, hipStream_t st);

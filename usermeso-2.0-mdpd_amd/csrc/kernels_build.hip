@@ -73,28 +73,33 @@ __device__ inline uint32_t particle_bins(const SysDev *d, const float4 &p, int b
 // --------------------------------------------------------------------------
 // K1: wrap into the box (Domain::pbc in FP32), reference sort key, sub-cell
 // slot (cell slot * SUBCELLS + top bits of the sub-bin key), arrival rank
-// inside the sub-cell.
+// inside the sub-cell.  `commit`: the commit of the pass before is still to
+// come (the scan makes it, when nobody here reads its fields any more), so
+// the decision it is going to make and the buffer it makes current are worked
+// out here, and the decision goes to d->due for the scan's workgroups.
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_keys(PoolDev P)
+__global__ void __launch_bounds__(256) k_keys(PoolDev P, int commit)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         P.work_count[0] = 0;                              // this rebuild's worklist starts empty
         // one system: the row build's waves read this word, not the flag that
         // their commit clears
-        if (P.one) P.work_count[1] = P.sys->active && P.sys->stale ? 1 : 0;
+        if (P.one) P.work_count[1] = due_after(P.sys, commit) ? 1 : 0;
     }
     if (i >= P.nact) return;
     const int s = P.one ? 0 : P.wave_sys[i >> 6];
     if (s < 0) return;
     SysDev *d = P.sys + s;
-    if (!d->active || !d->stale) return;
+    const bool due = due_after(d, commit);
+    if (i == d->part_base) d->due = due ? 1 : 0;
+    if (!due) return;
     // the wave stays whole (the slot's run below is found across lanes);
     // lanes past the system's last particle only take part in that
     const bool valid = i < d->part_base + d->n;
     int gc = -1;
     if (valid) {
-    const int cur = d->sel, cura = d->sela;
+    const int cur = d->sel ^ (commit && !d->overflow ? 1 : 0), cura = d->sela;
     float4 p = P.pos[cur][i];
     int img = P.image[cura][i];
     wrap_particle(d, p, img);
@@ -160,10 +165,13 @@ __device__ inline int block_excl_scan(int x, int *wsum, int *total)
     return before + incl - x;
 }
 
-__global__ void __launch_bounds__(SCAN_BLK) k_scan_sums(PoolDev P)
+__global__ void __launch_bounds__(SCAN_BLK) k_scan_sums(PoolDev P, int commit, int split, int seeded)
 {
     const SysDev *d = P.sys + blockIdx.y;
-    if (!d->active || !d->stale) return;
+    // a finished system is not due; the commit ends no system that is
+    const bool due = d->active && d->due;
+    if (commit && blockIdx.x == 0 && threadIdx.x == 0) commit_system(P, blockIdx.y, commit, split, seeded);
+    if (!due) return;
     __shared__ int wsum[SCAN_BLK / 64];
     const int nc = d->ncell * SUBCELLS, base = d->cell_base * SUBCELLS;
     for (int c0 = blockIdx.x * SCAN_CH; c0 < nc; c0 += gridDim.x * SCAN_CH) {
@@ -302,10 +310,12 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
 constexpr int SCAN1_BLK = 1024, SCAN1_CH = SCAN1_BLK * 4;
 constexpr int SCAN1_MAX = 40;          // chunks: past that the last workgroup's reads (10 rounds) cost the launches saved
 
-__global__ void __launch_bounds__(SCAN1_BLK) k_scan_one(PoolDev P)
+__global__ void __launch_bounds__(SCAN1_BLK) k_scan_one(PoolDev P, int commit, int split, int seeded)
 {
     const SysDev *d = P.sys;
-    if (!d->active || !d->stale) return;
+    const bool due = P.work_count[1] != 0;
+    if (commit && blockIdx.x == 0 && threadIdx.x == 0) commit_system(P, 0, commit, split, seeded);
+    if (!due) return;
     __shared__ int s_before[SCAN1_BLK / WAVE], s_own[SCAN1_BLK / WAVE];
     const int nc = d->ncell * SUBCELLS;                    // a multiple of four
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -438,14 +448,9 @@ __global__ void __launch_bounds__(SORT1_BLK) k_sort_one(PoolDev P, int commit, i
     __shared__ int s_wave[SORT1_BLK / WAVE], s_now[3];      // stale, sel, sela after the commit
     SysDev *d = P.sys;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const bool skip = !d->active || (commit && d->overflow);
-    if (commit && !skip) {
-        const int nt = d->npad / WAVE;
-        const int any = __syncthreads_or(t < nt ? P.moved[t] : 0);
-        if (t == 0) commit_decide(d, any != 0, seeded);
-    }
     if (t == 0) {
-        s_now[0] = skip ? 0 : d->stale;
+        if (commit) commit_system(P, 0, commit, 0, seeded);
+        s_now[0] = d->active && d->stale;
         s_now[1] = d->sel;
         s_now[2] = d->sela;
     }
@@ -838,44 +843,38 @@ static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t s
         hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(P.ncact))), dim3(WAVE), 0, st, P);
 }
 
-bool commit_in_rebuild(const PoolDev &P)
-{
-    return P.one && P.nact <= SORT1_N && (P.ncellslots - 1) * SUBCELLS <= SORT1_SUB;
-}
-
-hipError_t launch_rebuild(const PoolDev &P, int split, bool commit, hipStream_t st)
+hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
-    const bool small = commit_in_rebuild(P);
-    if (commit && !small) return hipErrorInvalidValue;
-    if (small) {
-        // such a system's first pass computes the seeds (at most 160 tiles)
-        const int c = commit ? 1 : 0;
+    if (commit != COMMIT_FINAL && commit != COMMIT_PHASED && commit != COMMIT_DECIDE) return hipErrorInvalidValue;
+    const bool fseed = first_seeds(split, P.nact / WAVE);
+    const int seeded = P.one || fseed ? 1 : 0;
+    if (P.one && P.nact <= SORT1_N && (P.ncellslots - 1) * SUBCELLS <= SORT1_SUB) {
         if (P.nact <= SORT1_BLK)
-            hipLaunchKernelGGL((k_sort_one<1>), dim3(1), dim3(SORT1_BLK), 0, st, P, c, 1);
+            hipLaunchKernelGGL((k_sort_one<1>), dim3(1), dim3(SORT1_BLK), 0, st, P, commit, seeded);
         else
-            hipLaunchKernelGGL((k_sort_one<SORT1_PER>), dim3(1), dim3(SORT1_BLK), 0, st, P, c, 1);
-        launch_nlist(P, 0, P.one && !first_seeds(split, P.nact / WAVE), st);
+            hipLaunchKernelGGL((k_sort_one<SORT1_PER>), dim3(1), dim3(SORT1_BLK), 0, st, P, commit, seeded);
+        launch_nlist(P, 0, !fseed, st);
         return hipGetLastError();
     }
     const dim3 g(nblk(P.nact, 256)), b(256);
-    hipLaunchKernelGGL(k_keys, g, b, 0, st, P);
+    hipLaunchKernelGGL(k_keys, g, b, 0, st, P, commit);
     const long long nsub = P.maxsub > 0 ? (long long)P.maxsub : (long long)P.ncellslots * SUBCELLS;
     const bool scan_one = P.one && nblk((int)nsub, SCAN1_CH) <= SCAN1_MAX;
     if (scan_one) {
-        hipLaunchKernelGGL(k_scan_one, dim3(nblk((int)nsub, SCAN1_CH)), dim3(SCAN1_BLK), 0, st, P);
+        hipLaunchKernelGGL(k_scan_one, dim3(nblk((int)nsub, SCAN1_CH)), dim3(SCAN1_BLK), 0, st, P, commit, split, seeded);
     } else {
         // workgroups per system for the chunked scan: as many as the largest
         // system has chunks, up to 64 (smaller systems' extra workgroups exit)
         const int nch = (int)((nsub + SCAN_CH - 1) / SCAN_CH);
         const int gs = std::max(1, std::min(64, nch));
-        hipLaunchKernelGGL(k_scan_sums, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
+        hipLaunchKernelGGL(k_scan_sums, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P, commit, split, seeded);
         hipLaunchKernelGGL(k_scan_chunks, dim3(P.nsys), dim3(SCAN_BLK), 0, st, P);
         hipLaunchKernelGGL(k_scan_apply, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
     }
     hipLaunchKernelGGL(k_scatter, g, b, 0, st, P, scan_one ? 1 : 0);
     hipLaunchKernelGGL(k_sortgather, g, b, 0, st, P);
-    launch_nlist(P, 0, P.one && !first_seeds(split, P.nact / WAVE), st);
+    launch_nlist(P, 0, P.one && !fseed, st);
     return hipGetLastError();
 }
 

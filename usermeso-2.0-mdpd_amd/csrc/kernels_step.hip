@@ -27,18 +27,12 @@ namespace mdpd {
 
 constexpr int BLK = 256;
 
-// Per-tile "a particle moved past skin/2" flags: each workgroup ORs its lanes
-// in LDS and stores one word per 64-particle tile it covers (plain stores, no
-// atomics: same-address device-scope atomics serialize across the XCDs and
-// cost ~50 ns each).  k_commit_step reduces them per system after the pass.
-__device__ inline void tile_flags(int *moved, int tile0, int ntile, int flag)
+// A wave that holds a particle past skin/2 says so in its system's flag: a
+// plain store, the same from every wave (same-address device-scope atomics
+// serialize across the XCDs and cost ~50 ns each), and none on most steps.
+__device__ inline void flag_moved(SysDev *d, bool moved)
 {
-    __shared__ int s_or[4];
-    if (threadIdx.x < 4) s_or[threadIdx.x] = 0;
-    __syncthreads();
-    if (flag) s_or[(threadIdx.x >> 6) % ntile] = 1;
-    __syncthreads();
-    if (threadIdx.x < ntile) moved[tile0 + threadIdx.x] = s_or[threadIdx.x];
+    if (__builtin_amdgcn_ballot_w64(moved) != 0 && (threadIdx.x & 63) == 0) d->moved = 1;
 }
 
 // a - (b + s L) with a single rounding.  Adding s L to the neighbor's
@@ -391,7 +385,7 @@ __global__ void __launch_bounds__(BLK) k_initial(PoolDev P, int nlogical)
         const float ex = p.x - h.x, ey = p.y - h.y, ez = p.z - h.z;
         moved = ex * ex + ey * ey + ez * ez > d->trig2;
     }
-    tile_flags(P.moved, lb * (BLK / WAVE), BLK / WAVE, moved);
+    if (!d->fix_arb) flag_moved(d, moved);          // else k_aboundary does, from the final positions
 }
 
 // --------------------------------------------------------------------------
@@ -756,9 +750,10 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_force(PoolDev P, int tile0, in
             for (int q = 0; q < SPLIT - 1; ++q)
                 for (int k = 0; k < NA; ++k) a.v[k] += s_acc[q][k][lane];
     }
+    if (w > 0) return;
     int moved = 0;
-    if (w == 0 && valid) moved = finish_particle<MODE, EV, STEP, false>(P, d, i, cur, pi, vi, ti, mk, a, 0u);
-    if (MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) tile_flags(P.moved, tile, 1, moved);
+    if (valid) moved = finish_particle<MODE, EV, STEP, false>(P, d, i, cur, pi, vi, ti, mk, a, 0u);
+    if ((MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) && !d->fix_arb) flag_moved(d, moved);
 }
 
 // --------------------------------------------------------------------------
@@ -941,10 +936,7 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
     int moved = 0;
     if (valid)
         moved = finish_particle<MODE, EV, STEP, STYLE == STYLE_MDPD>(P, d, i, cur, pi, vi, ti, mk, a, s_sig[lane]);
-    if (MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) {
-        const uint64_t any = __builtin_amdgcn_ballot_w64(moved != 0);
-        if (lane == 0) P.moved[tile] = any != 0 ? 1 : 0;
-    }
+    if ((MODE == MODE_FUSED || MODE == MODE_FUSED_OUT || MODE == MODE_PHASED) && !d->fix_arb) flag_moved(d, moved);
 }
 
 // --------------------------------------------------------------------------
@@ -954,7 +946,7 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
 // each mobile particle from the wall particles within cut_phi (every entry of
 // its neighbor row, positions after the drift), bounce-back when
 // phi_i > phi_c (v <- -v + 2 max(0, v.n) n, x <- x - v dtf/m + dt v_new),
-// then the tile's displacement flag from the final positions.  Works on the
+// then the system's displacement flag from the final positions.  Works on the
 // buffer the pass just wrote (sel ^ 1, before the step commit); one wave per
 // 64-particle tile.  `pooled`: apply only to systems whose pass integrated.
 // --------------------------------------------------------------------------
@@ -1056,77 +1048,27 @@ __global__ void __launch_bounds__(WAVE) k_aboundary(PoolDev P, int ntiles, int p
         const float ex = p.x - h.x, ey = p.y - h.y, ez = p.z - h.z;
         moved = ex * ex + ey * ey + ez * ez > d->trig2;
     }
-    const uint64_t any = __ballot(moved);
-    if (lane == 0) P.moved[tile] = any != 0 ? 1 : 0;
+    flag_moved(P.sys + s, moved);
 }
 
 // --------------------------------------------------------------------------
-// Step commit, one workgroup per system, after a pass that wrote the other
-// buffer: ADVANCE (initial kick or fused step) flips the buffer, advances the
-// step, precomputes the next TEA seed and ORs the tiles' moved flags into
-// `stale`; FINAL (end-of-run half-kick) only flips the buffer.  DECIDE (plain
-// engine) and PHASED (pooled engine) make the reneighbor decision of
-// Neighbor::decide (src/neighbor.cpp:1216-1290) on the device: after `ago`
-// steps since the last build, rebuild when ago >= delay, ago % every == 0 and
-// (no check, or a particle moved more than skin/2 since the last build);
-// PHASED also follows each system's lifecycle.  A system whose rows
-// overflowed was skipped by the pass and is not advanced.
+// Step commit, one thread per system, after a pass that wrote the other
+// buffer: FINAL (end-of-run half-kick) only flips the buffer; DECIDE (plain
+// engine) and PHASED (pooled engine) also advance the step and the seed and
+// make the reneighbor decision of Neighbor::decide (src/neighbor.cpp:
+// 1216-1290) on the device: after `ago` steps since the last build, rebuild
+// when ago >= delay, ago % every == 0 and (no check, or a particle moved more
+// than skin/2 since the last build); PHASED also follows each system's
+// lifecycle.  A system whose rows overflowed was skipped by the pass and is
+// not advanced.  Between the steps of one graph the next rebuild phase makes
+// the commit instead (launch_rebuild): a launch of one workgroup costs every
+// step 2 to 3 us whatever it does (97,000 particles: a step 94 -> 91.4 us,
+// 40,000 particles 59.4 -> 57.7).
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_commit_step(PoolDev P, int advance, int split, int seeded)
+__global__ void __launch_bounds__(WAVE) k_commit_step(PoolDev P, int kind, int split, int seeded)
 {
-    __shared__ int s_any;
-    SysDev *d = P.sys + blockIdx.x;
-    if (!d->active) return;
-    if (d->overflow) {
-        // skipped by the passes: no state change until the rows are regrown
-        if (advance == COMMIT_PHASED && threadIdx.x == 0)
-            P.status[blockIdx.x] = (d->job << 3) | (d->stale ? 1 : 0) | 4;
-        return;
-    }
-    if (threadIdx.x == 0) s_any = 0;
-    __syncthreads();
-    if (advance) {
-        const int t0 = d->part_base / WAVE, nt = d->npad / WAVE;
-        int any = 0;
-        // four tile flags in flight per thread, 1,024 threads: a 200k-particle
-        // system's ~3,000 tiles in one round (0.4% on the 193,600-particle slab)
-        for (int t = threadIdx.x; t < nt; t += 4 * (int)blockDim.x) {
-            int f[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int k = t + u * (int)blockDim.x;
-                f[u] = k < nt ? P.moved[t0 + k] : 0;
-            }
-            any |= f[0] | f[1] | f[2] | f[3];
-        }
-        if (any) s_any = 1;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        if (advance == COMMIT_PHASED) {
-            // pooled engine: per-system lifecycle
-            d->split_last = split;
-            if (d->phase == PH_LAST) {
-                d->sel ^= 1;
-                d->phase = PH_DONE;
-                d->active = 0;
-            } else {
-                commit_advance(d, false, seeded);
-                const int ago = ++d->ago;
-                const bool due = ago >= d->n_delay && ago % d->n_every == 0;
-                d->stale = due && (!d->n_check || s_any != 0) ? 1 : 0;
-                d->steps_left -= 1;
-                d->phase = d->steps_left <= 0 ? PH_LAST : PH_RUN;
-            }
-            P.status[blockIdx.x] = (d->job << 3) | (d->stale ? 1 : 0) | (d->phase == PH_DONE ? 2 : 0);
-        } else if (advance == COMMIT_DECIDE) {
-            commit_decide(d, s_any != 0, seeded);
-        } else if (advance == COMMIT_ADVANCE) {
-            commit_advance(d, s_any != 0, seeded);
-        } else {
-            d->sel ^= 1;
-        }
-    }
+    const int s = blockIdx.x * WAVE + threadIdx.x;
+    if (s < P.nsys) commit_system(P, s, kind, split, seeded);
 }
 
 // --------------------------------------------------------------------------
@@ -1327,7 +1269,7 @@ hipError_t launch_commit_step(const PoolDev &P, int kind, int split, bool after_
 {
     if (P.nsys == 0) return hipSuccess;
     const int seeded = after_pass && (P.one || first_seeds(split, P.nact / WAVE)) ? 1 : 0;
-    hipLaunchKernelGGL(k_commit_step, dim3(P.nsys), dim3(1024), 0, st, P, kind, split, seeded);
+    hipLaunchKernelGGL(k_commit_step, dim3((P.nsys + WAVE - 1) / WAVE), dim3(WAVE), 0, st, P, kind, split, seeded);
     return hipGetLastError();
 }
 

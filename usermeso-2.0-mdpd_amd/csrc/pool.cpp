@@ -221,7 +221,7 @@ struct mdpd_pool {
     DevBuf<int> pcell, pslot, psub, tmp, cell_count, cell_start, cell_xyz, cell_rank, cell_sys, work_count;
     DevBuf<int4> cell_work;
     DevBuf<int2> cell_lse;
-    DevBuf<int> nlist, ncount, clist, ccount, wave_sys, moved, status, cl, wall_near;
+    DevBuf<int> nlist, ncount, clist, ccount, wave_sys, status, cl, wall_near;
     DevBuf<SysDev> dsys;
     DevBuf<unsigned> obs_arena;           // per descriptor slot: POOL_RDF histograms of OBS_MAXBIN + 1
                                           // words, then POOL_DENS_WORDS of density windows
@@ -350,7 +350,7 @@ struct mdpd_pool {
         P.cell_rank = cell_rank.p; P.cell_sys = cell_sys.p;
         P.work_count = work_count.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
         P.nlist = nlist.p; P.ncount = ncount.p; P.wave_sys = wave_sys.p;
-        P.clist = clist.p; P.ccount = ccount.p; P.moved = moved.p; P.status = status.p;
+        P.clist = clist.p; P.ccount = ccount.p; P.status = status.p;
         P.cl = cl.p; P.wall_near = wall_near.p;
         P.sys = dsys.p; P.coef = coef.p; P.minv = minv.p; P.mass = mmass.p;
         P.cap = cap; P.nact = nact; P.ncellslots = nslots; P.ncact = ncact; P.nsys = nsys_act; P.maxsub = maxsub;
@@ -520,7 +520,7 @@ struct mdpd_pool {
         ncount.alloc(cap); ccount.alloc((size_t)MAXSPLIT * cap);
         nlist.alloc((size_t)cap * maxnbr);
         clist.alloc((size_t)cap * maxnbr);
-        wave_sys.alloc(cap / WAVE); moved.alloc(cap / WAVE); status.alloc(max_sys);
+        wave_sys.alloc(cap / WAVE); status.alloc(max_sys);
         cl.alloc(cap); wall_near.alloc(cap);
         cell_count.alloc((size_t)nslots * SUBCELLS); cell_start.alloc((size_t)nslots * SUBCELLS);
         cell_xyz.alloc(nslots);
@@ -788,8 +788,10 @@ struct mdpd_pool {
         return e;
     }
 
-    // one pass; with `ev`, events are recorded between its phases
-    void launch_pass(int sp, PassEvents *ev = nullptr)
+    // one pass; with `ev`, events are recorded between its phases.  pending:
+    // the pass before left its commit to this one's rebuild phase; commit:
+    // this one makes its own
+    void launch_pass(int sp, PassEvents *ev = nullptr, bool pending = false, bool commit = true)
     {
         PoolDev P = view();
         splits_used |= sp;
@@ -797,7 +799,7 @@ struct mdpd_pool {
             if (ev) hip_check(hipEventRecord(ev->e[k], stream), "hipEventRecord");
         };
         mark(PP_REBUILD);
-        hip_check(launch_rebuild(P, sp, false, stream), "rebuild");
+        hip_check(launch_rebuild(P, sp, pending ? COMMIT_PHASED : 0, stream), "rebuild");
         mark(PP_FIRST);
         hip_check(launch_first(P, with_rho, sp, stream), "first pass");
         mark(PP_FORCE);
@@ -805,7 +807,7 @@ struct mdpd_pool {
         if (with_arb) hip_check(launch_aboundary(P, 1, stream), "aboundary");
         if (with_obs) hip_check(launch_obs_pool(P, stream), "observables");
         mark(PP_COMMIT);
-        hip_check(launch_commit_step(P, COMMIT_PHASED, sp, true, stream), "commit step");
+        if (commit) hip_check(launch_commit_step(P, COMMIT_PHASED, sp, true, stream), "commit step");
         mark(PP_COUNT);
     }
 
@@ -835,7 +837,7 @@ struct mdpd_pool {
         hipGraph_t g = nullptr;
         hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try {
-            for (int k = 0; k < npass; ++k) launch_pass(split);
+            for (int k = 0; k < npass; ++k) launch_pass(split, nullptr, k > 0, k + 1 == npass);
         } catch (...) {
             (void)hipStreamEndCapture(stream, &g);
             if (g) (void)hipGraphDestroy(g);

@@ -224,7 +224,7 @@ struct mdpd_system {
     DevBuf<int> pcell, pslot, psub, tmp, cell_count, cell_start, cell_xyz, cell_rank, cell_sys, work_count;
     DevBuf<int4> cell_work;
     DevBuf<int2> cell_lse;
-    DevBuf<int> nlist, ncount, clist, ccount, wave_sys, moved, status, cl, wall_near;
+    DevBuf<int> nlist, ncount, clist, ccount, wave_sys, status, cl, wall_near;
     DevBuf<SysDev> dsys;
     int *pinned = nullptr;            // host-visible readback of flags
     static constexpr size_t STAGE_WORDS = 1 << 17;
@@ -1456,7 +1456,7 @@ struct mdpd_system {
         P.cell_rank = cell_rank.p; P.cell_sys = cell_sys.p;
         P.work_count = work_count.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
         P.nlist = nlist.p; P.ncount = ncount.p; P.wave_sys = wave_sys.p;
-        P.clist = clist.p; P.ccount = ccount.p; P.moved = moved.p; P.status = status.p;
+        P.clist = clist.p; P.ccount = ccount.p; P.status = status.p;
         P.cl = cl.p; P.wall_near = wall_near.p;
         P.sys = dsys.p; P.coef = coef.p; P.minv = minv.p; P.mass = mmass.p;
         P.cap = cap; P.nact = cap; P.ncellslots = nslots; P.ncact = nslots; P.nsys = 1; P.maxsub = 0; P.one = 1;
@@ -1650,7 +1650,7 @@ struct mdpd_system {
         ncount.alloc(cap); ccount.alloc((size_t)MAXSPLIT * cap);
         nlist.alloc((size_t)cap * maxnbr);
         clist.alloc((size_t)cap * maxnbr);
-        wave_sys.alloc(cap / WAVE); moved.alloc(cap / WAVE); status.alloc(1);
+        wave_sys.alloc(cap / WAVE); status.alloc(1);
         cl.alloc(cap); wall_near.alloc(cap);
         cell_count.alloc((size_t)nslots * SUBCELLS); cell_start.alloc((size_t)nslots * SUBCELLS);
         cell_xyz.alloc(nslots);
@@ -1710,7 +1710,7 @@ struct mdpd_system {
     void rebuild()
     {
         PoolDev P = view();
-        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, false, stream), "rebuild"); });
+        timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, 0, stream), "rebuild"); });
         for (int attempt = 0;; ++attempt) {
             int ovf = read_field(offsetof(SysDev, overflow));
             if (!ovf) break;
@@ -1812,7 +1812,7 @@ struct mdpd_system {
     // The rebuild phase of a step, launched every step: its kernels re-sort
     // and re-list the system only when the previous commit flagged it stale
     // (Neighbor::decide made on the device), otherwise they exit at once.
-    void rebuild_phase(bool commit = false)
+    void rebuild_phase(int commit = 0)
     {
         PoolDev P = view();
         timed(PH_REBUILD, [&]() { hip_check(launch_rebuild(P, split, commit, stream), "rebuild"); });
@@ -1842,16 +1842,15 @@ struct mdpd_system {
     }
 
     // fused steps (rebuild phase, passes, commit) as a hipGraph; between steps
-    // a small system's commit is made by the next rebuild phase
+    // the commit is made by the next rebuild phase
     hipGraphExec_t capture_steps(int steps, uint32_t mask)
     {
         hipGraph_t g = nullptr;
         hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try {
-            const bool fold = commit_in_rebuild(view());
             for (int q = 0; q < steps; ++q) {
-                rebuild_phase(fold && q > 0);
-                force_pass(MODE_FUSED, -1, mask, !fold || q + 1 == steps);
+                rebuild_phase(q > 0 ? COMMIT_DECIDE : 0);
+                force_pass(MODE_FUSED, -1, mask, q + 1 == steps);
             }
         } catch (...) {
             (void)hipStreamEndCapture(stream, &g);
