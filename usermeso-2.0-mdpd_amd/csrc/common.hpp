@@ -189,6 +189,7 @@ struct PoolDev {
     int *cell_sys;       // system of each cell slot
     int4 *cell_work;     // pools: the cells holding particles of the systems re-sorted this pass, as
                          // (system, packed coordinates, first particle, end) (k_scan_apply appends)
+    int *chunk_sum;      // per cell slot: a system's sub-cell chunk totals from its first slot on (k_scan_sums)
     int *work_count;     // [0]: entries of cell_work (k_keys clears it); [1]: one system: list its rows (k_keys)
     int2 *cell_lse;      // pools: particle range [start, end) of each cell by linear cell id (cell_base + lin)
     int *nlist;         // (cap/64) tiles * maxnbr * 64

@@ -135,13 +135,14 @@ __global__ void __launch_bounds__(256) k_keys(PoolDev P, int commit)
 // --------------------------------------------------------------------------
 // K2: exclusive scan of sub-cell counts in (cell Morton rank, sub-cell)
 // order, per system, from its first particle slot; clears the counts for the
-// next rebuild.  Chunks of SCAN_CH counts, three launches without waits:
-//   k_scan_sums   per chunk: its total, parked in the chunk's first start slot
-//   k_scan_chunks per system: exclusive scan of the chunk totals in place,
-//                 and the end entry
-//   k_scan_apply  per chunk: exclusive scan of its counts from its offset;
-//                 in a pool also each cell's particle range by linear cell
-//                 id and the worklist of occupied cells for the row build
+// next rebuild.  Chunks of SCAN_CH counts, two launches without waits:
+//   k_scan_sums   per chunk: its total, to chunk_sum[first cell slot + chunk]
+//   k_scan_apply  per chunk: exclusive scan of its counts from the sum of the
+//                 totals before it (each workgroup adds them up itself: one
+//                 load per thread up to a million sub-cells, where a launch
+//                 between the two cost a pass 3 us and more); in a pool also
+//                 each cell's particle range by linear cell id and the
+//                 worklist of occupied cells for the row build
 // Grid (G, nsys): workgroup g of a system takes chunks g, g + G, ...
 // --------------------------------------------------------------------------
 constexpr int SCAN_BLK = 256, SCAN_PER = 16, SCAN_CH = SCAN_BLK * SCAN_PER;
@@ -185,27 +186,8 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_sums(PoolDev P, int commit, i
         }
         int total;
         block_excl_scan(sum, wsum, &total);
-        if (threadIdx.x == 0) P.cell_start[base + c0] = total;
+        if (threadIdx.x == 0) P.chunk_sum[d->cell_base + c0 / SCAN_CH] = total;
     }
-}
-
-__global__ void __launch_bounds__(SCAN_BLK) k_scan_chunks(PoolDev P)
-{
-    const SysDev *d = P.sys + blockIdx.x;
-    if (!d->active || !d->stale) return;
-    __shared__ int wsum[SCAN_BLK / 64];
-    const int nc = d->ncell * SUBCELLS, base = d->cell_base * SUBCELLS;
-    const int nch = (nc + SCAN_CH - 1) / SCAN_CH;
-    int carry = d->part_base;
-    for (int k0 = 0; k0 < nch; k0 += SCAN_BLK) {
-        const int k = k0 + threadIdx.x;
-        const int v = k < nch ? P.cell_start[base + k * SCAN_CH] : 0;
-        int total;
-        const int ex = block_excl_scan(v, wsum, &total);
-        if (k < nch) P.cell_start[base + k * SCAN_CH] = carry + ex;
-        carry += total;
-    }
-    if (threadIdx.x == 0) P.cell_start[base + nc] = d->part_base + d->n;
 }
 
 __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
@@ -218,7 +200,8 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
     const int nc = d->ncell * SUBCELLS, base = d->cell_base * SUBCELLS;
     const int t = threadIdx.x;
     for (int c0 = blockIdx.x * SCAN_CH; c0 < nc; c0 += gridDim.x * SCAN_CH) {
-        const int off = P.cell_start[base + c0];     // the chunk's offset
+        int before = 0;
+        for (int k = t; k < c0 / SCAN_CH; k += SCAN_BLK) before += P.chunk_sum[d->cell_base + k];
         // coalesced load into LDS (counts cleared), SCAN_PER consecutive
         // counts per thread, workgroup scan, coalesced store
 #pragma unroll
@@ -239,7 +222,10 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
         constexpr int CPT = SCAN_PER / SUBCELLS;                 // cells per thread
         int cst[CPT];                                            // first particle of each
         int total;
-        int run = off + block_excl_scan(sum, wsum, &total);
+        int run = d->part_base + block_excl_scan(sum, wsum, &total);
+        block_excl_scan(before, wsum, &total);
+        run += total;
+        if (t == 0 && c0 + SCAN_CH >= nc) P.cell_start[base + nc] = d->part_base + d->n;
 #pragma unroll
         for (int k = 0; k < SCAN_PER; ++k) {
             if (k % SUBCELLS == 0) cst[k / SUBCELLS] = run;
@@ -303,8 +289,8 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
 // --------------------------------------------------------------------------
 // The same scan for one system in one launch: workgroup g adds up all the
 // counts before its chunk itself, which costs it reads (two rounds of loads
-// for the 54,000 sub-cells of a 97,000-particle slab) where k_scan_sums and
-// k_scan_chunks cost a launch each, 1.6 us idle and 4.7 us working.  Other
+// for the 54,000 sub-cells of a 97,000-particle slab) where k_scan_sums costs
+// a launch, 1.6 us idle and 4.7 us working.  Other
 // workgroups may still read a chunk's counts, so k_scatter clears them.
 // --------------------------------------------------------------------------
 constexpr int SCAN1_BLK = 1024, SCAN1_CH = SCAN1_BLK * 4;
@@ -579,9 +565,12 @@ __global__ void __launch_bounds__(SORT1_BLK) k_sort_one(PoolDev P, int commit, i
 constexpr int NL_ITER = 7;             // candidate tiles per batch: 448 candidates (a cell's stencil averages ~370)
 constexpr int NL_WAVES = 8;            // waves per SIMD of the worklist walk (63 VGPRs; measured
                                        // faster than seven, which needs no SGPR spills to VGPR lanes)
-constexpr int NL_GRID = 65536;         // its waves (measured against 7,168 and 16,384: more
-                                       // waves balance uneven cells better; 65,536 cost 14 us
-                                       // to dispatch when no cell is listed)
+// its waves: one per NL_PART particle slots, about what the cells of a liquid
+// hold (waves without a cell cost their dispatch, 14 us for 65,536, 3.8 us for
+// the 13,000 of 24 droplets, 8 and 32 slots measured the same within 1%;
+// fewer waves than cells balance uneven cells worse), at most NL_GRID
+// (measured against 7,168 and 16,384 at 256 droplets)
+constexpr int NL_PART = 16, NL_GRID = 65536;
 
 // LISTED: e = (system, packed coordinates, first particle, end) of a listed
 // cell, whose neighbor cells' ranges come from the linear table; otherwise
@@ -840,7 +829,7 @@ static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t s
         hipLaunchKernelGGL(k_nlist, dim3(xcd_grid(P.ncact << lparts) + (seeds ? seed_grid(P) : 0)), dim3(WAVE), 0, st, P,
                            relist, P.ncact, lparts, seeds ? seed_grid(P) : 0);
     } else
-        hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(P.ncact))), dim3(WAVE), 0, st, P);
+        hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(std::min(P.ncact, P.nact / NL_PART)))), dim3(WAVE), 0, st, P);
 }
 
 hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t st)
@@ -869,7 +858,6 @@ hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t s
         const int nch = (int)((nsub + SCAN_CH - 1) / SCAN_CH);
         const int gs = std::max(1, std::min(64, nch));
         hipLaunchKernelGGL(k_scan_sums, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P, commit, split, seeded);
-        hipLaunchKernelGGL(k_scan_chunks, dim3(P.nsys), dim3(SCAN_BLK), 0, st, P);
         hipLaunchKernelGGL(k_scan_apply, dim3(gs, P.nsys), dim3(SCAN_BLK), 0, st, P);
     }
     hipLaunchKernelGGL(k_scatter, g, b, 0, st, P, scan_one ? 1 : 0);

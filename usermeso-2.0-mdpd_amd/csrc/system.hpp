@@ -221,7 +221,7 @@ struct mdpd_system {
     DevBuf<float4> pos[2], vel[2], xhold, frc, vend, pr;
     DevBuf<int> tag[2], mask[2], origin[2], image[2];
     DevBuf<float> rho, vir, coef, minv, mmass, phi[2];
-    DevBuf<int> pcell, pslot, psub, tmp, cell_count, cell_start, cell_xyz, cell_rank, cell_sys, work_count;
+    DevBuf<int> pcell, pslot, psub, tmp, cell_count, cell_start, cell_xyz, cell_rank, cell_sys, work_count, chunk_sum;
     DevBuf<int4> cell_work;
     DevBuf<int2> cell_lse;
     DevBuf<int> nlist, ncount, clist, ccount, wave_sys, status, cl, wall_near;
@@ -1454,7 +1454,7 @@ struct mdpd_system {
         P.pcell = pcell.p; P.pslot = pslot.p; P.psub = psub.p; P.tmp = tmp.p;
         P.cell_count = cell_count.p; P.cell_start = cell_start.p; P.cell_xyz = cell_xyz.p;
         P.cell_rank = cell_rank.p; P.cell_sys = cell_sys.p;
-        P.work_count = work_count.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
+        P.work_count = work_count.p; P.chunk_sum = chunk_sum.p; P.cell_work = cell_work.p; P.cell_lse = cell_lse.p;
         P.nlist = nlist.p; P.ncount = ncount.p; P.wave_sys = wave_sys.p;
         P.clist = clist.p; P.ccount = ccount.p; P.status = status.p;
         P.cl = cl.p; P.wall_near = wall_near.p;
@@ -1655,7 +1655,7 @@ struct mdpd_system {
         cell_count.alloc((size_t)nslots * SUBCELLS); cell_start.alloc((size_t)nslots * SUBCELLS);
         cell_xyz.alloc(nslots);
         cell_rank.alloc(nslots); cell_sys.alloc(nslots);
-        cell_work.alloc(nslots); cell_lse.alloc(nslots); work_count.alloc(64);
+        cell_work.alloc(nslots); cell_lse.alloc(nslots); work_count.alloc(64); chunk_sum.alloc(nslots);
         coef.alloc(ds.coef.size()); minv.alloc(ntypes); mmass.alloc(ntypes); dsys.alloc(1);
 
         // ---- upload ----
