@@ -43,6 +43,15 @@ def _dpd(engine):
     return dpd_system(engine, x, v, 6.0)
 
 
+def _uneven(engine):
+    # a liquid next to its vapor: rows of none to ~50 pairs in one tile, the
+    # longest dealt over several rounds of raising the common part
+    x, v = uniform_box(700, 5.0, 23)
+    gas, _ = uniform_box(500, 12.0, 24)
+    x = np.concatenate([x, gas[np.any(gas > 5.5, axis=1)]])
+    return mdpd_system(engine, x, np.random.default_rng(2).normal(size=x.shape), 12.0)
+
+
 CASES = {
     "one": lambda e: _box(e, 1, 4.0),
     "tile - 1": lambda e: _box(e, 63, 4.0),
@@ -53,6 +62,7 @@ CASES = {
     # ~170 entries and ~80 pairs a row: several rounds of chunks and of pairs
     "dense": lambda e: _box(e, 1200, 4.0, rho_est=18.75, extra="timestep 0.001"),
     "two types": _two_types,
+    "uneven": _uneven,
     "walls": _walls,
     "dpd": _dpd,
 }

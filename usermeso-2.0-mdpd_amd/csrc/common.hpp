@@ -66,21 +66,36 @@ __device__ inline int xcd_logical(int b, int nlogical)
 }
 __host__ __device__ inline int xcd_grid(int nlogical) { return ((nlogical + NXCD - 1) / NXCD) * NXCD; }
 
-// inclusive prefix sum over the 64 lanes of a wave (every lane active)
-__device__ inline int wave_incl_scan(int x, int lane)
+// Across the 64 lanes of a wave (every lane active) with the data-parallel
+// moves of the vector unit: a step is an instruction, where a shuffle goes
+// through the LDS unit (~100 cycles, six in a row).  Lanes without a source
+// and the rows masked off get 0.
+template <int CTRL, int ROWS>
+__device__ inline int dpp_or_zero(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false); }
+
+// op over the lanes below and the lane itself: within rows of 16 (row_shr 1,
+// 2, 4, 8), then the last lane of row 0 and 2 to the row after it, then lane
+// 31 to the rows after it
+template <class Op>
+__device__ inline int wave_scan(int x, Op op)
 {
-    for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
-    return x;
+    x = op(x, dpp_or_zero<0x111, 0xF>(x));
+    x = op(x, dpp_or_zero<0x112, 0xF>(x));
+    x = op(x, dpp_or_zero<0x114, 0xF>(x));
+    x = op(x, dpp_or_zero<0x118, 0xF>(x));
+    x = op(x, dpp_or_zero<0x142, 0xA>(x));
+    return op(x, dpp_or_zero<0x143, 0xC>(x));
 }
 
-// sum over the 64 lanes of a wave, in every lane (every lane active)
-__device__ inline int wave_sum(int x)
+// inclusive prefix sum; sum and largest (of values >= 0) in every lane
+__device__ inline int wave_incl_scan(int x)
 {
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-    return x;
+    return wave_scan(x, [](int a, int b) { return a + b; });
+}
+__device__ inline int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
+__device__ inline int wave_max(int x)
+{
+    return __builtin_amdgcn_readlane(wave_scan(x, [](int a, int b) { return a > b ? a : b; }), 63);
 }
 
 enum Style : int { STYLE_MDPD = 0, STYLE_DPD = 1 };
@@ -435,11 +450,12 @@ __device__ inline float wall_ratio(float phi, float rcw)
 // image code -> shift multipliers
 __device__ inline void image_decode(uint32_t code, int &sx, int &sy, int &sz)
 {
-    int c = (int)code;
-    sz = (c * 57) >> 9;          // c / 9 for c < 27
-    int r = c - 9 * sz;
-    sy = (r * 11) >> 5;          // r / 3 for r < 9
-    sx = r - 3 * sy;
+    const int c = (int)code;
+    sz = (c * 57) >> 9;                 // c / 9 for c < 27
+    const int r = c - 9 * sz;
+    sy = (int)(((unsigned)r & 15u) * 11u) >> 5;     // r / 3 for r < 9 (the mask: a 24-bit product, not a
+                                                    // full one at a quarter of the rate)
+    sx = r - (sy + 2 * sy);
     sx -= 1; sy -= 1; sz -= 1;
 }
 

@@ -152,7 +152,7 @@ constexpr int SCAN_BLK = 256, SCAN_PER = 16, SCAN_CH = SCAN_BLK * SCAN_PER;
 __device__ inline int block_excl_scan(int x, int *wsum, int *total)
 {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int incl = wave_incl_scan(x, lane);
+    const int incl = wave_incl_scan(x);
     if (lane == 63) wsum[w] = incl;
     __syncthreads();
     int before = 0, all = 0;
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
             }
             const int cnt = __popc(full);
             const int lane = t & 63, wv = t >> 6;
-            const int incl = wave_incl_scan(cnt, lane);
+            const int incl = wave_incl_scan(cnt);
             if (lane == 63) s_wl[wv] = incl;
             __syncthreads();
             if (t == 0) {
@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(SCAN1_BLK) k_scan_one(PoolDev P, int commit, i
     }
     const int4 own = c < nc ? cnt4[c / 4] : make_int4(0, 0, 0, 0);
     const int sum = own.x + own.y + own.z + own.w;
-    const int incl = wave_incl_scan(sum, lane);
+    const int incl = wave_incl_scan(sum);
     before = wave_sum(before);
     if (lane == 63) {
         s_own[wv] = incl;
@@ -474,7 +474,7 @@ __global__ void __launch_bounds__(SORT1_BLK) k_sort_one(PoolDev P, int commit, i
         v[u] = c < nsub ? *(const int4 *)(s_cnt + c) : make_int4(0, 0, 0, 0);
         sum += v[u].x + v[u].y + v[u].z + v[u].w;
     }
-    const int incl = wave_incl_scan(sum, lane);
+    const int incl = wave_incl_scan(sum);
     if (lane == 63) s_wave[wv] = incl;
     __syncthreads();
     int run = incl - sum;
@@ -626,7 +626,7 @@ __device__ __attribute__((always_inline)) void nlist_cell(const PoolDev &P, int4
         ksy = (float)sy * d->L[1];
         ksz = (float)sz * d->L[2];
     }
-    const int kend = wave_incl_scan(klen, lane);
+    const int kend = wave_incl_scan(klen);
     const int kpre = kend - klen;                           // candidates before cell k
     const int ntot = __builtin_amdgcn_readlane(kend, 26);
     const float rc2 = d->rc2_list;
