@@ -179,3 +179,26 @@ def test_jobs_harvested_together_equal_their_own_runs(engine):
                 np.testing.assert_array_equal(p.gather(j, q), w, err_msg=f"batch {batch}, job {j}: {q}")
             p.release(j)
     p.close()
+
+
+# four waves share a tile's rows, a chunk of eight entries each in turn: fewer
+# rows than a tile, a partial and a full one, rows shorter than a chunk and
+# (1,200 particles in a box of 4) of some twenty chunks
+@pytest.mark.parametrize("n, L", [(2, 4.0), (63, 4.0), (65, 4.0), (257, 4.0), (1200, 4.0)])
+def test_rdf_counts_every_pair_once_from_each_side(engine, tmp_path, n, L):
+    x, v = uniform_box(n, L, 31 + n)
+    s = mdpd_system(engine, x, v, L, rho_est=max(6.0, n / L**3), extra=f"""
+        timestep 0.001
+        fix g all rdf/fast/meso output {tmp_path}/rdf.out nbin 20 every 3""")
+    s.run(3)
+    xr = s.gather("x")
+    g = s.fix_result("g")[1]
+    d = xr[:, None, :] - xr[None, :, :]
+    d -= L * np.round(d / L)
+    r = np.sqrt((d * d).sum(-1))[~np.eye(n, dtype=bool)]
+    unit = 1.0 / n / (4.0 / 3.0 * 3.1415 * ((np.arange(1, 21) * 0.05) ** 3 - (np.arange(20) * 0.05) ** 3)) / (n / L**3)
+    # a distance within 1e-5 of a bin's edge may fall on either side of it
+    lo = np.array([((r >= b * 0.05 + 1e-5) & (r < (b + 1) * 0.05 - 1e-5)).sum() for b in range(20)])
+    hi = np.array([((r >= b * 0.05 - 1e-5) & (r < (b + 1) * 0.05 + 1e-5)).sum() for b in range(20)])
+    assert np.all(g >= (lo - 1e-6) * unit) and np.all(g <= (hi + 1e-6) * unit)
+    s.close()
