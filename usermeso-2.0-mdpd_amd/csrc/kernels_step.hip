@@ -1066,36 +1066,48 @@ __global__ void __launch_bounds__(WAVE) k_aboundary(PoolDev P, int ntiles, int p
             const float c = d->cut_phi, c2 = c * c;
             const int wbit = d->fix_wall_bit;
             float phi = 0.f, nx = 0.f, ny = 0.f, nz = 0.f;
-            // the row in chunks of eight entries: the chunk's eight masks in
-            // flight, then the positions of its wall neighbors, the next
-            // chunk's entries loading meanwhile; terms added in row order
+            // the row in chunks of eight entries, the next chunk's masks and
+            // positions and the entries of the one after it loading meanwhile
+            // (two waves per SIMD: nothing else hides the chain of entry,
+            // mask, position; 122,000 particles 25 -> 18 us); terms added in
+            // row order
             const int nch = (cnt + NBR_CHUNK - 1) / NBR_CHUNK;
             int4 ea = make_int4(0, 0, 0, 0), eb = ea;
-            if (nch > 0) {
-                ea = row4[0];
-                eb = row4[1];
-            }
-            for (int ch = 0; ch < nch; ++ch) {
-                const uint32_t e[NBR_CHUNK] = {(uint32_t)ea.x, (uint32_t)ea.y, (uint32_t)ea.z, (uint32_t)ea.w,
-                                               (uint32_t)eb.x, (uint32_t)eb.y, (uint32_t)eb.z, (uint32_t)eb.w};
-                if (ch + 1 < nch) {
-                    ea = row4[(size_t)(ch + 1) * (NBR_CHUNK * WAVE / 4)];
-                    eb = row4[(size_t)(ch + 1) * (NBR_CHUNK * WAVE / 4) + 1];
+            auto entries = [&](int ch) {
+                if (ch < nch) {
+                    ea = row4[(size_t)ch * (NBR_CHUNK * WAVE / 4)];
+                    eb = row4[(size_t)ch * (NBR_CHUNK * WAVE / 4) + 1];
                 }
-                bool wall[NBR_CHUNK];
+            };
+            uint32_t e[NBR_CHUNK];
+            int m[NBR_CHUNK];
+            float4 q[NBR_CHUNK];
+            // past the row's end a lane takes itself, which is not a wall
+            auto gather = [&](int ch, uint32_t *eo, int *mo, float4 *qo) {
+                const uint32_t en[NBR_CHUNK] = {(uint32_t)ea.x, (uint32_t)ea.y, (uint32_t)ea.z, (uint32_t)ea.w,
+                                                (uint32_t)eb.x, (uint32_t)eb.y, (uint32_t)eb.z, (uint32_t)eb.w};
 #pragma unroll
                 for (int k = 0; k < NBR_CHUNK; ++k) {
                     const bool in = ch * NBR_CHUNK + k < cnt;
-                    wall[k] = in && (mask[(in ? e[k] : (uint32_t)i) & IDX_MASK] & wbit);
-                    near |= wall[k] ? 1 : 0;
+                    eo[k] = in ? en[k] : (uint32_t)i;
+                    mo[k] = mask[eo[k] & IDX_MASK];
+                    qo[k] = pos[eo[k] & IDX_MASK];
+                    if (!in) mo[k] = 0;
                 }
-                float4 q[NBR_CHUNK];
-#pragma unroll
-                for (int k = 0; k < NBR_CHUNK; ++k)
-                    if (wall[k]) q[k] = pos[e[k] & IDX_MASK];
+            };
+            entries(0);
+            gather(0, e, m, q);
+            entries(1);
+            for (int ch = 0; ch < nch; ++ch) {
+                uint32_t e1[NBR_CHUNK];
+                int m1[NBR_CHUNK];
+                float4 q1[NBR_CHUNK];
+                gather(ch + 1, e1, m1, q1);
+                entries(ch + 2);
 #pragma unroll
                 for (int k = 0; k < NBR_CHUNK; ++k) {
-                    if (!wall[k]) continue;
+                    if (!(m[k] & wbit)) continue;
+                    near = 1;
                     float dx, dy, dz;
                     pair_delta(p, q[k], e[k] >> IMG_SHIFT, d, dx, dy, dz);
                     const float rsq = dx * dx + dy * dy + dz * dz;
@@ -1106,6 +1118,12 @@ __global__ void __launch_bounds__(WAVE) k_aboundary(PoolDev P, int ntiles, int p
                     phi += (c + 3.f * r) * dd * dd * dd * d->phi_factor;
                     const float g = r * dd * dd * d->dw_factor * rinv;
                     nx -= g * dx; ny -= g * dy; nz -= g * dz;
+                }
+#pragma unroll
+                for (int k = 0; k < NBR_CHUNK; ++k) {
+                    e[k] = e1[k];
+                    m[k] = m1[k];
+                    q[k] = q1[k];
                 }
             }
             if (fresh) P.wall_near[i] = near;
