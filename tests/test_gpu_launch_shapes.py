@@ -202,3 +202,22 @@ def test_rdf_counts_every_pair_once_from_each_side(engine, tmp_path, n, L):
     hi = np.array([((r >= b * 0.05 - 1e-5) & (r < (b + 1) * 0.05 + 1e-5)).sum() for b in range(20)])
     assert np.all(g >= (lo - 1e-6) * unit) and np.all(g <= (hi + 1e-6) * unit)
     s.close()
+
+
+# systems admitted together are unpacked sixteen to a launch, as wide as the
+# largest of them
+@pytest.mark.parametrize("count", [1, 16, 17])
+def test_jobs_admitted_together_equal_their_own_runs(engine, count):
+    sizes = [(40 + 61 * k % 700, 4.0 + k % 3) for k in range(count)]
+    p = engine.Pool(float(1 << 29), 32)
+    p.tune("split", 2)
+    made = [_box(engine, n, L) for n, L in sizes]
+    jobs = [p.submit(s, 4) for s in made]
+    p.run()
+    for s, j in zip(made, jobs):
+        s.tune("split", 2)
+        s.run(4)
+        for k in ("x", "v", "tag", "image"):
+            np.testing.assert_array_equal(p.gather(j, k), s.gather(k), err_msg=f"job {j}: {k}")
+        s.close()
+    p.close()

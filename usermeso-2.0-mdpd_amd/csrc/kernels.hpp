@@ -49,6 +49,7 @@ hipError_t launch_aboundary(const PoolDev &P, int pooled, hipStream_t st);
 struct InLayout {
     size_t pos, vel, tag, mask, image, phi, rank, xyz, coef, mass, sys, bytes;
     int n, npad, nc1, ncoef, nt, has_phi;
+    InLayout() = default;
     InLayout(int n_, int npad_, int nc1_, int ncoef_, int nt_, bool phi_)
         : n(n_), npad(npad_), nc1(nc1_), ncoef(ncoef_), nt(nt_), has_phi(phi_ ? 1 : 0)
     {
@@ -68,8 +69,14 @@ struct InLayout {
         bytes = at;
     }
 };
-hipError_t launch_admit(const PoolDev &P, const InLayout &in, const void *block, int s, int part_base, int cell_base,
-                        hipStream_t st);
+// a submitted system on its way in: block (InLayout, readable from the
+// device), descriptor slot, first particle and cell slot
+struct AdmitItem {
+    InLayout in;
+    const char *block;
+    int slot, part_base, cell_base;
+};
+hipError_t launch_admit(const PoolDev &P, const AdmitItem *items, int count, hipStream_t st);
 
 // pooled engine, finished systems in descriptor slots[0 .. count): each one's
 // results in creation order, packed at the start of its own neighbor-row range

@@ -557,14 +557,14 @@ __global__ void __launch_bounds__(SORT1_BLK) k_sort_one(PoolDev P, int commit, i
 // mostly empty (a droplet fills a quarter of its box) or belong to systems
 // not re-sorted, and dispatching one workgroup per cell slot costs ~0.2 ns
 // each whether it works or exits (136 us per pass for 650,000 slots), so a
-// fixed grid of NL_GRID waves takes the list instead, XCD x the x-th eighth
+// grid of at most NL_GRID waves takes the list instead, XCD x the x-th eighth
 // of it in strides, so that cells next to each other in Morton order share
 // that XCD's L2 (batched droplets: rebuild phase 0.379 -> 0.278 ms per pass).
 // A relist covers every cell slot, one wave per slot.
 // --------------------------------------------------------------------------
 constexpr int NL_ITER = 7;             // candidate tiles per batch: 448 candidates (a cell's stencil averages ~370)
-constexpr int NL_WAVES = 8;            // waves per SIMD of the worklist walk (63 VGPRs; measured
-                                       // faster than seven, which needs no SGPR spills to VGPR lanes)
+constexpr int NL_WAVES = 8;            // waves per SIMD of the worklist walk (61 VGPRs; measured
+                                       // faster than seven)
 // its waves: one per NL_PART particle slots, about what the cells of a liquid
 // hold (waves without a cell cost their dispatch, 14 us for 65,536, 3.8 us for
 // the 13,000 of 24 droplets, 8 and 32 slots measured the same within 1%;

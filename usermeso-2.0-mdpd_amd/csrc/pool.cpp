@@ -186,7 +186,8 @@ struct HarvestView {
 static_assert(HARVEST_SLOT_BYTES == 88, "stage layout");
 // bytes of device memory per particle slot (state and scratch), per cell
 // slot (rank, coordinates, system; worklist entry, linear range; count and
-// start per sub-cell), and per neighbor-row entry (nlist + clist);
+// start per sub-cell; the chunk totals' word is in the slot's figure), and per
+// neighbor-row entry (nlist + clist);
 // CELLS_PER_SLOT cell slots are kept per particle slot
 constexpr double BYTES_PER_SLOT = 256.0;
 constexpr double BYTES_PER_CELL = 12.0 + 16.0 + 8.0 + 8.0 * SUBCELLS;
@@ -265,6 +266,8 @@ struct mdpd_pool {
     size_t held_pinned = 0;               // stage bytes kept by finished jobs
     size_t max_held = (size_t)1 << 30;    // beyond this their results move to pageable memory
     std::vector<std::pair<hipEvent_t, std::pair<void *, size_t>>> uploads;
+    std::vector<AdmitItem> admits;            // admitted, still to be unpacked (flush_admits)
+    std::vector<size_t> admit_bytes;
     std::vector<hipEvent_t> ev_free;
 
     // ---- counters ----
@@ -293,6 +296,7 @@ struct mdpd_pool {
             (void)hipEventDestroy(u.first);
             (void)hipHostFree(u.second.first);
         }
+        for (auto &a : admits) (void)hipHostFree((void *)a.block);
         for (auto &j : jobs) {
             if (j.second->ev) (void)hipEventDestroy(j.second->ev);
             if (j.second->stage) (void)hipHostFree(j.second->stage);
@@ -626,7 +630,10 @@ struct mdpd_pool {
                 ++k;
                 continue;
             }
-            if (j.ds.want_maxnbr > maxnbr) regrow(j.ds.want_maxnbr);
+            if (j.ds.want_maxnbr > maxnbr) {
+                flush_admits();
+                regrow(j.ds.want_maxnbr);
+            }
             const int s = free_slots.back();
             free_slots.pop_back();
             if (k == 0) head_bypass = 0;
@@ -635,8 +642,23 @@ struct mdpd_pool {
             upload(j, s, pb * 256, cb);
             any = true;
         }
+        flush_admits();
         if (any) update_extent();
         return any;
+    }
+
+    // the systems admitted since the last flush, unpacked in one launch
+    void flush_admits()
+    {
+        if (admits.empty()) return;
+        hip_check(launch_admit(view(), admits.data(), (int)admits.size(), stream), "admit");
+        while (!admits.empty()) {                 // a block returns to the cache once the launch has read it
+            hipEvent_t e = take_event();
+            hip_check(hipEventRecord(e, stream), "hipEventRecord");
+            uploads.push_back({e, {(void *)admits.back().block, admit_bytes.back()}});
+            admits.pop_back();
+            admit_bytes.pop_back();
+        }
     }
 
     void upload(Job &j, int s, long long pbase, long long cbase)
@@ -699,10 +721,8 @@ struct mdpd_pool {
         }
         j.in = nullptr;
         memcpy(st + L.sys, &d, sizeof(SysDev));
-        hip_check(launch_admit(view(), L, st, s, (int)pbase, (int)cbase, stream), "admit");
-        hipEvent_t e = take_event();
-        hip_check(hipEventRecord(e, stream), "hipEventRecord");
-        uploads.push_back({e, {st, got}});
+        admits.push_back({L, st, s, (int)pbase, (int)cbase});
+        admit_bytes.push_back(got);
 
         j.slot = s;
         j.part_base = pbase;
