@@ -207,25 +207,49 @@ __global__ void __launch_bounds__(WAVE * SPLIT) k_first(PoolDev P, int ntiles, i
             }
         }
         float4 q[U * NBR_CHUNK];
-        // when every active lane's row covers all of this iteration's
-        // entries and its staging area has room for all of them, the
-        // per-entry row-end and staging checks are skipped (same result)
-        const bool full = (c + (U - 1) * SPLIT + 1) * NBR_CHUNK <= cnt && nc + U * NBR_CHUNK <= STAGE;
-        if (__builtin_amdgcn_ballot_w64(!full) == 0) {
+        if constexpr (SPLIT == 1) {
+            // past the row's end a lane takes itself (r = 0, skipped), so only
+            // the room in the staging area is left to check, by iteration
+            // (256 droplets 214 -> 210 us; with two or four waves per tile it
+            // costs registers: 480,000 particles 80 -> 86)
 #pragma unroll
-            for (int k = 0; k < U * NBR_CHUNK; ++k) q[k] = pos[e[k] & IDX_MASK];
+            for (int u = 0; u < U; ++u) {
+                const int left = cnt - (c + u) * NBR_CHUNK;
+                if (__builtin_amdgcn_ballot_w64(left < NBR_CHUNK) != 0)
 #pragma unroll
-            for (int k = 0; k < U * NBR_CHUNK; ++k) visit(e[k], q[k], std::true_type{});
-        } else {
-#pragma unroll
-            for (int k = 0; k < U * NBR_CHUNK; ++k) {
-                const int p = (c + (k / NBR_CHUNK) * SPLIT) * NBR_CHUNK + k % NBR_CHUNK;
-                q[k] = pos[(p < cnt ? e[k] : (uint32_t)i) & IDX_MASK];
+                    for (int k = 0; k < NBR_CHUNK; ++k)
+                        if (k >= left) e[u * NBR_CHUNK + k] = (uint32_t)i | ((uint32_t)IMG_ZERO << IMG_SHIFT);
             }
 #pragma unroll
-            for (int k = 0; k < U * NBR_CHUNK; ++k) {
-                const int p = (c + (k / NBR_CHUNK) * SPLIT) * NBR_CHUNK + k % NBR_CHUNK;
-                if (p < cnt) visit(e[k], q[k], std::false_type{});
+            for (int k = 0; k < U * NBR_CHUNK; ++k) q[k] = pos[e[k] & IDX_MASK];
+            if (__builtin_amdgcn_ballot_w64(nc + U * NBR_CHUNK > STAGE) == 0) {
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) visit(e[k], q[k], std::true_type{});
+            } else {
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) visit(e[k], q[k], std::false_type{});
+            }
+        } else {
+            // when every active lane's row covers all of this iteration's
+            // entries and its staging area has room for all of them, the
+            // per-entry row-end and staging checks are skipped (same result)
+            const bool full = (c + (U - 1) * SPLIT + 1) * NBR_CHUNK <= cnt && nc + U * NBR_CHUNK <= STAGE;
+            if (__builtin_amdgcn_ballot_w64(!full) == 0) {
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) q[k] = pos[e[k] & IDX_MASK];
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) visit(e[k], q[k], std::true_type{});
+            } else {
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) {
+                    const int p = (c + (k / NBR_CHUNK) * SPLIT) * NBR_CHUNK + k % NBR_CHUNK;
+                    q[k] = pos[(p < cnt ? e[k] : (uint32_t)i) & IDX_MASK];
+                }
+#pragma unroll
+                for (int k = 0; k < U * NBR_CHUNK; ++k) {
+                    const int p = (c + (k / NBR_CHUNK) * SPLIT) * NBR_CHUNK + k % NBR_CHUNK;
+                    if (p < cnt) visit(e[k], q[k], std::false_type{});
+                }
             }
         }
     }
@@ -562,6 +586,7 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
     __shared__ float4 s_pi[BAL ? WAVE : 1], s_vi[BAL ? WAVE : 1];
     __shared__ float s_ri[BAL ? WAVE : 1];
     __shared__ float s_tail[TAIL_CAP * NA];
+    __shared__ int s_own[TAIL_CAP];
     // the same between a wave's sub-rows (two or four waves per tile)
     constexpr int NB = SPLIT > 1 ? SPLIT : 1, NL = SPLIT > 1 ? WAVE : 1;
     __shared__ float4 s_bp[NB][NL], s_bv[NB][NL], s_bt[NB][NL];
@@ -715,16 +740,19 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
             s_pi[lane] = pi;
             s_vi[lane] = vi;
             s_ri[lane] = rho_i;
+            for (int f0 = 0; f0 < TAIL_CAP; f0 += WAVE) s_own[f0 + lane] = 0;
+            __syncthreads();
+            if (sur > 0) s_own[first] = lane;
             __syncthreads();
             const int *ctile = P.clist + (size_t)tile * maxnbr * WAVE;
+            int carry = 0;
             for (int f0 = 0; f0 < tail; f0 += WAVE) {
                 const int f = f0 + lane;
-                // owner: the last particle whose first slot is <= f (the
-                // particles before it with no tail share its first slot)
-                int p = 0;
-#pragma unroll
-                for (int step = 32; step > 0; step >>= 1)
-                    if (__shfl(first, p + step) <= f) p += step;
+                // owner: the last particle whose tail starts at or before f,
+                // spread from where the tails start (a search of six
+                // shuffles per round takes four registers more)
+                const int p = max(wave_scan(s_own[f], [](int x, int y) { return max(x, y); }), carry);
+                carry = __builtin_amdgcn_readlane(p, 63);
                 const int t = M + f - __shfl(first, p);
                 const bool act = f < tail;
                 // a lane past the last tail evaluates its own particle with
