@@ -241,3 +241,28 @@ def test_one_wave_per_tile_sums_the_same_terms(engine, case):
     rms = np.sqrt((fb**2).sum(-1).mean())
     size = np.maximum(np.sqrt((fb**2).sum(-1)), rms)
     assert np.all(np.sqrt(((fa - fb) ** 2).sum(-1)) <= 2e-5 * size + 1e-30)
+
+
+# a wall fraction below zero (rho_wall < 0) scales a mobile particle's pairs
+# with wall particles as any other does: a pool's launches (more tiles than the
+# wide kernels take) deal the ends of long rows to other lanes
+@pytest.mark.parametrize("split", [2, 4])
+def test_negative_wall_fractions_scale_every_pair(engine, split):
+    x, v, types, nf = channel()
+    s = engine.System()
+    s.command("atom_style mdpd/atomic/meso 8.0")
+    s.create_box(2, (0, 0, 0), (LX, LY, LZ))
+    s.create_atoms(types, x, v)
+    s.commands(DECK.replace("rho_wall 8.0", "rho_wall -8.0"))
+    p = engine.Pool(float(1 << 29), 16)
+    p.tune("split", split)
+    j = p.submit(s, 6)
+    p.run()
+    assert p.stat("capacity") > 512 * 64
+    s.tune("split", split)
+    s.run(6)
+    assert s.gather("phi")[:nf].min() < 0
+    for k in ("x", "v", "f", "rho"):
+        np.testing.assert_array_equal(p.gather(j, k), s.gather(k), err_msg=f"split {split}: {k}")
+    p.close()
+    s.close()

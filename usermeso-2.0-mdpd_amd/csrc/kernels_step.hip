@@ -825,10 +825,12 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
             s_bp[w][lane] = pi;
             s_bv[w][lane] = vi;
             s_br[w][lane] = rho_i;
-            s_bphi[w][lane] = arb_i ? phi_i : -1.f;
-            // entry k of the tail: its particle, its row position, odd last entry
+            s_bphi[w][lane] = phi_i;
+            // entry k of the tail: its particle, its row position, odd last
+            // entry, scaled by the wall fraction (whatever its sign)
             for (int k = 0; k < sur; ++k)
-                s_who[w][first + k] = lane | (M + k) << 6 | ((cnt & 1) && M + k == cnt - 1 ? 1 << 30 : 0);
+                s_who[w][first + k] = (int)((uint32_t)(lane | (M + k) << 6) |
+                                            ((cnt & 1) && M + k == cnt - 1 ? 1u << 30 : 0u) | (arb_i ? 1u << 31 : 0u));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             const bool act = lane < tail;
@@ -840,9 +842,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
             float rj;
             nbr(j, q, rj);
             const float4 vj = vel[j], pp = s_bp[w][p];
-            const float ph = s_bphi[w][p];
             PairC c = UNI ? cu : load_coef(coef, __float_as_int(pp.w) * nt + (act ? __float_as_int(q.w) : 0));
-            wall_scale_of(c, j, ph >= 0.f, ph);
+            wall_scale_of(c, j, who < 0, s_bphi[w][p]);
             const PairF o = pair_eval<STYLE, EV, !UNI>(pp, s_bv[w][p], s_br[w][p], q, vj, rj, e >> IMG_SHIFT, c, dtis, d,
                                                        who >> 30 & 1);
             s_bt[w][lane] = make_float4(o.dx, o.dy, o.dz, o.fpair);
