@@ -266,3 +266,25 @@ def test_negative_wall_fractions_scale_every_pair(engine, split):
         np.testing.assert_array_equal(p.gather(j, k), s.gather(k), err_msg=f"split {split}: {k}")
     p.close()
     s.close()
+
+
+# energies and virials of the last pass are evaluated by one launch over all
+# jobs that end together: sixty of them are more tiles than the wide kernels
+# take, a job's own handle is not
+@pytest.mark.parametrize("split", [2, 4])
+@pytest.mark.parametrize("case", ["liquid", "two types", "dpd"])
+def test_results_of_many_jobs_ending_together_equal_their_own_runs(engine, case, split):
+    s = CASES[case](engine)
+    count = -(-513 * 64 // ((s.natoms + 255) // 256 * 256))
+    p = engine.Pool(float(1 << 29), count)
+    p.tune("split", split)
+    jobs = [p.submit(s, 5) for _ in range(count)]
+    p.run()
+    s.tune("split", split)
+    s.run(5)
+    for k in ("f", "e_pair", "virial"):
+        want = s.gather(k)
+        for j in jobs:
+            np.testing.assert_array_equal(p.gather(j, k), want, err_msg=f"{case}, split {split}, job {j}: {k}")
+    p.close()
+    s.close()

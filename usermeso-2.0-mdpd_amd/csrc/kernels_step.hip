@@ -446,9 +446,14 @@ struct Acc {
 // yx: dx.dv starts from the y product, as it does for the odd last entry of
 // the rows (or row parts) that the loops below walk in pairs; its rounding is
 // part of a trajectory, which grows any difference, so every kernel keeps it.
+// Energy: en * eg, added with one rounding (eg = 1: en, which has had its own).
+// DPD of one type keeps the factors apart so that every kernel rounds alike.
 struct PairF {
-    float dx, dy, dz, fpair, en;
+    float dx, dy, dz, fpair, en, eg;
 };
+
+// styles whose energy is kept as two factors
+constexpr bool en_factors(int style) { return style == STYLE_DPD; }
 
 template <int STYLE, bool EV, bool TEST = true>
 __device__ inline PairF pair_eval(const float4 &pi, const float4 &vi, float rho_i, const float4 &q, const float4 &vj,
@@ -467,7 +472,7 @@ __device__ inline PairF pair_eval(const float4 &pi, const float4 &vi, float rho_
     const float xi = pair_gaussian(__float_as_uint(vi.w), __float_as_uint(vj.w));
     // sigma / sqrt(dt): uniform for a one-type system away from walls
     const float sdt = c.sigma * dtis;
-    float fpair, en = 0.f;
+    float fpair, en = 0.f, eg = 1.f;
     if (STYLE == STYLE_MDPD) {
         // pair_mdpd_meso.cu:156-191: F = [A wc + B (rho_i + rho_j) wr
         //   - gamma wc^2 (dx.dv)/r + sigma wc xi / sqrt(dt)] / r, evaluated as
@@ -485,11 +490,16 @@ __device__ inline PairF pair_eval(const float4 &pi, const float4 &vi, float rho_
         const float wr = c.expw == 1.f ? wc : powf(wc, c.expw);
         const float t = fmaf(-(c.gamma * wr * rinv), dot, sdt * xi);
         fpair = fmaf(c.a, wc, wr * t) * rinv;
-        if (EV) en = 0.5f * c.a * c.rc * wc * wc;
+        if (EV) {
+            en = 0.5f * c.a * c.rc * wc;
+            if (TEST) en = en * wc;
+            else eg = wc;
+        }
     }
     o.dx = dx; o.dy = dy; o.dz = dz;
     o.fpair = in ? fpair : 0.f;
     o.en = in ? en : 0.f;
+    o.eg = eg;
     return o;
 }
 
@@ -503,7 +513,7 @@ __device__ inline void pair_add(Acc<EV> &a, const PairF &o)
     a.v[1] = fmaf(o.dy, o.fpair, a.v[1]);
     a.v[2] = fmaf(o.dz, o.fpair, a.v[2]);
     if (EV) {
-        a.v[3] += o.en;
+        a.v[3] = fmaf(o.en, o.eg, a.v[3]);
         a.v[4] = fmaf(o.dx * o.dx, o.fpair, a.v[4]);
         a.v[5] = fmaf(o.dy * o.dy, o.fpair, a.v[5]);
         a.v[6] = fmaf(o.dz * o.dz, o.fpair, a.v[6]);
@@ -591,6 +601,8 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
     constexpr int NB = SPLIT > 1 ? SPLIT : 1, NL = SPLIT > 1 ? WAVE : 1;
     __shared__ float4 s_bp[NB][NL], s_bv[NB][NL], s_bt[NB][NL];
     __shared__ float s_br[NB][NL], s_bphi[NB][NL], s_be[EV ? NB : 1][EV ? NL : 1];
+    constexpr bool EG = EV && en_factors(STYLE);
+    __shared__ float s_bg[EG ? NB : 1][EG ? NL : 1];
     __shared__ int s_who[NB][NL];
     const int lt = xcd_logical(blockIdx.x, ntiles);
     if (lt >= ntiles) return;
@@ -848,11 +860,12 @@ __global__ void __launch_bounds__(WAVE * SPLIT)
                                                        who >> 30 & 1);
             s_bt[w][lane] = make_float4(o.dx, o.dy, o.dz, o.fpair);
             if (EV) s_be[w][lane] = o.en;
+            if (EG) s_bg[w][lane] = o.eg;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             for (int f = first; f < first + sur; ++f) {
                 const float4 x = s_bt[w][f];
-                pair_add<EV>(a, PairF{x.x, x.y, x.z, x.w, EV ? s_be[w][f] : 0.f});
+                pair_add<EV>(a, PairF{x.x, x.y, x.z, x.w, EV ? s_be[w][f] : 0.f, EG ? s_bg[w][f] : 1.f});
             }
         }
     } else {
@@ -895,7 +908,8 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
     constexpr int UPW = (NU + FW_WAVES - 1) / FW_WAVES;
     static_assert(FW_WAVES % SPLIT == 0, "a wave's rows belong to one sub-row");
     __shared__ float s_d[3][R][WAVE], s_f[R][WAVE];    // dx, dy, dz and F / r of each pair
-    __shared__ float s_en[EV ? R : 1][WAVE];
+    constexpr bool EG = EV && en_factors(STYLE);
+    __shared__ float s_en[EV ? R : 1][WAVE], s_eg[EG ? R : 1][WAVE];
     __shared__ float s_acc[SPLIT][NA][WAVE];
     __shared__ uint32_t s_sig[WAVE];
     const int lt = xcd_logical(blockIdx.x, ntiles);
@@ -997,6 +1011,7 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
                 s_d[2][k][lane] = o.dz;
                 s_f[k][lane] = o.fpair;
                 if (EV) s_en[k][lane] = o.en;
+                if (EG) s_eg[k][lane] = o.eg;
             }
         }
         __syncthreads();
@@ -1006,6 +1021,7 @@ __global__ void __launch_bounds__(WAVE * (FW_WAVES + 1)) k_force_wide(PoolDev P,
                     PairF o;
                     o.dx = s_d[0][k][lane]; o.dy = s_d[1][k][lane]; o.dz = s_d[2][k][lane];
                     o.fpair = s_f[k][lane]; o.en = s_en[k][lane];
+                    o.eg = EG ? s_eg[k][lane] : 1.f;
                     pair_add<EV>(a, o);
                 }
         } else if (wv < FW_WAVES) {
