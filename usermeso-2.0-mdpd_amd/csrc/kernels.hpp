@@ -87,7 +87,9 @@ hipError_t launch_admit(const PoolDev &P, const AdmitItem *items, int count, hip
 constexpr size_t HARVEST_SLOT_BYTES = 3 * 16 + 3 * 4 + 4 + 6 * 4;
 inline size_t harvest_bytes(size_t npad) { return npad * HARVEST_SLOT_BYTES + sizeof(SysDev); }
 inline size_t harvest_dst(const PoolDev &P, int part_base) { return (size_t)part_base * P.maxnbr; }
-hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, hipStream_t st);
+// bad: a word per descriptor slot, writable from the device; set to 1 when a
+// particle of that system has no valid creation index (its results are not whole)
+hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, int *bad, hipStream_t st);
 
 // one system: a per-atom quantity in creation order, gather_words(field) 4-byte
 // words per particle (floats, or ints from G_TAG on; image unpacked, type 1-based)
@@ -96,7 +98,8 @@ constexpr int gather_words(int field)
 {
     return field == G_X || field == G_V || field == G_F || field == G_IMAGE ? 3 : field == G_VIRIAL ? 6 : 1;
 }
-hipError_t launch_gather(const PoolDev &P, int field, int *out, hipStream_t st);
+// bad: one word, as for launch_harvest
+hipError_t launch_gather(const PoolDev &P, int field, int *out, int *bad, hipStream_t st);
 
 // observables (accumulate into device histograms of nbin + 1 slots, slot nbin
 // counting the samples; a system whose rows overflowed is not sampled)

@@ -1287,14 +1287,15 @@ __global__ void __launch_bounds__(256) k_admit(PoolDev P, AdmitList list)
 // order), so the host copies one range.  Runs after the HARVEST force pass,
 // which reads the other buffer.  The system's tiles and cell slots are
 // unmapped here (no kernel after it finds the system through them); the host
-// frees the ranges once the copy has landed.
+// frees the ranges once the copy has landed.  A creation index outside the
+// system would leave a slot of the block unwritten: it is reported in `bad`.
 // --------------------------------------------------------------------------
 constexpr int HARVEST_LIST = 64;
 struct HarvestList {
     int slot[HARVEST_LIST];
 };
 
-__global__ void __launch_bounds__(256) k_harvest(PoolDev P, HarvestList list)
+__global__ void __launch_bounds__(256) k_harvest(PoolDev P, HarvestList list, int *bad)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     const SysDev *d = P.sys + list.slot[blockIdx.y];
@@ -1310,7 +1311,10 @@ __global__ void __launch_bounds__(256) k_harvest(PoolDev P, HarvestList list)
     if (k >= d->n) return;
     const int i = pb + k, cur = d->sel, cura = d->sela;
     const int c = P.origin[cura][i];                          // creation index
-    if (c < 0 || c >= d->n) return;
+    if (c < 0 || c >= d->n) {
+        bad[list.slot[blockIdx.y]] = 1;
+        return;
+    }
     const size_t n = npad;
     float4 *o4 = (float4 *)dst;
     o4[c] = P.pos[cur][i];
@@ -1330,14 +1334,17 @@ __global__ void __launch_bounds__(256) k_harvest(PoolDev P, HarvestList list)
 // One system's per-atom quantity in creation order (the host copies one block
 // and only widens it).
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_gather(PoolDev P, int field, int *out)
+__global__ void __launch_bounds__(256) k_gather(PoolDev P, int field, int *out, int *bad)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const SysDev *d = P.sys;
     if (i >= d->n) return;
     const int sel = d->sel, sela = d->sela;
     const int c = P.origin[sela][i];
-    if (c < 0 || c >= d->n) return;
+    if (c < 0 || c >= d->n) {
+        *bad = 1;
+        return;
+    }
     float *of = (float *)out;
     auto put3 = [&](const float4 &q) { of[3 * c] = q.x; of[3 * c + 1] = q.y; of[3 * c + 2] = q.z; };
     switch (field) {
@@ -1462,11 +1469,11 @@ hipError_t launch_admit(const PoolDev &P, const AdmitItem *items, int count, hip
     return hipGetLastError();
 }
 
-hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, hipStream_t st)
+hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npad_max, int *bad, hipStream_t st)
 {
     // the packed block fits the rows: maxnbr entries per slot, at least NBR_ALIGN
     static_assert(sizeof(SysDev) <= 256 * (4 * NBR_ALIGN - HARVEST_SLOT_BYTES), "harvest block fits the rows");
-    if (P.maxnbr < NBR_ALIGN || npad_max <= 0 || npad_max > P.cap) return hipErrorInvalidValue;
+    if (P.maxnbr < NBR_ALIGN || npad_max <= 0 || npad_max > P.cap || !bad) return hipErrorInvalidValue;
     for (int q0 = 0; q0 < count; q0 += HARVEST_LIST) {
         HarvestList list{};
         const int m = count - q0 < HARVEST_LIST ? count - q0 : HARVEST_LIST;
@@ -1474,16 +1481,16 @@ hipError_t launch_harvest(const PoolDev &P, const int *slots, int count, int npa
             list.slot[q] = slots[q0 + q];
             if (list.slot[q] < 0 || list.slot[q] >= P.nsys) return hipErrorInvalidValue;
         }
-        hipLaunchKernelGGL(k_harvest, dim3((npad_max + 255) / 256, m), dim3(256), 0, st, P, list);
+        hipLaunchKernelGGL(k_harvest, dim3((npad_max + 255) / 256, m), dim3(256), 0, st, P, list, bad);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_gather(const PoolDev &P, int field, int *out, hipStream_t st)
+hipError_t launch_gather(const PoolDev &P, int field, int *out, int *bad, hipStream_t st)
 {
-    if (!P.one || field < G_X || field > G_IMAGE || !out) return hipErrorInvalidValue;
+    if (!P.one || field < G_X || field > G_IMAGE || !out || !bad) return hipErrorInvalidValue;
     if (P.nact == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gather, dim3((P.nact + 255) / 256), dim3(256), 0, st, P, field, out);
+    hipLaunchKernelGGL(k_gather, dim3((P.nact + 255) / 256), dim3(256), 0, st, P, field, out, bad);
     return hipGetLastError();
 }
 

@@ -257,6 +257,7 @@ struct mdpd_pool {
 
     // ---- status polling and staging ----
     int *pin_status[2] = {nullptr, nullptr};
+    int *pin_bad = nullptr;               // per descriptor slot: launch_harvest's error word
     hipEvent_t ev_poll[2] = {nullptr, nullptr};
     bool poll_pending[2] = {false, false};
     int poll_cur = 0;
@@ -310,6 +311,7 @@ struct mdpd_pool {
             if (ev_poll[k]) (void)hipEventDestroy(ev_poll[k]);
             if (pin_status[k]) (void)hipHostFree(pin_status[k]);
         }
+        if (pin_bad) (void)hipHostFree(pin_bad);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -327,17 +329,20 @@ struct mdpd_pool {
 
     void ensure_stream()
     {
-        if (stream) return;
+        if (pin_bad) return;                  // the last thing made here
         int ndev = 0;
         if (hipGetDeviceCount(&ndev) != hipSuccess || device >= ndev)
             fail(MDPD_E_HIP, "HIP device %d is not available", device);
         hip_check(hipSetDevice(device), "hipSetDevice");
-        hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
+        if (!stream) hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
         for (int k = 0; k < 2; ++k) {
-            hip_check(hipHostMalloc((void **)&pin_status[k], sizeof(int) * max_sys, hipHostMallocDefault),
-                      "hipHostMalloc");
-            hip_check(hipEventCreateWithFlags(&ev_poll[k], hipEventDisableTiming), "hipEventCreate");
+            if (!pin_status[k])
+                hip_check(hipHostMalloc((void **)&pin_status[k], sizeof(int) * max_sys, hipHostMallocDefault),
+                          "hipHostMalloc");
+            if (!ev_poll[k])
+                hip_check(hipEventCreateWithFlags(&ev_poll[k], hipEventDisableTiming), "hipEventCreate");
         }
+        hip_check(hipHostMalloc((void **)&pin_bad, sizeof(int) * max_sys, hipHostMallocDefault), "hipHostMalloc");
     }
 
     PoolDev view()
@@ -1044,6 +1049,7 @@ struct mdpd_pool {
             hi = std::max(hi, j->part_base + j->npad);
             npad_max = std::max(npad_max, j->npad);
             slots.push_back(j->slot);
+            pin_bad[j->slot] = 0;
             kinds.insert({j->ds.d.style, j->ntypes == 1});
         }
         // each system is evaluated by the launch of its last pass's split
@@ -1052,7 +1058,7 @@ struct mdpd_pool {
                 if (splits_used & sp)
                     hip_check(launch_force_range(P, k.first, MODE_HARVEST, k.second, sp, (int)(lo / WAVE),
                                                  (int)((hi - lo) / WAVE), stream), "harvest");
-        hip_check(launch_harvest(P, slots.data(), (int)slots.size(), npad_max, stream), "harvest");
+        hip_check(launch_harvest(P, slots.data(), (int)slots.size(), npad_max, pin_bad, stream), "harvest");
         for (Job *j : fin) copy_harvest(P, *j);
     }
 
@@ -1093,6 +1099,7 @@ struct mdpd_pool {
             const hipError_t q = block ? hipEventSynchronize(j.ev) : hipEventQuery(j.ev);
             if (q == hipErrorNotReady) continue;
             hip_check(q, "harvest event");
+            if (pin_bad[j.slot]) fail(MDPD_E_HIP, "harvest of job %d: a particle without a valid creation index", j.id);
             const HarvestView h(j);
             SysDev d;
             memcpy(&d, h.desc, sizeof(SysDev));

@@ -228,7 +228,7 @@ struct mdpd_system {
     DevBuf<SysDev> dsys;
     int *pinned = nullptr;            // host-visible readback of flags
     static constexpr size_t STAGE_WORDS = 1 << 17;
-    int *stage = nullptr;             // two pinned halves of STAGE_WORDS words (gather)
+    int *stage = nullptr;             // two pinned halves of STAGE_WORDS words (gather), and its error word
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 
     // ---- kernel timing with HIP events (phase -> total ms, launches) ----
@@ -2016,11 +2016,13 @@ struct mdpd_system {
     {
         static_assert(NBR_ALIGN >= 6, "six words per particle fit the narrowest compact rows");
         if (!stage) {
-            hip_check(hipHostMalloc((void **)&stage, 2 * STAGE_WORDS * sizeof(int), hipHostMallocDefault),
+            hip_check(hipHostMalloc((void **)&stage, (2 * STAGE_WORDS + 1) * sizeof(int), hipHostMallocDefault),
                       "hipHostMalloc");
             for (auto &e : stage_ev) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
         }
-        hip_check(launch_gather(view(), field, clist.p, stream), "gather");
+        int *bad = stage + 2 * STAGE_WORDS;
+        *bad = 0;
+        hip_check(launch_gather(view(), field, clist.p, bad, stream), "gather");
         const size_t nc = (words + STAGE_WORDS - 1) / STAGE_WORDS;
         auto len = [&](size_t c) { return std::min(STAGE_WORDS, words - c * STAGE_WORDS); };
         for (size_t c = 0; c <= nc; ++c) {
@@ -2038,6 +2040,7 @@ struct mdpd_system {
             else
                 memcpy(k + at, src, m * sizeof(int));
         }
+        if (*bad) fail(MDPD_E_HIP, "gather: a particle without a valid creation index");
     }
 
     // pull the device state back into the creation-order host arrays
