@@ -110,7 +110,8 @@ long long mdpd_get_nbuild(const mdpd_system *sys);
  * fraction of the arbitrary-boundary branch) "e_pair" (1,1)
  * "virial" (1,6: xx yy zz xy xz yz) "tag" (0,1) "type" (0,1) "mask" (0,1)
  * "image" (0,3).  f, e_pair and virial are those of the last force pass of
- * setup or of the last step of a run. */
+ * setup or of the last step of a run.  The first call keeps 1 MiB of pinned
+ * host memory with the handle. */
 int mdpd_gather_atoms(mdpd_system *sys, const char *name, int type, int count, void *data);
 /* lammps_scatter_atoms (src/library.h:42) for "x" and "v" (type 1, count 3):
  * overwrite positions / velocities in creation order; the next run repeats
@@ -205,8 +206,11 @@ int mdpd_tea_gaussian_noalloc(int device, int n, const unsigned int *a, const un
  * times before it goes first),
  * keeps its state resident while it runs, and leaves when done; its results
  * stay readable until mdpd_pool_release (88 bytes per particle slot of host
- * memory, pinned while finished jobs hold less than 1 GiB of it).  One host
- * thread drives a pool. */
+ * memory, pinned while finished jobs hold less than 1 GiB of it).  A waiting
+ * job's input (40 to 44 bytes per particle and 8 per cell) is host memory too:
+ * once the pool is on its device pinned, in blocks of powers of two from 1 MiB
+ * up, while waiting jobs hold less than 512 MiB of them.  Blocks are reused and
+ * freed with the pool.  One host thread drives a pool. */
 typedef struct mdpd_pool mdpd_pool;
 
 enum { MDPD_JOB_QUEUED = 0, MDPD_JOB_RUNNING = 1, MDPD_JOB_DONE = 2 };

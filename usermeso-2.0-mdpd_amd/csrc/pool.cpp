@@ -21,6 +21,7 @@
 // per-system status word every few passes (asynchronously, one batch behind):
 // finished systems are harvested (energy/virial pass + copy-out), their
 // particle and cell ranges freed, and queued jobs admitted into the space.
+#include "pinned.hpp"
 #include "system.hpp"
 
 #include <chrono>
@@ -84,32 +85,6 @@ struct RangeAlloc {
             }
         }
     }
-};
-
-// page-locked staging buffers, reused by size (asynchronous copies need them)
-struct PinnedCache {
-    std::multimap<size_t, void *> free_;
-    ~PinnedCache()
-    {
-        for (auto &f : free_) (void)hipHostFree(f.second);
-    }
-    void *get(size_t bytes, size_t &got)
-    {
-        auto it = free_.lower_bound(bytes);
-        if (it != free_.end()) {
-            got = it->first;
-            void *p = it->second;
-            free_.erase(it);
-            return p;
-        }
-        size_t sz = (size_t)1 << 16;
-        while (sz < bytes) sz <<= 1;
-        void *p = nullptr;
-        hip_check(hipHostMalloc(&p, sz, hipHostMallocDefault), "hipHostMalloc");
-        got = sz;
-        return p;
-    }
-    void put(void *p, size_t sz) { free_.emplace(sz, p); }
 };
 
 enum JobState { JOB_QUEUED = 0, JOB_RUNNING = 1, JOB_DONE = 2 };
@@ -199,7 +174,6 @@ constexpr size_t ADMIT_LOOKAHEAD = 64;    // queued jobs considered per admissio
 // density windows
 constexpr size_t SLOT_OBS_WORDS = (size_t)POOL_RDF * (OBS_MAXBIN + 1) + POOL_DENS_WORDS;
 constexpr int MAX_BATCH = 16;             // passes captured in one batch graph
-constexpr size_t MAX_STAGED = (size_t)1 << 28;   // pinned bytes of inputs packed ahead of their admission
 constexpr int MAX_BYPASS = 64;            // admissions past one waiting head job
 
 }  // namespace
@@ -263,7 +237,6 @@ struct mdpd_pool {
     int poll_cur = 0;
     bool need_regrow = false;
     PinnedCache pinned;
-    size_t staged = 0;                    // pinned bytes of packed inputs waiting for admission
     size_t held_pinned = 0;               // stage bytes kept by finished jobs
     size_t max_held = (size_t)1 << 30;    // beyond this their results move to pageable memory
     std::vector<std::pair<hipEvent_t, std::pair<void *, size_t>>> uploads;
@@ -453,16 +426,13 @@ struct mdpd_pool {
     }
 
     // the input block, packed once where the admission kernel reads it: in
-    // pinned memory while the waiting blocks stay below MAX_STAGED (and once
-    // the pool is on its device), else in pageable memory
+    // a staged block where there is one (and once the pool is on its device),
+    // else in pageable memory
     void pack_input(Job &j, const mdpd_system *sys)
     {
         const InLayout L = j.in_layout();
-        if (allocated && staged + L.bytes <= MAX_STAGED) {
-            hip_check(hipSetDevice(device), "hipSetDevice");
-            j.in = (char *)pinned.get(L.bytes, j.in_bytes);
-            staged += j.in_bytes;
-        } else {
+        if (allocated) hip_check(hipSetDevice(device), "hipSetDevice");
+        if (!allocated || !pinned.stage(L.bytes, (void **)&j.in, j.in_bytes)) {
             j.in_heap.reset(new char[L.bytes]);
             j.in = j.in_heap.get();
         }
@@ -718,11 +688,11 @@ struct mdpd_pool {
         char *st = j.in;
         size_t got = j.in_bytes;
         if (j.in_heap) {
-            st = (char *)pinned.get(L.bytes, got);
+            hip_check(pinned.get(L.bytes, (void **)&st, got), "hipHostMalloc");
             memcpy(st, j.in, L.bytes);
             j.in_heap.reset();
         } else {
-            staged -= got;
+            pinned.unstage(got);
         }
         j.in = nullptr;
         memcpy(st + L.sys, &d, sizeof(SysDev));
@@ -1067,7 +1037,7 @@ struct mdpd_pool {
     {
         const size_t bytes = harvest_bytes(j.npad);
         const int *dst = nlist.p + harvest_dst(P, (int)j.part_base);
-        j.stage = pinned.get(j.result_bytes(), j.stage_bytes);
+        hip_check(pinned.get(j.result_bytes(), &j.stage, j.stage_bytes), "hipHostMalloc");
         hip_check(hipMemcpyAsync(j.stage, dst, bytes, hipMemcpyDeviceToHost, stream), "harvest copy");
         size_t at = bytes;
         const unsigned *base = obs_arena.p + (size_t)j.slot * SLOT_OBS_WORDS;
