@@ -118,6 +118,28 @@ def test_sorted_order_over_scan_sizes(engine, orc, n, L):
     s.close()
 
 
+# the one-launch sort is taken by the steps between re-sorts (a slow fluid's
+# many: up to its largest; a re-sort every step: up to a third of that)
+@pytest.mark.parametrize("n, extra", [(10240, "timestep 0.001"), (10241, "timestep 0.001"),
+                                      (3072, "neigh_modify every 1 delay 0 check no"),
+                                      (3400, "neigh_modify every 1 delay 0 check no")])
+def test_sorted_order_over_resort_rates(engine, orc, n, extra):
+    L = (n / 6.05) ** (1.0 / 3.0)
+    x, v = uniform_box(n, L, n)
+    s = mdpd_system(engine, x, v, L, extra=extra)
+    s.setup()
+    keys = orc.sort_keys(orc.wrap(x.astype(np.float32), (0, 0, 0), (L, L, L)), (0, 0, 0), (L, L, L), 1.3)
+    origin, got, _ = s.debug_sorted()
+    assert np.array_equal(origin, orc.stable_sort(keys))
+    assert np.array_equal(got, keys[origin])
+    s.run(40)
+    origin, got, xw = s.debug_sorted()
+    assert np.array_equal(np.sort(origin), np.arange(n))
+    assert np.array_equal(got, orc.sort_keys(xw, (0, 0, 0), (L, L, L), 1.3))
+    assert np.all(np.diff(got.astype(np.int64)) >= 0)
+    s.close()
+
+
 # within a graph of several steps the rebuild phase makes the commit of the
 # step before, launched by itself the commit is its own launch: the one-launch
 # sort, the one-launch scan, the chunked scan, wall passes, a pool's jobs

@@ -228,6 +228,7 @@ struct PoolDev {
     int maxsub;          // sub-cell slots of the largest system (0: all cell slots, one system)
     int maxnbr;
     int one;             // one system (slot 0) holds every tile and cell slot: the plain engine
+    int sort1;           // one system: it re-sorts in one launch up to this many particle slots (sort_one_limit)
 };
 
 // ----------------------------------------------------------------------------

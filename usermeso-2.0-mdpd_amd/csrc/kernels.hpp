@@ -18,6 +18,9 @@ enum ForceMode : int {
 // split: of the pass that follows; commit: the commit that the pass before,
 // at the same split, has left to this phase (its CommitKind after_pass), or 0
 hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t st);
+// particle slots up to which one system that re-sorts every `period` steps is
+// better off with the one-launch sort
+int sort_one_limit(int period);
 hipError_t launch_nlist_only(const PoolDev &P, hipStream_t st);
 // neighbor rows of every sorted active system rebuilt in place (row width grew)
 hipError_t launch_relist(const PoolDev &P, hipStream_t st);

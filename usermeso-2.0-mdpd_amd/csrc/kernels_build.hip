@@ -417,11 +417,10 @@ __global__ void __launch_bounds__(256) k_sortgather(PoolDev P)
 
 // --------------------------------------------------------------------------
 // K1 to K4 for one small system in one launch: a workgroup holds the sub-cell
-// counts and the sort keys in LDS, each thread up to SORT1_PER particles.  Four
-// launches of a few workgroups cost 6.8 us per step when no re-sort is due
-// and 10 to 17 us when one is; this one 1.7 us, and 6 us at 1,000 particles,
-// 29 us at 8,667 (~340 instructions per particle on one CU), where it still
-// wins: a re-sort is due every third step.  `commit`: the previous step's
+// counts and the sort keys in LDS, each thread up to SORT1_PER particles.  A
+// step without a re-sort saves the idle time of three launches, a step with
+// one pays ~340 instructions per particle on one CU (sort_one_limit weighs the
+// two).  `commit`: the previous step's
 // commit (COMMIT_DECIDE) is made here first, one launch of 2.7 us less.
 // --------------------------------------------------------------------------
 constexpr int SORT1_BLK = 1024, SORT1_PER = 10, SORT1_N = SORT1_BLK * SORT1_PER, SORT1_SUB = 16384;
@@ -843,13 +842,28 @@ static void launch_nlist(const PoolDev &P, int relist, bool seeds, hipStream_t s
         hipLaunchKernelGGL(k_nlist_listed, dim3(std::min(NL_GRID, xcd_grid(std::min(P.ncact, P.nact / NL_PART)))), dim3(WAVE), 0, st, P);
 }
 
+// A step with the one-launch sort against the four launches, us (DPD fluid of
+// density 3; mDPD droplets within 2 us of it), by the steps between re-sorts:
+//   particles   1             2             3             4             none due
+//   1,000       25.2 / 31.5   21.0 / 26.7   19.4 / 24.8   18.8 / 24.0   16.7 / 21.3
+//   3,500       33.0 / 32.8   25.1 / 27.5   22.2 / 25.4   20.9 / 24.5   17.0 / 21.7
+//   5,000       38.4 / 33.4   28.0 / 27.8   24.3 / 25.7   22.6 / 24.8   17.3 / 21.8
+//   7,000       44.6 / 34.7   31.3 / 28.6   26.7 / 26.4   24.4 / 25.3   17.7 / 22.2
+//   9,000       50.6 / 35.6   34.4 / 29.2   28.9 / 26.9   26.1 / 25.8   18.0 / 22.5
+// One launch gains 4.5 us on a step without a re-sort and loses ~2.7 ns per
+// particle past 3,300 on a step with one: even at 3,300 + 1,650 (period - 1).
+int sort_one_limit(int period)
+{
+    return (int)std::min<long long>(SORT1_N, 3300 + 1650 * ((long long)std::max(period, 1) - 1));
+}
+
 hipError_t launch_rebuild(const PoolDev &P, int split, int commit, hipStream_t st)
 {
     if (P.nact == 0) return hipSuccess;
     if (commit != COMMIT_FINAL && commit != COMMIT_PHASED && commit != COMMIT_DECIDE) return hipErrorInvalidValue;
     const bool fseed = first_seeds(split, P.nact / WAVE);
     const int seeded = P.one || fseed ? 1 : 0;
-    if (P.one && P.nact <= SORT1_N && (P.ncellslots - 1) * SUBCELLS <= SORT1_SUB) {
+    if (P.one && P.nact <= std::min(P.sort1, SORT1_N) && (P.ncellslots - 1) * SUBCELLS <= SORT1_SUB) {
         if (P.nact <= SORT1_BLK)
             hipLaunchKernelGGL((k_sort_one<1>), dim3(1), dim3(SORT1_BLK), 0, st, P, commit, seeded);
         else
