@@ -194,7 +194,7 @@ struct PoolDev {
     float4 *vend;        // end-of-step velocity  (output steps only)
     // sort / cell scratch
     int *pcell;          // global sub-cell slot per particle (cell slot * SUBCELLS + sub-cell)
-    int *pslot;          // arrival rank within the sub-cell; after the re-sort: sub-cell slot of each sorted slot
+    int *pslot;          // arrival rank within the sub-cell
     int *psub;           // 12-bit sub-bin Morton code
     int *tmp;            // particle index per sorted slot (pre-order)
     int *cell_count;     // per sub-cell slot

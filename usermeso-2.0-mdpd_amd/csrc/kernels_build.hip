@@ -288,10 +288,11 @@ __global__ void __launch_bounds__(SCAN_BLK) k_scan_apply(PoolDev P)
 
 // --------------------------------------------------------------------------
 // The same scan for one system in one launch: workgroup g adds up all the
-// counts before its chunk itself, which costs it reads (two rounds of loads
-// for the 54,000 sub-cells of a 97,000-particle slab) where k_scan_sums costs
-// a launch, 1.6 us idle and 4.7 us working.  Other
-// workgroups may still read a chunk's counts, so k_scatter clears them.
+// counts before its chunk itself, which costs it reads (four chunks a round:
+// the last of the 14 workgroups for the 54,000 sub-cells of a 97,000-particle
+// slab makes four rounds) where k_scan_sums costs a launch, 1.6 us idle and 4.7
+// us working.  Other workgroups may still read a chunk's counts, so k_scatter
+// clears them.
 // --------------------------------------------------------------------------
 constexpr int SCAN1_BLK = 1024, SCAN1_CH = SCAN1_BLK * 4;
 constexpr int SCAN1_MAX = 40;          // chunks: past that the last workgroup's reads (10 rounds) cost the launches saved
@@ -336,7 +337,7 @@ __global__ void __launch_bounds__(SCAN1_BLK) k_scan_one(PoolDev P, int commit, i
 
 // --------------------------------------------------------------------------
 // K3: scatter particle indices into their sub-cell segments (arrival order),
-// the sub-bin key beside each (cl is free once k_scan has used it); with
+// the sub-bin key beside each (in cl, for the ranks of k_sortgather); with
 // `clear` the sub-cell counts of the one system are cleared here.
 // --------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_scatter(PoolDev P, int clear)
@@ -360,9 +361,7 @@ __global__ void __launch_bounds__(256) k_scatter(PoolDev P, int clear)
 // sub-cell by (sub-bin key, previous index) -- with the sub-cells in key
 // order this is the stable sort of the 2-level Morton key -- gives its sorted
 // slot; every per-particle array moves there in the other buffer (loads in
-// the previous order, issued while the rank is found; stores scattered), and
-// the sorted slot records its sub-cell (in pslot, free after k_scatter) for
-// the neighbor-row build.
+// the previous order, issued while the rank is found; stores scattered).
 // --------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_sortgather(PoolDev P)
 {
@@ -412,7 +411,6 @@ __global__ void __launch_bounds__(256) k_sortgather(PoolDev P)
     P.origin[cura ^ 1][dst] = og;
     P.image[cura ^ 1][dst] = im;
     P.phi[cura ^ 1][dst] = ph;
-    P.pslot[dst] = cell;
 }
 
 // --------------------------------------------------------------------------
