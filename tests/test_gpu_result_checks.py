@@ -12,7 +12,8 @@ import re
 import numpy as np
 import pytest
 
-from conftest import PKG
+from conftest import PKG, uniform_box
+from test_gpu_parity import mdpd_system
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +100,22 @@ def test_creation_index_outside_the_system_is_reported(engine, kernel, index, wa
         np.testing.assert_array_equal(out[origin[:N]], tag[:N])
     assert ok.sum() == N - want
     pinned.close()
+
+
+def test_gather_of_a_handle_whose_device_is_not_current(engine):
+    pinned, count = _Pinned(engine), ctypes.c_int()
+    assert pinned.hip.hipGetDeviceCount(ctypes.byref(count)) == 0
+    if count.value < 2:
+        pytest.skip("one device")
+    x, v = uniform_box(300, 4.0, 1)
+    a, b = mdpd_system(engine, x, v, 4.0), mdpd_system(engine, x, v, 4.0)
+    for s in (a, b):
+        s.run(2)
+    want = a.gather("x"), a.debug_sorted()[1]
+    pinned.hip.hipSetDevice(1)
+    np.testing.assert_array_equal(b.gather("x"), want[0])
+    pinned.hip.hipSetDevice(1)
+    np.testing.assert_array_equal(b.debug_sorted()[1], want[1])
+    pinned.hip.hipSetDevice(0)
+    a.close()
+    b.close()

@@ -261,6 +261,7 @@ int mdpd_debug_sorted(mdpd_system *sys, int *origin_out, unsigned long long *key
             // two words per key in the compact rows (free between passes)
             static_assert(NBR_ALIGN >= 2, "a key per particle fits the narrowest compact rows");
             unsigned long long *keys = (unsigned long long *)sys->clist.p;
+            hip_check(hipSetDevice(sys->device), "hipSetDevice");
             hip_check(launch_sort_keys(sys->view(), keys, sys->stream), "sort keys");
             auto k = sys->download(keys, n);
             hip_check(hipStreamSynchronize(sys->stream), "sync");

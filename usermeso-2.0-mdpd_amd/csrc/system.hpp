@@ -2043,6 +2043,8 @@ struct mdpd_system {
     void gather_field(int field, size_t words, double *d, int *k)
     {
         static_assert(NBR_ALIGN >= 6, "six words per particle fit the narrowest compact rows");
+        // events belong to the device that is current when they are made
+        hip_check(hipSetDevice(device), "hipSetDevice");
         if (!stage) {
             hip_check(hipHostMalloc((void **)&stage, (2 * STAGE_WORDS + 1) * sizeof(int), hipHostMallocDefault),
                       "hipHostMalloc");
