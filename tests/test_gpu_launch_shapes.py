@@ -294,7 +294,7 @@ def test_negative_wall_fractions_scale_every_pair(engine, split):
 # jobs that end together: sixty of them are more tiles than the wide kernels
 # take, a job's own handle is not
 @pytest.mark.parametrize("split", [2, 4])
-@pytest.mark.parametrize("case", ["liquid", "two types", "dpd"])
+@pytest.mark.parametrize("case", ["liquid", "two types", "uneven", "walls", "dpd"])
 def test_results_of_many_jobs_ending_together_equal_their_own_runs(engine, case, split):
     s = CASES[case](engine)
     count = -(-513 * 64 // ((s.natoms + 255) // 256 * 256))
