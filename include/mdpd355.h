@@ -210,7 +210,8 @@ int mdpd_tea_gaussian_noalloc(int device, int n, const unsigned int *a, const un
  * job's input (40 to 44 bytes per particle and 8 per cell) is host memory too:
  * once the pool is on its device pinned, in blocks of powers of two from 1 MiB
  * up, while waiting jobs hold less than 512 MiB of them.  Blocks are reused and
- * freed with the pool.  One host thread drives a pool. */
+ * freed with the pool (free ones past 2 GiB when new ones are needed).  One
+ * host thread drives a pool. */
 typedef struct mdpd_pool mdpd_pool;
 
 enum { MDPD_JOB_QUEUED = 0, MDPD_JOB_RUNNING = 1, MDPD_JOB_DONE = 2 };

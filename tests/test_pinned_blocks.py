@@ -64,10 +64,81 @@ int main()
 }
 """
 
+# page-locked memory runs out at MEMORY bytes
+FREE_BLOCKS = r"""
+#include "pinned.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+static const size_t MEMORY = (size_t)6 << 30;
+static size_t used = 0;
+static std::map<void *, size_t> size;
+extern "C" hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    if (used + n > MEMORY) return hipErrorOutOfMemory;
+    used += n;
+    size[*p = malloc(1)] = n;
+    return hipSuccess;
+}
+extern "C" hipError_t hipHostFree(void *p)
+{
+    used -= size.at(p);
+    size.erase(p);
+    free(p);
+    return hipSuccess;
+}
+extern "C" hipError_t hipGetLastError(void) { return hipSuccess; }
+#define CHECK(c) do { if (!(c)) { printf("line %d: %s\n", __LINE__, #c); return 1; } } while (0)
+int main()
+{
+    using mdpd::PinnedCache;
+    const size_t MiB = 1 << 20;
+    void *p[2048];
+    size_t got;
+    {   // sizes that drift: every class holds a GiB at its time, one by one
+        PinnedCache c;
+        for (size_t sz = MiB; sz <= 64 * MiB; sz *= 2) {
+            const size_t n = 1024 * MiB / sz;
+            for (size_t k = 0; k < n; ++k) CHECK(c.get(sz, &p[k], got) == hipSuccess && got == sz);
+            CHECK(used <= PinnedCache::MAX_FREE + n * sz);
+            for (size_t k = 0; k < n; ++k) c.put(p[k], sz);
+            CHECK(c.free_bytes == used);
+            for (size_t k = 0; k < n; ++k) CHECK(c.get(sz, &p[k], got) == hipSuccess);     // its own again
+            CHECK(c.free_bytes + n * sz == used);
+            for (size_t k = 0; k < n; ++k) c.put(p[k], sz);
+        }
+    }
+    CHECK(used == 0 && size.empty());
+    {   // no memory left but what larger free blocks hold
+        PinnedCache c;
+        for (size_t k = 0; k < 16; ++k) CHECK(c.get(128 * MiB, &p[k], got) == hipSuccess);
+        for (size_t k = 0; k < 16; ++k) c.put(p[k], 128 * MiB);
+        for (size_t k = 0; k < 1024; ++k) CHECK(c.get(4 * MiB, &p[k], got) == hipSuccess);
+        CHECK(used == MEMORY && c.free_bytes == 2048 * MiB);
+        void *q, *r;
+        CHECK(c.get(3 * MiB, &q, got) == hipSuccess && used == MEMORY - 2044 * MiB && c.free_bytes == 0);
+        for (size_t k = 0; k < 511; ++k) CHECK(c.get(4 * MiB, &p[1024 + k], got) == hipSuccess);
+        CHECK(used == MEMORY && c.get(MiB, &r, got) != hipSuccess);
+        for (size_t k = 0; k < 1535; ++k) c.put(p[k], 4 * MiB);
+        c.put(q, 4 * MiB);
+    }
+    CHECK(used == 0 && size.empty());
+    return 0;
+}
+"""
+
+
+def test_free_pinned_blocks_are_bounded_and_given_back(tmp_path):
+    run_program(tmp_path, FREE_BLOCKS)
+
 
 def test_pinned_blocks(tmp_path):
+    run_program(tmp_path, PROGRAM)
+
+
+def run_program(tmp_path, program):
     src, exe = tmp_path / "blocks.cpp", tmp_path / "blocks"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(PKG, "csrc"),
                     "-I", "/opt/rocm/include", str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstddef>
+#include <iterator>
 #include <map>
 
 namespace mdpd {
@@ -21,12 +22,23 @@ struct PinnedCache {
     // in pageable memory, which costs each a copy (256 droplets of 2,000 to
     // 40,000 particles hold 260 MiB)
     static constexpr size_t MAX_STAGED = (size_t)1 << 29;
+    // free blocks kept (a full hold of results, the inputs that wait and as
+    // much again): a request that finds none of its class first gives back the
+    // largest of more than this, so that sizes that drift from class to class
+    // do not each leave their most behind
+    static constexpr size_t MAX_FREE = (size_t)1 << 31;
     std::multimap<size_t, void *> free_;
-    size_t staged = 0;
+    size_t staged = 0, free_bytes = 0;
 
-    ~PinnedCache()
+    ~PinnedCache() { trim(0); }
+    void trim(size_t keep)
     {
-        for (auto &f : free_) (void)hipHostFree(f.second);
+        while (free_bytes > keep) {
+            auto it = std::prev(free_.end());
+            (void)hipHostFree(it->second);
+            free_bytes -= it->first;
+            free_.erase(it);
+        }
     }
     static size_t size_class(size_t bytes)
     {
@@ -38,12 +50,24 @@ struct PinnedCache {
     {
         got = size_class(bytes);
         auto it = free_.find(got);
-        if (it == free_.end()) return hipHostMalloc(p, got, hipHostMallocDefault);
+        if (it == free_.end()) {
+            trim(MAX_FREE);
+            const hipError_t e = hipHostMalloc(p, got, hipHostMallocDefault);
+            if (e == hipSuccess || free_.empty()) return e;
+            (void)hipGetLastError();
+            trim(0);                          // what other classes hold may be what is missing
+            return hipHostMalloc(p, got, hipHostMallocDefault);
+        }
         *p = it->second;
+        free_bytes -= got;
         free_.erase(it);
         return hipSuccess;
     }
-    void put(void *p, size_t sz) { free_.emplace(sz, p); }
+    void put(void *p, size_t sz)
+    {
+        free_.emplace(sz, p);
+        free_bytes += sz;
+    }
 
     // a block for an input that waits; false: none to be had
     bool stage(size_t bytes, void **p, size_t &got)
